@@ -234,8 +234,13 @@ void MeshLevel::upload()
     std::vector<float> gf(geo.begin(), geo.end());
     d_geo_f.upload(gf);
     d_owned_lat.upload(owned_lat);
-    d_grp_off.upload(grp_off);
-    d_grp_mem.upload(grp_mem);
+    std::vector<int32_t> pad((size_t)GRP_PAD * ngroups(), -1);
+    for (int g = 0; g < ngroups(); ++g) {
+        const int cnt = grp_off[g + 1] - grp_off[g];
+        TN_REQUIRE(cnt >= 2 && cnt <= GRP_PAD, "mesh: node copies out of range");
+        for (int k = 0; k < cnt; ++k) pad[(size_t)GRP_PAD * g + k] = grp_mem[grp_off[g] + k];
+    }
+    d_grp_pad.upload(pad);
     d_scratch.alloc(64);
     d_part.alloc(REDUCE_PART_DOUBLES);
     uploaded = true;

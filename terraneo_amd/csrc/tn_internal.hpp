@@ -89,8 +89,10 @@ struct MeshLevel {
     DevBuf<double> d_geo;
     DevBuf<float> d_geo_f;
     DevBuf<uint8_t> d_owned_lat;
-    DevBuf<int32_t> d_grp_off;
-    DevBuf<int32_t> d_grp_mem;
+    // the groups for the device: GRP_PAD members each, -1 past the last (a lateral
+    // node has at most five copies, at the icosahedron's poles)
+    static constexpr int GRP_PAD = 8;
+    DevBuf<int32_t> d_grp_pad;
     DevBuf<double> d_scratch;  // reduction results (doubles)
     DevBuf<double> d_part;     // per-block partial sums of the reductions (REDUCE_PART_DOUBLES)
     bool uploaded = false;
