@@ -161,6 +161,30 @@ int tn::march_seg_for(int n, int own, int waves_per_cu)
     }
     return best;
 }
+// Blocks of the carried-corner march over `cols` node columns (all strips),
+// `resident` blocks fitting a CU.  A block takes (columns + 2) steps -- the
+// column before its run again, and about a step of start-up -- and a CU runs
+// two blocks together 1.55 times as long as one (a step costs 2.7 us at 12
+// resident waves, 4.2 us at 24; FP32, level 5 to 7), so: one or two equal runs
+// per CU, whichever ends sooner, and further rounds only where a run would be
+// longer than the kernel's carried level (MARCH_SEG_MAX columns).
+int tn::march_run_blocks(int cols, int resident)
+{
+    const int64_t cus = device_cus();
+    int64_t best = 1;
+    double best_cost = -1.0;
+    for (int per_cu = 1; per_cu <= resident; ++per_cu) {
+        const int64_t slots = cus * per_cu;
+        const int64_t rounds = (cols + slots * MARCH_SEG_MAX - 1) / (slots * MARCH_SEG_MAX);
+        const int64_t blocks = std::min<int64_t>(slots * rounds, cols);
+        const double cost = (double)rounds * ((cols + blocks - 1) / blocks + 2) * (per_cu == 1 ? 1.0 : 1.55);
+        if (best_cost < 0 || cost < best_cost) {
+            best_cost = cost;
+            best = blocks;
+        }
+    }
+    return (int)best;
+}
 namespace {
 
 int march_seg(int n, int dtype_size)
@@ -197,9 +221,11 @@ void eps_apply_t(tn_eps* op, const void* src_v, void* dst_v, hipStream_t s)
         const tn::Geom<T> g = geom_of<T>(m);
         // penalty positions: every copy (the reference's rule) or the owned copy only
         const double* pen_coords = op->penalty_once ? m.d_coords_owned.p : m.d_coords.p;
+        const int rows = tn::march_block_rows((int)sizeof(T));
         tn::MarchArgs<T> a{src, dst, eta, eta_cell, g.geo, g.coords, g.radii, pen_coords, m.d_radii.p,
                            need_blk ? (const T*)op->blk.p : nullptr, penalty ? op->pen.p : nullptr,
-                           m.n, m.nr, march_seg(m.n, (int)sizeof(T)), op->bc_cmb, op->bc_surf, add ? 1 : 0,
+                           m.n, m.nr, march_seg(m.n, (int)sizeof(T)),
+                           tn::march_run_blocks(10 * ((m.n + rows - 1) / rows) * m.n, tn::march_resident(sizeof(T))), op->bc_cmb, op->bc_surf, add ? 1 : 0,
                            tn::march_guard()};
         tn::launch_eps_march<T>(a, op->diagonal, s);
     } else {

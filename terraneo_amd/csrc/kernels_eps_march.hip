@@ -517,8 +517,9 @@ __device__ __forceinline__ double shift_up1(double v)
 // CFG bits: 1 a shell is not Neumann (boundary lanes), 2 fs/fs rotation
 // penalty, 4 per-cell viscosity; each case is compiled on its own so the
 // common ones carry no dead state in registers
+// (FP32: held to 6 waves per SIMD, so that two 12-wave blocks fit a CU)
 template <typename T, int W, int CFG>
-__global__ __launch_bounds__(64 * W) void k_eps_flow(MarchArgs<T> a, const T* __restrict__ geo_tab,
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 6 : 1))) void k_eps_flow(MarchArgs<T> a, const T* __restrict__ geo_tab,
                                                      const T* __restrict__ coords, const T* __restrict__ blk_tab,
                                                      const double* __restrict__ coords_d,
                                                      const double* __restrict__ pen)
@@ -538,16 +539,18 @@ __global__ __launch_bounds__(64 * W) void k_eps_flow(MarchArgs<T> a, const T* __
     __shared__ T xkeep[W][2][2][3];          // raw boundary-level source of node (x, y): [parity][cmb / surface]
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int n = a.n, nr = a.nr, ncr = nr - 1, ncl = n - 1;
-    const int nxb = (n + OWN - 1) / OWN, nys = (n + a.seg - 1) / a.seg;
-    int b = xcd_tile(blockIdx.x, gridDim.x);
-    const int ys = b % nys;
-    b /= nys;
-    const int xb = b % nxb;
-    const int d = b / nxb;
-    const int x = xb * OWN - 1 + w;
-    const bool strip_ok = x >= 0 && x <= n - 2;
-    const bool row_own = w >= 1 && x <= n - 1;
-    const int y0 = ys * a.seg, y1 = min(y0 + a.seg, n);
+    const int nxb = (n + OWN - 1) / OWN;
+    // This block's run of node columns: the columns of all strips (row block xb of
+    // diamond d, y fastest) are split evenly over the blocks, so a run may cover the
+    // end of one strip and the start of the next; each part is one march.  Equal
+    // segments per strip left CUs idle in the last round: at lateral level 7 x 129
+    // (FP64) 450 blocks of 26 columns on 256 CUs took 507 us, even runs of 45
+    // columns 471 us; at level 3 x 9 (runs of one column) 22.7 -> 11.4 us, at
+    // 4 x 17 34.5 -> 18.7 us.
+    const int ncols = 10 * nxb * n;
+    const int tile = xcd_tile(blockIdx.x, gridDim.x);
+    int col = march::run_begin(ncols, tile, gridDim.x);
+    const int col_end = march::run_begin(ncols, tile + 1, gridDim.x);
     const uint32_t Nn = 10u * n * n * nr;    // nodes per component
     const uint32_t Nb = Nn * SZ;
     const __amdgpu_buffer_rsrc_t rs_src = buf_rsrc(a.src, 3 * Nb);
@@ -559,11 +562,17 @@ __global__ __launch_bounds__(64 * W) void k_eps_flow(MarchArgs<T> a, const T* __
     // byte offsets of radial columns: node (xc, yc) of this diamond at ((d n + xc) n + yc) nr
     const uint32_t colstep = (uint32_t)nr * SZ;             // next y
     const uint32_t rowstep = (uint32_t)n * nr * SZ;         // next x
-    const uint32_t colx = (uint32_t)((d * n + x) * n) * nr * SZ;  // column (x, 0) (x >= -1: wraps for x = -1, unused)
     if (lane == 0) done[w] = used[w] = 0;
     __syncthreads();
     int step = 0;
 
+    while (col < col_end) {
+    const int strip = col / n, y0 = col - strip * n, y1 = min(n, y0 + (col_end - col));
+    col += y1 - y0;
+    const int d = strip / nxb, x = (strip - d * nxb) * OWN - 1 + w;
+    const bool strip_ok = x >= 0 && x <= n - 2;
+    const bool row_own = w >= 1 && x <= n - 1;
+    const uint32_t colx = (uint32_t)((d * n + x) * n) * nr * SZ;  // column (x, 0) (x >= -1: wraps for x = -1, unused)
     for (int h = 0; h < nchunks; ++h) {
         const int c = 64 * h + lane;
         const bool valid = c < ncr;
@@ -775,6 +784,7 @@ __global__ __launch_bounds__(64 * W) void k_eps_flow(MarchArgs<T> a, const T* __
         }
         step += y1 - qs;
     }
+    }
 }
 
 // Quadratic forms of the 3x3 diagonal block of the Neumann operator at every
@@ -895,6 +905,8 @@ int march_block_rows(int dtype_size) { return (dtype_size == 8 ? march_waves<dou
 
 int march_waves_per_cu(int dtype_size) { return march_block_rows(dtype_size) + 1; }
 
+int march_resident(int dtype_size) { return dtype_size == 4 && march_waves<float>() <= 12 ? 2 : 1; }
+
 // matrix-apply kernel variant: 0 the per-quad-load march, 1 the carried-corner
 // march, 2 the same with each step's loads issued a step ahead (TN_EPS_KERNEL
 // overrides; tuning)
@@ -924,12 +936,15 @@ void launch_march_w(const MarchArgs<T>& a, bool diagonal, hipStream_t s)
         if constexpr (W >= 8) {
             const int cfg = ((a.bc_cmb != TN_NEUMANN || a.bc_surf != TN_NEUMANN) ? 1 : 0) | (a.pen ? 2 : 0) |
                             (a.eta_cell ? 4 : 0) | (var == 2 ? 8 : 0);
+            const dim3 fr((unsigned)a.blocks);
+            TN_REQUIRE(a.blocks >= 1 && ((int64_t)10 * nxb * a.n + a.blocks - 1) / a.blocks <= MARCH_SEG_MAX,
+                       "march kernel: run of columns out of range");
             TN_REQUIRE(3ULL * 10 * a.n * a.n * a.nr * sizeof(T) < (1ULL << 32),
                        "apply: field larger than 4 GB (buffer resources address 32-bit byte offsets)");
             switch (cfg) {
 #define TN_FLOW(C)                                                                                                \
     case C:                                                                                                      \
-        hipLaunchKernelGGL((k_eps_flow<T, W, C>), gr, bl, 0, s, a, a.geo, a.coords, a.blk, a.coords_d, a.pen); \
+        hipLaunchKernelGGL((k_eps_flow<T, W, C>), fr, bl, 0, s, a, a.geo, a.coords, a.blk, a.coords_d, a.pen); \
         break;
                 TN_FLOW(0) TN_FLOW(1) TN_FLOW(2) TN_FLOW(3) TN_FLOW(4) TN_FLOW(5) TN_FLOW(6) TN_FLOW(7)
                 TN_FLOW(8) TN_FLOW(9) TN_FLOW(10) TN_FLOW(11) TN_FLOW(12) TN_FLOW(13) TN_FLOW(14) TN_FLOW(15)

@@ -43,6 +43,13 @@ __host__ __device__ inline int blocks_for(int n, int seg, int waves)
     return 10 * ((n + own - 1) / own) * ((n + seg - 1) / seg);
 }
 
+// first column of run `b` when `total` columns are split over `blocks` runs
+// (run lengths differ by at most one)
+__host__ __device__ inline int run_begin(int total, int b, int blocks)
+{
+    return (int)((int64_t)total * b / blocks);
+}
+
 // Point-to-point hand-off between neighbouring waves through LDS counters
 // instead of a block barrier per step: the waves of a SIMD drift apart and hide
 // each other's memory latency.  The waves of a workgroup are co-resident and
