@@ -67,7 +67,7 @@ struct MeanFree {
     BVec ones;
     DevBuf<double> sum, part;
     double inv_count = 0.0;
-    MeanFree(Ctx& c, const Field& like) : m(like.m), dtype(like.dtype), sum(1), part(REDUCE_PART_DOUBLES)
+    MeanFree(Ctx& c, const Field& like) : m(like.m), dtype(like.dtype), st(c.s), sum(1), part(REDUCE_PART_DOUBLES)
     {
         ones = st.make(vec1(like));
         v_fill(c, ones, 1.0);
@@ -163,6 +163,7 @@ namespace {
 void gmg_setup(tn_gmg* g, const tn_gmg_options& o, hipStream_t s)
 {
     g->ctx.s = s;
+    g->store.s = s;
     Ctx& c = g->ctx;
     const int L = (int)g->ops.size();
     for (int l = 0; l < L; ++l) {
@@ -327,7 +328,7 @@ int tn_pcg_solve(tn_eps* A, tn_gmg* prec, void* x, const void* b, const tn_krylo
     TN_REQUIRE(A && x && b && o, "null pointer");
     Ctx c;
     c.s = (hipStream_t)s;
-    VecStore st;
+    VecStore st(c.s);
     const BVec X = vec1(field_of(A->mesh, A->dtype, 3, x)), B = vec1(field_of(A->mesh, A->dtype, 3, b));
     std::vector<BVec> t;
     for (int i = 0; i < 4; ++i) t.push_back(st.make(X));
@@ -357,7 +358,7 @@ int tn_stokes_solve(tn_stokes* K, int method, tn_gmg* prec_u, const void* schur_
     TN_REQUIRE(K && prec_u && schur_diag && u && p && bu && bp && o, "null pointer");
     Ctx c;
     c.s = (hipStream_t)s;
-    VecStore st;
+    VecStore st(c.s);
     const int dt = K->A->dtype;
     const Field fu = field_of(K->vel, dt, 3, u), fp = field_of(K->pre, dt, 1, p);
     const BVec X = vec2(fu, fp);
@@ -462,7 +463,7 @@ int tn_fv_to_fe(tn_fv* fv, const double* Tfv, double* Tfe, const tn_krylov_optio
     TN_REQUIRE(fv && Tfv && Tfe && o, "null pointer");
     Ctx c;
     c.s = (hipStream_t)s;
-    VecStore st;
+    VecStore st(c.s);
     const BVec X = vec1(field_of(fv->mesh, TN_F64, 1, Tfe));
     const BVec B = st.make(X);
     launch_fv_to_fe_rhs(fv->args(), Tfv, (double*)B.b[0].p, c.s);

@@ -26,11 +26,13 @@ BVec VecStore::make_like(const BVec& like, int dtype)
     BVec v = like;
     for (int i = 0; i < like.nb; ++i) {
         v.b[i].dtype = dtype;
-        void* p = nullptr;
-        TN_HIP(hipMalloc(&p, (size_t)v.b[i].count() * v.b[i].esize()));
-        TN_HIP(hipMemset(p, 0, (size_t)v.b[i].count() * v.b[i].esize()));
+        void* p = dev_alloc((size_t)v.b[i].count() * v.b[i].esize());
         ptrs_.push_back(p);
         v.b[i].p = p;
+        if (dtype == TN_F64)
+            launch_fill<double>((double*)p, v.b[i].count(), 0.0, s);
+        else
+            launch_fill<float>((float*)p, v.b[i].count(), 0.0f, s);
     }
     return v;
 }
@@ -39,7 +41,7 @@ BVec VecStore::make(const BVec& like) { return make_like(like, like.b[0].dtype);
 
 VecStore::~VecStore()
 {
-    for (void* p : ptrs_) (void)hipFree(p);
+    for (void* p : ptrs_) dev_free(p);
 }
 
 Ctx::Ctx()

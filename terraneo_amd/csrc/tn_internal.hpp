@@ -33,6 +33,10 @@ void set_last_error(const std::string& msg);
     } while (0)
 
 // ---------------------------------------------------------------- device buffers
+// device memory of the library's objects, with a bounded cache of freed blocks (devmem.cpp)
+void* dev_alloc(size_t bytes);
+void dev_free(void* ptr);
+
 template <typename T>
 struct DevBuf {
     T* p = nullptr;
@@ -45,12 +49,12 @@ struct DevBuf {
     void alloc(size_t count)
     {
         release();
+        p = static_cast<T*>(dev_alloc(sizeof(T) * count));
         n = count;
-        if (count) TN_HIP(hipMalloc(&p, sizeof(T) * count));
     }
     void release()
     {
-        if (p) (void)hipFree(p);
+        dev_free(p);
         p = nullptr;
         n = 0;
     }

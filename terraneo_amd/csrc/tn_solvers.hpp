@@ -35,9 +35,12 @@ struct BVec {
     const Field& p() const { return b[1]; }
 };
 
-// Device memory owner for vectors shaped like a template.
+// Device memory owner for vectors shaped like a template; new vectors are
+// zeroed on stream s, the stream of the work that uses them.
 class VecStore {
   public:
+    hipStream_t s = nullptr;
+    explicit VecStore(hipStream_t stream = nullptr) : s(stream) {}
     BVec make(const BVec& like);
     BVec make_like(const BVec& like, int dtype);
     ~VecStore();
