@@ -324,50 +324,65 @@ __global__ void k_restrict(const T* __restrict__ xf, T* __restrict__ xc, const u
 
 // ---------------------------------------------------------------- GCA assembly
 
-// Interpolation from the 6 coarse wedge dofs onto the 6 dofs of one fine
-// wedge (gca.hpp:195-345, constant mode).  (fx, fy, fr) = fine hex cell,
-// fine wedge w, nrf = fine radial node count.  Reproduces the coded radial
-// bracket r_bot = r/2 (gca.hpp:213-216); geometric != 0 takes the bracket of
-// the coarse cell R the fine dof lies in instead (exact Galerkin product).
-__device__ inline void gca_local_P(int fx, int fy, int fr, int w, int nrf, int R, int geometric, double P[6][6])
+// Interpolation from the 6 coarse wedge dofs onto the 6 dofs of the fine
+// wedges of a coarse wedge (gca.hpp:195-345, constant mode): scalar weights,
+// the same for the three components.  A fine dof at a coarse vertex takes it, a
+// radial midpoint halves its two vertices, a lateral midpoint averages the two
+// ends of its coarse edge on the coarse levels of the radial bracket it uses:
+// the coded one, r_bot = r/2 (gca.hpp:213-216), sends an even radial index
+// to the bracket above -- weights of the coarse cell's bottom nodes -- except at
+// the surface; `own` (the surface, or geometric != 0) takes the bracket of the
+// coarse cell itself.
+//
+// fine wedges of coarse wedge W (gca.hpp:353-370): offsets of the fine hex cell, wedge
+struct GcaWedge {
+    int8_t sx, sy, sr, w;
+};
+__device__ constexpr GcaWedge GCA_LIST[2][8] = {
+    {{0, 0, 0, 0}, {1, 0, 0, 0}, {0, 1, 0, 0}, {0, 0, 1, 0}, {1, 0, 1, 0}, {0, 1, 1, 0}, {0, 0, 0, 1}, {0, 0, 1, 1}},
+    {{1, 0, 0, 1}, {0, 1, 0, 1}, {1, 1, 0, 1}, {1, 0, 1, 1}, {0, 1, 1, 1}, {1, 1, 1, 1}, {1, 1, 0, 0}, {1, 1, 1, 0}}};
+
+// P = C + the lateral midpoints on the coarse cell's top plane: B_im is their
+// weight of coarse lateral node m, at the bottom nodes, or with `own` at the top
+struct GcaWeights {
+    double C[2][8][6][6];  // [coarse wedge][fine wedge][fine dof][coarse dof]
+    double B[2][8][3][3];  // [coarse wedge][fine wedge][fine dof - 3][coarse lateral node]
+};
+__host__ __device__ constexpr GcaWeights make_gca_weights()
 {
-    for (int i = 0; i < 6; ++i)
-        for (int j = 0; j < 6; ++j) P[i][j] = 0.0;
-    for (int fl = 0; fl < 6; ++fl) {
-        const int ix = fx + WOFF[w][fl][0], iy = fy + WOFF[w][fl][1], ir = fr + WOFF[w][fl][2];
-        if (!(ix & 1) && !(iy & 1) && !(ir & 1)) {
-            P[fl][fl] = 1.0;
-            continue;
-        }
-        const int rb = geometric ? R : (ir < nrf - 1 ? ir / 2 : ir / 2 - 1), rt = rb + 1;
-        if (!(ix & 1) && !(iy & 1)) {
-            const int a = fl % 3;
-            P[fl][a] = 0.5;
-            P[fl][a + 3] = 0.5;
-            continue;
-        }
-        int x0, x1, y0, y1, cl[4];
-        if (!(ix & 1)) {
-            x0 = x1 = ix / 2; y0 = iy / 2; y1 = iy / 2 + 1;
-            cl[0] = 0; cl[1] = 2; cl[2] = 3; cl[3] = 5;
-        } else if (!(iy & 1)) {
-            x0 = ix / 2; x1 = ix / 2 + 1; y0 = y1 = iy / 2;
-            cl[0] = 0; cl[1] = 1; cl[2] = 3; cl[3] = 4;
-        } else {
-            x0 = ix / 2 + 1; x1 = ix / 2; y0 = iy / 2; y1 = iy / 2 + 1;
-            cl[0] = 1; cl[1] = 2; cl[2] = 4; cl[3] = 5;
-        }
-        auto wgt = [&](int xc, int yc, int rc) {
-            const int dr = ir - 2 * rc;
-            const double lw = pc_lat_weight(ix - 2 * xc, iy - 2 * yc);
-            return dr == 0 ? lw : ((dr == 1 || dr == -1) ? 0.5 * lw : 0.0);
-        };
-        P[fl][cl[0]] = wgt(x0, y0, rb);
-        P[fl][cl[1]] = wgt(x1, y1, rb);
-        P[fl][cl[2]] = wgt(x0, y0, rt);
-        P[fl][cl[3]] = wgt(x1, y1, rt);
-    }
+    GcaWeights t{};
+    constexpr int OFF[2][3][2] = {{{0, 0}, {1, 0}, {0, 1}}, {{1, 1}, {0, 1}, {1, 0}}};
+    constexpr GcaWedge L[2][8] = {
+        {{0, 0, 0, 0}, {1, 0, 0, 0}, {0, 1, 0, 0}, {0, 0, 1, 0}, {1, 0, 1, 0}, {0, 1, 1, 0}, {0, 0, 0, 1}, {0, 0, 1, 1}},
+        {{1, 0, 0, 1}, {0, 1, 0, 1}, {1, 1, 0, 1}, {1, 0, 1, 1}, {0, 1, 1, 1}, {1, 1, 1, 1}, {1, 1, 0, 0}, {1, 1, 1, 0}}};
+    for (int W = 0; W < 2; ++W)
+        for (int k = 0; k < 8; ++k)
+            for (int i = 0; i < 6; ++i) {
+                const GcaWedge f = L[W][k];
+                const int m = i % 3;
+                // the fine dof's offset from the coarse cell's corner, in fine steps
+                const int a = f.sx + OFF[f.w][m][0], b = f.sy + OFF[f.w][m][1], c = f.sr + (i >= 3 ? 1 : 0);
+                double* P = t.C[W][k][i];
+                if (a % 2 == 0 && b % 2 == 0) {
+                    if (c % 2 == 0) {
+                        P[i] = 1.0;
+                    } else {
+                        P[m] = P[m + 3] = 0.5;
+                    }
+                    continue;
+                }
+                // ends of the coarse edge: along y (a even), along x (b even), the diagonal
+                const int e0 = (a % 2 != 0 && b % 2 != 0) ? 1 : 0, e1 = a % 2 == 0 ? 2 : (b % 2 == 0 ? 1 : 2);
+                if (c == 0)
+                    P[e0] = P[e1] = 0.5;
+                else if (c == 1)
+                    P[e0] = P[e1] = P[e0 + 3] = P[e1 + 3] = 0.25;
+                else
+                    t.B[W][k][i - 3][e0] = t.B[W][k][i - 3][e1] = 0.5;
+            }
+    return t;
 }
+__device__ constexpr GcaWeights GCA_P = make_gca_weights();
 
 // Fine-level 6x6 block (row component q, column component p) of the raw
 // epsilon wedge matrix assembled from geometry (one-point quadrature):
@@ -393,92 +408,240 @@ __device__ inline void eps_block_geo(const T* __restrict__ geo_w, T r0, T r1, do
         }
 }
 
-template <typename S>
-__device__ inline void stored_block(const S* __restrict__ st, int64_t ncells, int64_t cell, int w, int q, int p,
-                                    double A[6][6])
+// Galerkin matrices sum P^T A P over the 8 fine wedges of a coarse wedge.
+//
+// Matrix-free fine operator: its wedge matrix is a sum of products of the six
+// shape gradients g_i,
+//   A_(i,q),(j,p) = kwJ [ delta_pq g_i.g_j + g_i[p] g_j[q] - 2/3 g_i[q] g_j[p] ],
+// and P acts on the nodes alone, so P^T A P is the same expression in the
+// projected gradients G_a = sum_i P_ia g_i: no 6x6 products.  Two threads per
+// (coarse cell, coarse wedge): HALF 0 the component blocks (0, p), the packed
+// entries [0, 93), HALF 1 the blocks (1, 1), (1, 2), (2, 2), the entries
+// [93, 171).  The sums stay in registers in FP64 (a whole wedge's 171 would need
+// accumulation registers and their moves) and are written once as 16-byte
+// vectors of the tile layout, a wave's 64 consecutive cells side by side.  The
+// weights are wave-uniform (scalar loads).
+// Lateral level 6 -> 5 (65 -> 33 radial nodes, 0.90 GB of FP64 matrices): 14.8 ms
+// with a thread per component block that formed A and both 6x6 products in local
+// arrays; 0.33 ms in this form (2.7 TB/s of writes).
+template <typename T, typename S, typename SF, int HALF>
+__device__ __forceinline__ void gca_geo_half(const GcaArgs<T, S, SF>& a, int64_t cell, int W)
 {
-    for (int i = 0; i < 6; ++i)
-        for (int j = 0; j < 6; ++j) {
-            int r = i + 6 * q, c = j + 6 * p;
-            if (r > c) {
-                const int t = r;
-                r = c;
-                c = t;
-            }
-            A[i][j] = (double)st[stored_at<S>(cell, w, pk(r, c))];
-        }
-}
-
-// One thread per (coarse cell, coarse wedge, component block q <= p).
-// FINE_GEO: fine operator is matrix-free (raw local matrices from geometry);
-// otherwise it is read from the fine level's packed storage.
-template <typename T, typename S, typename SF, bool FINE_GEO>
-__global__ void k_gca_build(GcaArgs<T, S, SF> a)
-{
-    constexpr int QP[6][2] = {{0, 0}, {0, 1}, {0, 2}, {1, 1}, {1, 2}, {2, 2}};
-    const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t ncc = 10LL * (a.nc - 1) * (a.nc - 1) * (a.nrc - 1);
-    if (tid >= ncc * 12) return;
-    const int blk = (int)(tid % 6);
-    const int W = (int)((tid / 6) % 2);
-    const int64_t cell = tid / 12;
-    const int q = QP[blk][0], p = QP[blk][1];
+    constexpr int LO = HALF ? 93 : 0, CNT = HALF ? PACKED - 93 : 93;
+    constexpr int Q0 = HALF ? 1 : 0, Q1 = HALF ? 3 : 1;  // block rows q of this half
     const int R = (int)(cell % (a.nrc - 1));
     int64_t lat = cell / (a.nrc - 1);
     const int Y = (int)(lat % (a.nc - 1));
     lat /= (a.nc - 1);
     const int X = (int)(lat % (a.nc - 1));
     const int d = (int)(lat / (a.nc - 1));
-    constexpr int SH[8][3] = {{0, 0, 0}, {1, 0, 0}, {0, 1, 0}, {1, 1, 0}, {0, 0, 1}, {1, 0, 1}, {0, 1, 1}, {1, 1, 1}};
-    // fine wedges of coarse wedge W (gca.hpp:353-370)
-    constexpr int LIST[2][8][2] = {{{0, 0}, {1, 0}, {2, 0}, {4, 0}, {5, 0}, {6, 0}, {0, 1}, {4, 1}},
-                                   {{1, 1}, {2, 1}, {3, 1}, {5, 1}, {6, 1}, {7, 1}, {3, 0}, {7, 0}}};
-    double out[6][6];
-    for (int i = 0; i < 6; ++i)
-        for (int j = 0; j < 6; ++j) out[i][j] = 0.0;
     const int ncf = a.nf - 1, ncrf = a.nrf - 1;
+    const bool own = a.geometric || R == a.nrc - 2;
+    const double b_top = own ? 1.0 : 0.0, b_bot = own ? 0.0 : 1.0;
+    double out[CNT];
+#pragma unroll
+    for (int i = 0; i < CNT; ++i) out[i] = 0.0;
+#pragma unroll 1
     for (int k = 0; k < 8; ++k) {
-        const int h = LIST[W][k][0], w = LIST[W][k][1];
-        const int fx = 2 * X + SH[h][0], fy = 2 * Y + SH[h][1], fr = 2 * R + SH[h][2];
-        double P[6][6], A[6][6];
-        gca_local_P(fx, fy, fr, w, a.nrf, R, a.geometric, P);
-        const int64_t fcell = (((int64_t)d * ncf + fx) * ncf + fy) * ncrf + fr;
-        if constexpr (FINE_GEO) {
-            const double* geo_w = a.geo_f + ((((int64_t)d * ncf + fx) * ncf + fy) * 2 + w) * GEO_STRIDE;
-            double ksum = 0.0;
-            if (a.eta_cell_f) {
-                ksum = 6.0 * (double)a.eta_cell_f[fcell];
-            } else {
-                for (int j = 0; j < 6; ++j)
-                    ksum += (double)a.eta_f[(((int64_t)d * a.nf + fx + WOFF[w][j][0]) * a.nf + fy + WOFF[w][j][1]) *
-                                                a.nrf +
-                                            fr + WOFF[w][j][2]];
-            }
-            eps_block_geo<double>(geo_w, a.radii_f[fr], a.radii_f[fr + 1], ksum, q, p, A);
+        const GcaWedge f = GCA_LIST[W][k];
+        const int fx = 2 * X + f.sx, fy = 2 * Y + f.sy, fr = 2 * R + f.sr, w = f.w;
+        const int64_t fquad = ((int64_t)d * ncf + fx) * ncf + fy;
+        const double* gw = a.geo_f + (fquad * 2 + w) * GEO_STRIDE;
+        double ksum = 0.0;
+        if (a.eta_cell_f) {
+            ksum = 6.0 * (double)a.eta_cell_f[fquad * ncrf + fr];
         } else {
-            const int64_t ncellf = 10LL * ncf * ncf * ncrf;
-            stored_block<SF>(a.stored_f, ncellf, fcell, w, q, p, A);
+            // wedge w's lateral corners: (w, w), (1 - w, w), (w, 1 - w)
+            const int64_t l00 = ((int64_t)d * a.nf + fx + w) * a.nf + fy + w;
+            const int64_t l10 = l00 + (w ? -a.nf : a.nf), l01 = l00 + (w ? -1 : 1);
+            const T* e0 = a.eta_f + l00 * a.nrf + fr;
+            const T* e1 = a.eta_f + l10 * a.nrf + fr;
+            const T* e2 = a.eta_f + l01 * a.nrf + fr;
+            ksum = (double)e0[0] + (double)e1[0] + (double)e2[0] + (double)e0[1] + (double)e1[1] + (double)e2[1];
         }
-        // out += P^T A P
-        double T1[6][6];
-        for (int i = 0; i < 6; ++i)
-            for (int j = 0; j < 6; ++j) {
-                double s = 0.0;
-                for (int l = 0; l < 6; ++l) s += A[i][l] * P[l][j];
-                T1[i][j] = s;
+        const double r0 = a.radii_f[fr], r1 = a.radii_f[fr + 1];
+        const double half_dr = 0.5 * (r1 - r0), r_mid = 0.5 * (r0 + r1);
+        const double alpha = 1.0 / r_mid, beta = 1.0 / half_dr;
+        const double kwJ = ksum / 6.0 * r_mid * r_mid * half_dr * gw[9];
+        double G[6][3];
+#pragma unroll
+        for (int l = 0; l < 3; ++l) {
+            const double a1 = alpha * gw[l], a2 = alpha * gw[3 + l], z = beta * gw[6 + l];
+            const double a0 = -(a1 + a2);
+            const double g[6] = {a0 - z, a1 - z, a2 - z, a0 + z, a1 + z, a2 + z};
+#pragma unroll
+            for (int c = 0; c < 6; ++c) {
+                double v = 0.0;
+#pragma unroll
+                for (int i = 0; i < 6; ++i) v += GCA_P.C[W][k][i][c] * g[i];
+                G[c][l] = v;
             }
-        for (int i = 0; i < 6; ++i)
-            for (int j = 0; j < 6; ++j) {
-                double s = 0.0;
-                for (int l = 0; l < 6; ++l) s += P[l][i] * T1[l][j];
-                out[i][j] += s;
+#pragma unroll
+            for (int m = 0; m < 3; ++m) {
+                double v = 0.0;
+#pragma unroll
+                for (int i = 0; i < 3; ++i) v += GCA_P.B[W][k][i][m] * g[3 + i];
+                G[m][l] += b_bot * v;
+                G[m + 3][l] += b_top * v;
             }
+        }
+        // component blocks (q, p): rows r = node + 6 q, columns node + 6 p
+#pragma unroll
+        for (int i = 0; i < 6; ++i) {
+            const double h[3] = {kwJ * G[i][0], kwJ * G[i][1], kwJ * G[i][2]};
+#pragma unroll
+            for (int j = 0; j < 6; ++j) {
+                if (j >= i) {
+                    const double gg = h[0] * G[j][0] + h[1] * G[j][1] + h[2] * G[j][2];
+#pragma unroll
+                    for (int q = Q0; q < Q1; ++q)
+                        out[pk(i + 6 * q, j + 6 * q) - LO] += gg + (1.0 / 3.0) * (h[q] * G[j][q]);
+                }
+#pragma unroll
+                for (int q = Q0; q < Q1; ++q)
+#pragma unroll
+                    for (int p = q + 1; p < 3; ++p)
+                        out[pk(i + 6 * q, j + 6 * p) - LO] += h[p] * G[j][q] - (2.0 / 3.0) * (h[q] * G[j][p]);
+            }
+        }
     }
-    for (int i = 0; i < 6; ++i)
-        for (int j = 0; j < 6; ++j) {
-            const int r = i + 6 * q, c = j + 6 * p;
-            if (r <= c) a.stored_c[stored_at<S>(cell, W, pk(r, c))] = (S)out[i][j];
+    // vectors wholly inside the half as such, the shared one (entry 93 is no
+    // multiple of the vector length) by elements; the pad slot 171 is not read
+    constexpr int V = stored_vec<S>();
+    constexpr int VA = (LO + V - 1) / V, VB = (LO + CNT) / V;
+    S* base = a.stored_c + stored_at<S>(cell, W, 0);
+    VecOf<S>* o = reinterpret_cast<VecOf<S>*>(base);
+#pragma unroll
+    for (int v = VA; v < VB; ++v) {
+        VecOf<S> x;
+        x.x = (S)out[v * V - LO];
+        x.y = (S)out[v * V + 1 - LO];
+        if constexpr (V == 4) {
+            x.z = (S)out[v * V + 2 - LO];
+            x.w = (S)out[v * V + 3 - LO];
         }
+        o[v * 64] = x;
+    }
+#pragma unroll
+    for (int e = LO; e < LO + CNT; ++e)
+        if (e < VA * V || e >= VB * V) base[(e / V) * 64 * V + e % V] = (S)out[e - LO];
+}
+
+// grid: 4 blocks per tile of 64 coarse cells (coarse wedge, half)
+template <typename T, typename S, typename SF>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_gca_geo(GcaArgs<T, S, SF> a)
+{
+    const int64_t ncc = 10LL * (a.nc - 1) * (a.nc - 1) * (a.nrc - 1);
+    const int W = (int)(blockIdx.x & 1), half = (int)((blockIdx.x >> 1) & 1);
+    const int64_t cell = (int64_t)(blockIdx.x >> 2) * 64 + threadIdx.x;
+    if (cell >= ncc) return;
+    if (half == 0)
+        gca_geo_half<T, S, SF, 0>(a, cell, W);
+    else
+        gca_geo_half<T, S, SF, 1>(a, cell, W);
+}
+
+// Fine operator with stored matrices: a thread per (coarse cell, coarse wedge,
+// component block q <= p) sums P^T A_qp P over the 8 fine wedges, the 6x6 block
+// and its sum in registers (a whole wedge would not fit beside A).  What binds is
+// reading the fine matrices.  Level 5 -> 4 (0.90 GB read): 2.52 ms with the
+// products in local arrays and P built per thread, 0.34 ms now.
+template <typename T, typename S, typename SF, int Q, int P>
+__device__ __forceinline__ void gca_stored_block(const GcaArgs<T, S, SF>& a, int64_t cell, int W)
+{
+    const int R = (int)(cell % (a.nrc - 1));
+    int64_t lat = cell / (a.nrc - 1);
+    const int Y = (int)(lat % (a.nc - 1));
+    lat /= (a.nc - 1);
+    const int X = (int)(lat % (a.nc - 1));
+    const int d = (int)(lat / (a.nc - 1));
+    const int ncf = a.nf - 1, ncrf = a.nrf - 1;
+    const bool own = a.geometric || R == a.nrc - 2;
+    const double b_top = own ? 1.0 : 0.0, b_bot = own ? 0.0 : 1.0;
+    double out[6][6];
+#pragma unroll
+    for (int i = 0; i < 6; ++i)
+#pragma unroll
+        for (int j = 0; j < 6; ++j) out[i][j] = 0.0;
+#pragma unroll 1
+    for (int k = 0; k < 8; ++k) {
+        const GcaWedge f = GCA_LIST[W][k];
+        const int64_t fcell =
+            (((int64_t)d * ncf + 2 * X + f.sx) * ncf + 2 * Y + f.sy) * ncrf + 2 * R + f.sr;
+        const SF* base = a.stored_f + stored_at<SF>(fcell, f.w, 0);
+        constexpr int V = stored_vec<SF>();
+        double A[6][6];
+#pragma unroll
+        for (int i = 0; i < 6; ++i)
+#pragma unroll
+            for (int j = 0; j < 6; ++j) {
+                if (Q == P && j < i) continue;
+                const int e = pk(i + 6 * Q, j + 6 * P);
+                A[i][j] = (double)base[(e / V) * 64 * V + e % V];
+            }
+        if constexpr (Q == P) {
+#pragma unroll
+            for (int i = 1; i < 6; ++i)
+#pragma unroll
+                for (int j = 0; j < i; ++j) A[i][j] = A[j][i];
+        }
+        // weights of the fine dofs 3..5 per lane (the bracket depends on the cell)
+        double Pt[3][6];
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int m = 0; m < 3; ++m) {
+                Pt[i][m] = GCA_P.C[W][k][i + 3][m] + b_bot * GCA_P.B[W][k][i][m];
+                Pt[i][m + 3] = GCA_P.C[W][k][i + 3][m + 3] + b_top * GCA_P.B[W][k][i][m];
+            }
+#pragma unroll
+        for (int j = 0; j < 6; ++j) {
+            double t[6];  // column j of A P
+#pragma unroll
+            for (int i = 0; i < 6; ++i) {
+                double v = 0.0;
+#pragma unroll
+                for (int l = 0; l < 6; ++l) v += A[i][l] * (l < 3 ? GCA_P.C[W][k][l < 3 ? l : 0][j] : Pt[l < 3 ? 0 : l - 3][j]);
+                t[i] = v;
+            }
+#pragma unroll
+            for (int i = 0; i < 6; ++i) {
+                if (Q == P && j < i) continue;
+                double v = out[i][j];
+#pragma unroll
+                for (int l = 0; l < 6; ++l) v += (l < 3 ? GCA_P.C[W][k][l < 3 ? l : 0][i] : Pt[l < 3 ? 0 : l - 3][i]) * t[l];
+                out[i][j] = v;
+            }
+        }
+    }
+    constexpr int V = stored_vec<S>();
+    S* base = a.stored_c + stored_at<S>(cell, W, 0);
+#pragma unroll
+    for (int i = 0; i < 6; ++i)
+#pragma unroll
+        for (int j = 0; j < 6; ++j) {
+            if (Q == P && j < i) continue;
+            const int e = pk(i + 6 * Q, j + 6 * P);
+            base[(e / V) * 64 * V + e % V] = (S)out[i][j];
+        }
+}
+
+// grid: 12 blocks per tile of 64 coarse cells (coarse wedge, component block)
+template <typename T, typename S, typename SF>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_gca_stored(GcaArgs<T, S, SF> a)
+{
+    const int64_t ncc = 10LL * (a.nc - 1) * (a.nc - 1) * (a.nrc - 1);
+    const int part = (int)(blockIdx.x % 12), W = part / 6;
+    const int64_t cell = (int64_t)(blockIdx.x / 12) * 64 + threadIdx.x;
+    if (cell >= ncc) return;
+    switch (part % 6) {
+    case 0: gca_stored_block<T, S, SF, 0, 0>(a, cell, W); break;
+    case 1: gca_stored_block<T, S, SF, 0, 1>(a, cell, W); break;
+    case 2: gca_stored_block<T, S, SF, 0, 2>(a, cell, W); break;
+    case 3: gca_stored_block<T, S, SF, 1, 1>(a, cell, W); break;
+    case 4: gca_stored_block<T, S, SF, 1, 2>(a, cell, W); break;
+    default: gca_stored_block<T, S, SF, 2, 2>(a, cell, W); break;
+    }
 }
 
 // ---------------------------------------------------------------- selective GCA
@@ -1032,12 +1195,12 @@ template <typename T, typename S, typename SF>
 void launch_gca_build(const GcaArgs<T, S, SF>& a, bool fine_geo, hipStream_t s)
 {
     const int64_t ncc = 10LL * (a.nc - 1) * (a.nc - 1) * (a.nrc - 1);
-    const int64_t total = ncc * 12;
-    const dim3 gr((unsigned)((total + 127) / 128)), bl(128);
+    const int64_t tiles = (ncc + 63) / 64;
+    TN_REQUIRE(12 * tiles < (1LL << 31), "GCA: mesh too large");
     if (fine_geo)
-        hipLaunchKernelGGL((k_gca_build<T, S, SF, true>), gr, bl, 0, s, a);
+        hipLaunchKernelGGL((k_gca_geo<T, S, SF>), dim3((unsigned)(4 * tiles)), dim3(64), 0, s, a);
     else
-        hipLaunchKernelGGL((k_gca_build<T, S, SF, false>), gr, bl, 0, s, a);
+        hipLaunchKernelGGL((k_gca_stored<T, S, SF>), dim3((unsigned)(12 * tiles)), dim3(64), 0, s, a);
     TN_HIP(hipGetLastError());
 }
 

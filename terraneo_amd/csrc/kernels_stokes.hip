@@ -29,41 +29,6 @@ namespace {
 using cellops::dot3;
 using cellops::V3;
 
-__device__ constexpr int WOFF[2][6][3] = {{{0, 0, 0}, {1, 0, 0}, {0, 1, 0}, {0, 0, 1}, {1, 0, 1}, {0, 1, 1}},
-                                         {{1, 1, 0}, {0, 1, 0}, {1, 0, 0}, {1, 1, 1}, {0, 1, 1}, {1, 0, 1}}};
-__device__ constexpr double Q6P[6][3] = {{0.6666666666666666, 0.1666666666666667, -0.5773502691896257},
-                                        {0.1666666666666667, 0.6666666666666666, -0.5773502691896257},
-                                        {0.1666666666666667, 0.1666666666666667, -0.5773502691896257},
-                                        {0.6666666666666666, 0.1666666666666667, 0.5773502691896257},
-                                        {0.1666666666666667, 0.6666666666666666, 0.5773502691896257},
-                                        {0.1666666666666667, 0.1666666666666667, 0.5773502691896257}};
-__device__ constexpr double Q6W = 0.1666666666666667;
-
-__device__ inline double shape_lat(int k, double xi, double eta)
-{
-    const int m = k % 3;
-    return m == 0 ? 1.0 - xi - eta : (m == 1 ? xi : eta);
-}
-__device__ inline double shape_rad(int k, double zeta) { return k < 3 ? 0.5 * (1 - zeta) : 0.5 * (1 + zeta); }
-
-struct WedgeGeo {
-    double P[3][3];  // lateral vertices (unit sphere)
-    double r1, r2;
-};
-
-__device__ inline void load_wedge(const double* coords, const double* radii, int n, int d, int x, int y, int rc, int w,
-                                  WedgeGeo& G)
-{
-    for (int k = 0; k < 3; ++k) {
-        const double* c = coords + 3 * (((int64_t)d * n + x + WOFF[w][k][0]) * n + y + WOFF[w][k][1]);
-        G.P[k][0] = c[0];
-        G.P[k][1] = c[1];
-        G.P[k][2] = c[2];
-    }
-    G.r1 = radii[rc];
-    G.r2 = radii[rc + 1];
-}
-
 // ---------------------------------------------------------------------------
 // B and B^T by per-wedge moments.
 //
@@ -281,7 +246,7 @@ __device__ inline void grad_wedge(const LatWedge<T>& L, const T (*M)[3], const R
 }
 
 // Lateral corners of a quad: k = 0 (x, y), 1 (x+1, y), 2 (x, y+1), 3 (x+1, y+1);
-// wedge w's vertices 0, 1, 2 in that numbering (WOFF[w][0..2]).
+// wedge w's vertices 0, 1, 2 in that numbering.
 __device__ constexpr int WK[2][3] = {{0, 1, 2}, {3, 2, 1}};
 
 // B: a wave per coarse lateral quad (X, Y) and chunk of 64 coarse radial
@@ -360,7 +325,7 @@ __global__ __launch_bounds__(256) void k_div(DivArgs<T> a)
                     const V3<T> u2[2] = {u[k2][frw], u[k2][frw + 1]};
                     div_wedge(L, M, rm[frw], u0, u1, u2, out);
                 }
-                // coarse corners of wedge w: WOFF[w][il] in the k numbering
+                // coarse corners of wedge w in the k numbering
 #pragma unroll
                 for (int il = 0; il < 3; ++il) {
                     acc[WK[w][il]][0] += out[il][0];
@@ -507,77 +472,12 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(3))) voi
     march::run<T, W>(op, a.nf, a.nrf, a.seg, a.guard);
 }
 
-// One row sum of a wedge's k-weighted mass matrix (kmass.hpp): vertex j of
-// wedge w of hex cell (d, x, y, rc), the reference's 6-point quadrature.
-template <typename T>
-__device__ double kmass_wedge_row(const MassArgs<T>& a, int d, int x, int y, int rc, int w, int jrow)
-{
-    WedgeGeo G;
-    load_wedge(a.coords, a.radii, a.n, d, x, y, rc, w, G);
-    int64_t idx[6];
-    for (int j = 0; j < 6; ++j)
-        idx[j] = (((int64_t)d * a.n + x + WOFF[w][j][0]) * a.n + y + WOFF[w][j][1]) * a.nr + rc + WOFF[w][j][2];
-    const double gr = 0.5 * (G.r2 - G.r1);
-    double M[6][6] = {{0}};
-    for (int q = 0; q < 6; ++q) {
-        const double* qp = Q6P[q];
-        double Jl[3][3];  // lateral Jacobian (kernel_helpers.hpp:153-176)
-        for (int c = 0; c < 3; ++c) {
-            Jl[c][0] = G.P[1][c] - G.P[0][c];
-            Jl[c][1] = G.P[2][c] - G.P[0][c];
-            Jl[c][2] = (1 - qp[0] - qp[1]) * G.P[0][c] + qp[0] * G.P[1][c] + qp[1] * G.P[2][c];
-        }
-        const double det = fabs(Jl[0][0] * (Jl[1][1] * Jl[2][2] - Jl[1][2] * Jl[2][1]) -
-                                Jl[0][1] * (Jl[1][0] * Jl[2][2] - Jl[1][2] * Jl[2][0]) +
-                                Jl[0][2] * (Jl[1][0] * Jl[2][1] - Jl[1][1] * Jl[2][0]));
-        const double rr = G.r1 + 0.5 * (G.r2 - G.r1) * (1 + qp[2]);
-        double N6[6];
-        for (int j = 0; j < 6; ++j) N6[j] = shape_lat(j, qp[0], qp[1]) * shape_rad(j, qp[2]);
-        double kq = 0.0;
-        for (int j = 0; j < 6; ++j) kq += N6[j] * (double)a.k[idx[j]];
-        const double f = Q6W * kq * rr * rr * gr * det;
-        for (int i = 0; i < 6; ++i)
-            for (int j = 0; j < 6; ++j) M[i][j] += f * N6[i] * N6[j];
-    }
-    double s = 0.0;
-    for (int j = 0; j < 6; ++j) s += M[jrow][j];
-    return s;
-}
-
-// lumped k-weighted mass (kmass.hpp): row sums of the k-weighted wedge mass
-// matrices, as a gather (setup only): one thread per node copy adds the row
-// sums of the wedges of its diamond that contain it, in a fixed order, so the
-// result repeats bit for bit (the Schur-complement diagonal of the solves)
-template <typename T>
-__global__ __launch_bounds__(128) void k_kmass_lumped(MassArgs<T> a)
-{
-    const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int n = a.n, nr = a.nr, ncr = nr - 1, ncl = n - 1;
-    if (tid >= 10LL * n * n * nr) return;
-    const int lev = (int)(tid % nr);
-    int64_t lat = tid / nr;
-    const int Y = (int)(lat % n);
-    lat /= n;
-    const int X = (int)(lat % n);
-    const int d = (int)(lat / n);
-    double acc = 0.0;
-    for (int rc = lev - 1; rc <= lev; ++rc) {
-        if (rc < 0 || rc >= ncr) continue;
-        for (int qx = X - 1; qx <= X; ++qx) {
-            if (qx < 0 || qx >= ncl) continue;
-            for (int qy = Y - 1; qy <= Y; ++qy) {
-                if (qy < 0 || qy >= ncl) continue;
-                for (int w = 0; w < 2; ++w)
-                    for (int j = 0; j < 6; ++j)
-                        if (qx + WOFF[w][j][0] == X && qy + WOFF[w][j][1] == Y && rc + WOFF[w][j][2] == lev)
-                            acc += kmass_wedge_row(a, d, qx, qy, rc, w, j);
-            }
-        }
-    }
-    a.y[tid] = (T)acc;
-}
-
-// VectorMass as a gather: one thread per node copy writes y_i = sum over the
+// VectorMass and the lumped k-mass (kmass.hpp) as a gather.  The lumped k-mass is
+// the row sum of the k-weighted matrix: with sum_j N_j = 1 its entry is
+// sum_q w_q k_h(q) N_i(q) |det|, the consistent mass matrix applied to the nodal
+// k by the same rule, so both are this kernel (the Schur diagonal of 0.36 M
+// pressure nodes took 426 us as quadrature per node and wedge, under 10 us here).
+// One thread per node copy writes y_i = sum over the
 // wedges of its diamond that contain it of (M_w x)_i; no atomics, so the
 // result repeats bit for bit.  The reference's Felippa 3x2 rule factors into
 // the 3-point triangle rule, exact for the lateral products (the P1 triangle
@@ -672,17 +572,12 @@ void launch_grad(const GradArgs<T>& a, hipStream_t s)
 }
 
 template <typename T>
-void launch_mass(const MassArgs<T>& a, bool lumped_k, hipStream_t s)
+void launch_mass(const MassArgs<T>& a, hipStream_t s)
 {
-    if (lumped_k) {
-        const int64_t N = 10LL * a.n * a.n * a.nr;
-        hipLaunchKernelGGL((k_kmass_lumped<T>), dim3((unsigned)((N + 127) / 128)), dim3(128), 0, s, a);
-    } else {
-        TN_REQUIRE(a.ncomp >= 1 && a.ncomp <= 3, "mass: ncomp must be 1..3");
-        const int64_t N = 10LL * a.n * a.n * a.nr;
-        TN_REQUIRE(a.geo, "mass: wedge table missing");
-        hipLaunchKernelGGL((k_mass_stencil<T>), dim3((unsigned)((N + 255) / 256)), dim3(256), 0, s, a);
-    }
+    TN_REQUIRE(a.ncomp >= 1 && a.ncomp <= 3, "mass: ncomp must be 1..3");
+    const int64_t N = 10LL * a.n * a.n * a.nr;
+    TN_REQUIRE(a.geo, "mass: wedge table missing");
+    hipLaunchKernelGGL((k_mass_stencil<T>), dim3((unsigned)((N + 255) / 256)), dim3(256), 0, s, a);
     TN_HIP(hipGetLastError());
 }
 
@@ -690,7 +585,7 @@ template void launch_div<double>(const DivArgs<double>&, hipStream_t);
 template void launch_div<float>(const DivArgs<float>&, hipStream_t);
 template void launch_grad<double>(const GradArgs<double>&, hipStream_t);
 template void launch_grad<float>(const GradArgs<float>&, hipStream_t);
-template void launch_mass<double>(const MassArgs<double>&, bool, hipStream_t);
-template void launch_mass<float>(const MassArgs<float>&, bool, hipStream_t);
+template void launch_mass<double>(const MassArgs<double>&, hipStream_t);
+template void launch_mass<float>(const MassArgs<float>&, hipStream_t);
 
 }  // namespace tn

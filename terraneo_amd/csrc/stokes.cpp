@@ -214,9 +214,8 @@ int tn_vector_mass_apply(const tn_mesh* m, int dtype, const void* x, void* y, tn
     auto& L = const_cast<tn_mesh*>(m)->lvl.dev();
     auto go = [&](auto* yy) {
         using T = std::remove_pointer_t<decltype(yy)>;
-        tn::launch_fill<T>(yy, 3 * L.N, T(0), (hipStream_t)s);
-        tn::MassArgs<T> a{L.d_coords.p, L.d_radii.p, L.n, L.nr, 3, (const T*)x, nullptr, yy, L.d_geo.p};
-        tn::launch_mass<T>(a, false, (hipStream_t)s);
+        tn::MassArgs<T> a{L.d_radii.p, L.n, L.nr, 3, (const T*)x, yy, L.d_geo.p};
+        tn::launch_mass<T>(a, (hipStream_t)s);
         tn::launch_interface_sum<T>(L, 3, yy, (hipStream_t)s);
     };
     if (dtype == TN_F64)
@@ -233,9 +232,8 @@ int tn_kmass_lumped(const tn_mesh* m, int dtype, const void* k, void* d, tn_stre
     auto& L = const_cast<tn_mesh*>(m)->lvl.dev();
     auto go = [&](auto* dd) {
         using T = std::remove_pointer_t<decltype(dd)>;
-        tn::launch_fill<T>(dd, L.N, T(0), (hipStream_t)s);
-        tn::MassArgs<T> a{L.d_coords.p, L.d_radii.p, L.n, L.nr, 1, nullptr, (const T*)k, dd};
-        tn::launch_mass<T>(a, true, (hipStream_t)s);
+        tn::MassArgs<T> a{L.d_radii.p, L.n, L.nr, 1, (const T*)k, dd, L.d_geo.p};
+        tn::launch_mass<T>(a, (hipStream_t)s);
         tn::launch_interface_sum<T>(L, 1, dd, (hipStream_t)s);
     };
     if (dtype == TN_F64)
@@ -345,9 +343,8 @@ int tn_stokes_rhs_from_temperature(tn_stokes* K, const void* temperature, double
                            (const T*)temperature, L.d_coords.p, L.N, L.nr, rayleigh);
         TN_HIP(hipGetLastError());
         // f_u = M g, additive communication (vector_mass.hpp:59-153)
-        tn::launch_fill<T>(fu, 3 * L.N, T(0), st);
-        tn::MassArgs<T> a{L.d_coords.p, L.d_radii.p, L.n, L.nr, 3, g, nullptr, fu, L.d_geo.p};
-        tn::launch_mass<T>(a, false, st);
+        tn::MassArgs<T> a{L.d_radii.p, L.n, L.nr, 3, g, fu, L.d_geo.p};
+        tn::launch_mass<T>(a, st);
         tn::launch_interface_sum<T>(L, 3, fu, st);
         // strong enforcement of the velocity BCs on the right-hand side
         // (mantlecirculation.cpp:890-898): homogeneous Dirichlet rows zero,

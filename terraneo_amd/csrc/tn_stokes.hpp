@@ -46,13 +46,11 @@ constexpr int grad_march_waves()
 
 template <typename T>
 struct MassArgs {
-    const double* coords;
     const double* radii;
     int n, nr, ncomp;
-    const T* x;  // input (vector mass)
-    const T* k;  // coefficient (lumped k-mass)
-    T* y;        // output: written (vector mass), accumulated (lumped k-mass)
-    const double* geo = nullptr;  // the mesh's wedge table [10][n-1][n-1][2][GEO_STRIDE] (vector mass)
+    const T* x;         // input field (lumped k-mass: the coefficient)
+    T* y;               // output, every node copy written (before the interface sum)
+    const double* geo;  // the mesh's wedge table [10][n-1][n-1][2][GEO_STRIDE]
 };
 
 template <typename T>
@@ -60,6 +58,6 @@ void launch_div(const DivArgs<T>& a, hipStream_t s);
 template <typename T>
 void launch_grad(const GradArgs<T>& a, hipStream_t s);
 template <typename T>
-void launch_mass(const MassArgs<T>& a, bool lumped_k, hipStream_t s);
+void launch_mass(const MassArgs<T>& a, hipStream_t s);
 
 }  // namespace tn
