@@ -471,13 +471,20 @@ int tn_fv_to_fe(tn_fv* fv, const double* Tfv, double* Tfe, const tn_krylov_optio
     launch_interface_sum<double>(L, 1, (double*)B.b[0].p, c.s);
     struct MassOp : LinOp {
         MeshLevel* L;
-        void apply(Ctx& c, const BVec& x, const BVec& y) override
+        void mass(Ctx& c, const BVec& x, const BVec& y, double* part)
         {
             double* yy = (double*)y.b[0].p;
-            MassArgs<double> a{L->d_radii.p, L->n, L->nr, 1, (const double*)x.b[0].p, yy, L->d_geo.p};
+            MassArgs<double> a{L->d_radii.p, L->n, L->nr, 1, (const double*)x.b[0].p, yy, L->d_geo.p, part};
             launch_mass<double>(a, c.s);
-            launch_interface_sum<double>(*L, 1, yy, c.s);
         }
+        void apply(Ctx& c, const BVec& x, const BVec& y) override
+        {
+            mass(c, x, y, nullptr);
+            launch_interface_sum<double>(*L, 1, (double*)y.b[0].p, c.s);
+        }
+        void apply_dot(Ctx& c, const BVec& x, const BVec& y, double* part) override { mass(c, x, y, part); }
+        int dot_blocks(const BVec&) const override { return mass_blocks(L->n); }
+        bool dot_partial() const override { return true; }
     } op;
     op.L = &L;
     std::vector<BVec> t;

@@ -130,4 +130,37 @@ void dev_free(void* ptr)
     if (c.live == 0) release(c);
 }
 
+// Pinned pages: a solve takes one or two; freed pages are kept (as many as
+// were ever in use at once).
+namespace {
+struct Pages {
+    std::mutex mu;
+    std::vector<double*> idle;
+};
+Pages& pages()
+{
+    static Pages* p = new Pages;
+    return *p;
+}
+}  // namespace
+
+HostPage::HostPage() : p(nullptr)
+{
+    {
+        std::lock_guard<std::mutex> lk(pages().mu);
+        if (!pages().idle.empty()) {
+            p = pages().idle.back();
+            pages().idle.pop_back();
+            return;
+        }
+    }
+    TN_HIP(hipHostMalloc((void**)&p, HOST_PAGE_BYTES, hipHostMallocPortable));
+}
+
+HostPage::~HostPage()
+{
+    std::lock_guard<std::mutex> lk(pages().mu);
+    pages().idle.push_back(p);
+}
+
 }  // namespace tn

@@ -8,6 +8,7 @@
 // (fs/fs penalty).
 #include "tn_coarse.hpp"
 #include "tn_internal.hpp"
+#include "tn_reduce.hpp"
 
 namespace tn {
 namespace {
@@ -41,40 +42,6 @@ __global__ void k_lincomb(T* __restrict__ y, int64_t count, LinArgs<T> a)
     }
 }
 
-__device__ inline double wave_sum(double v)
-{
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-
-// Block total of `v`, valid in thread 0 (no atomics).
-__device__ inline double block_total(double v)
-{
-    __shared__ double part[16];
-    v = wave_sum(v);
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    if (lane == 0) part[wv] = v;
-    __syncthreads();
-    double s = 0.0;
-    if (wv == 0) {
-        const int nw = blockDim.x >> 6;
-        s = lane < nw ? part[lane] : 0.0;
-        s = wave_sum(s);
-    }
-    __syncthreads();
-    return s;
-}
-
-// The block's total of `v` into part[blockIdx.x].  Reductions leave one
-// partial per block and k_reduce_finalize adds them in a fixed order, so a
-// reduction gives the same bits on every run (no floating-point atomics).
-__device__ inline void block_partial(double v, double* __restrict__ part)
-{
-    const double t = block_total(v);
-    if (threadIdx.x == 0) part[blockIdx.x] = t;
-}
-
 // out[k] += sum over b < nblk of part[k * nblk + b], k < nk (one block)
 __global__ __launch_bounds__(256) void k_reduce_finalize(const double* __restrict__ part, int nblk, int nk,
                                                          double* __restrict__ out)
@@ -102,6 +69,88 @@ struct ColumnWalk {
     {
     }
 };
+
+// ---- conjugate gradients without a preconditioner, scalars on the device
+// (CgState in tn_internal.hpp).  An iteration is the product with its dot
+// (p, A p), this update and the direction; both kernels add the preceding
+// reduction's partials themselves, so no launch and no host round trip stands
+// between them.  A solve that has converged leaves the later kernels of the
+// queue as returns (done < it).
+// x += alpha p, r -= alpha A p, alpha = (r, r) / (p, A p); part_rr: blocks' parts of
+// the new (r, r).  With st.groups the copies of a node hold their diamond's part of
+// A p only, and the update adds them up (the interface sum's order) on the way.
+constexpr int CG_WAVES = 4;
+template <typename T>
+__global__ __launch_bounds__(64 * CG_WAVES) void k_cg_update(T* __restrict__ x, T* __restrict__ r, const T* __restrict__ p,
+                                                   const T* __restrict__ ap, const uint8_t* __restrict__ owned_lat,
+                                                   int64_t N, int nr, int ncomp, CgState st, int it)
+{
+    const double done = st.ctl[CgState::DONE];
+    const double rr = st.rr[CgState::slot(it - 1)];
+    const double pap = partials_total(st.part_pap, st.npap);
+    if (done != 0.0 && done < (double)it) return;
+    const T alpha = (T)(rr / pap);
+    double s = 0.0;
+    const int lane = threadIdx.x & 63;
+    const int nlat = (int)(N / nr), ncol = nlat * ncomp, step = gridDim.x * CG_WAVES;
+    const int4* groups = reinterpret_cast<const int4*>(st.groups);
+    for (int col = blockIdx.x * CG_WAVES + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); col < ncol; col += step) {
+        const int c = col / nlat, lat = col - c * nlat;
+        const bool own = owned_lat[lat];
+        const int g = groups ? st.group_of[lat] : -1;
+        const int64_t base = (int64_t)col * nr;
+        for (int k = lane; k < nr; k += 64) {
+            const int64_t i = base + k;
+            const T xv = x[i], pv = p[i], rv = r[i];
+            T av;
+            if (g < 0) {
+                av = ap[i];
+            } else {
+                const int4 q = groups[2 * g], q2 = groups[2 * g + 1];
+                const T* ac = ap + c * N + k;
+                double v = 0.0 + (double)ac[(int64_t)q.x * nr] + (double)ac[(int64_t)q.y * nr];
+                if (q.z >= 0) v += (double)ac[(int64_t)q.z * nr];
+                if (q.w >= 0) v += (double)ac[(int64_t)q.w * nr];
+                if (q2.x >= 0) v += (double)ac[(int64_t)q2.x * nr];
+                if (q2.y >= 0) v += (double)ac[(int64_t)q2.y * nr];
+                if (q2.z >= 0) v += (double)ac[(int64_t)q2.z * nr];
+                if (q2.w >= 0) v += (double)ac[(int64_t)q2.w * nr];
+                av = (T)v;
+            }
+            x[i] = xv + alpha * pv;
+            const T rn = rv - alpha * av;
+            r[i] = rn;
+            if (own) s += (double)rn * (double)rn;
+        }
+    }
+    block_partial(s, st.part_rr);
+}
+
+// p = r + beta p, beta = the new (r, r) over the last; records (r, r) and the stopping test
+template <typename T>
+__global__ __launch_bounds__(256) void k_cg_direction(T* __restrict__ p, const T* __restrict__ r, int64_t count,
+                                                      CgState st, int it)
+{
+    const double done = st.ctl[CgState::DONE];
+    const double rr_old = st.rr[CgState::slot(it - 1)];
+    const double rr = partials_total(st.part_rr, st.nrr);
+    if (done != 0.0 && done < (double)it) return;
+    const T beta = (T)(rr / rr_old);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        st.rr[CgState::slot(it)] = rr;
+        const double res = sqrt(rr);
+        if (res / st.ctl[CgState::R0] <= st.rtol || res < st.atol) st.ctl[CgState::DONE] = (double)it;
+    }
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (int64_t)gridDim.x * blockDim.x)
+        p[i] = r[i] + beta * p[i];
+}
+
+__global__ void k_cg_begin(CgState st, const double* __restrict__ rr0)
+{
+    st.rr[CgState::slot(0)] = rr0[0];
+    st.ctl[CgState::DONE] = 0.0;
+    st.ctl[CgState::R0] = sqrt(rr0[0]);
+}
 
 template <typename T>
 __global__ __launch_bounds__(256) void k_dot_owned(const T* __restrict__ a, const T* __restrict__ b,
@@ -506,6 +555,34 @@ static void launch_reduce_finalize(const double* part, int nblk, int nk, double*
 
 int reduce_blocks(const MeshLevel& m, int ncomp) { return (int)grid_for(m.N / m.nr * ncomp, 4, REDUCE_MAX_BLOCKS); }
 
+int cg_update_blocks(const MeshLevel& m, int ncomp) { return (int)grid_for(m.N / m.nr * ncomp, CG_WAVES, REDUCE_MAX_BLOCKS / 2); }
+
+void launch_cg_begin(const CgState& st, const double* rr0, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_cg_begin, dim3(1), dim3(1), 0, s, st, rr0);
+    TN_HIP(hipGetLastError());
+}
+
+template <typename T>
+void launch_cg_step(const MeshLevel& m, int ncomp, T* x, T* r, T* p, const T* ap, const CgState& st, int it,
+                    hipStream_t s)
+{
+    hipLaunchKernelGGL(k_cg_update<T>, dim3(st.nrr), dim3(64 * CG_WAVES), 0, s, x, r, p, ap, m.d_owned_lat.p, m.N, m.nr, ncomp,
+                       st, it);
+    TN_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_cg_direction<T>, dim3(grid_for(m.N * ncomp, 256, 1024)), dim3(256), 0, s, p, r, m.N * ncomp, st,
+                       it);
+    TN_HIP(hipGetLastError());
+}
+
+template <typename T>
+void launch_dot_partials(const MeshLevel& m, int ncomp, const T* a, const T* b, double* part_dev, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_dot_owned<T>, dim3(reduce_blocks(m, ncomp)), dim3(256), 0, s, a, b, m.d_owned_lat.p, m.N, m.nr,
+                       ncomp, part_dev);
+    TN_HIP(hipGetLastError());
+}
+
 template <typename T>
 void launch_dot_owned(const MeshLevel& m, int ncomp, const T* a, const T* b, double* out_dev, double* part_dev,
                       hipStream_t s)
@@ -674,6 +751,8 @@ template void launch_cast<float, double>(float*, const double*, int64_t, hipStre
     template void launch_fill<T>(T*, int64_t, T, hipStream_t);                                                   \
     template void launch_lincomb<T>(int64_t, T*, int, const double*, const T* const*, double, hipStream_t);     \
     template void launch_dot_owned<T>(const MeshLevel&, int, const T*, const T*, double*, double*, hipStream_t); \
+    template void launch_dot_partials<T>(const MeshLevel&, int, const T*, const T*, double*, hipStream_t);       \
+    template void launch_cg_step<T>(const MeshLevel&, int, T*, T*, T*, const T*, const CgState&, int, hipStream_t); \
     template void launch_sub_scaled<T>(T*, int64_t, const double*, double, hipStream_t);                         \
     template void launch_sum_owned<T>(const MeshLevel&, const T*, double*, double*, hipStream_t);                 \
     template void launch_axpy_dot<T>(const MeshLevel&, int, T*, double, const T*, const T*, double*, double*,    \

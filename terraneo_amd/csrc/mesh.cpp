@@ -234,13 +234,17 @@ void MeshLevel::upload()
     std::vector<float> gf(geo.begin(), geo.end());
     d_geo_f.upload(gf);
     d_owned_lat.upload(owned_lat);
-    std::vector<int32_t> pad((size_t)GRP_PAD * ngroups(), -1);
+    std::vector<int32_t> pad((size_t)GRP_PAD * ngroups(), -1), of(owned_lat.size(), -1);
     for (int g = 0; g < ngroups(); ++g) {
         const int cnt = grp_off[g + 1] - grp_off[g];
         TN_REQUIRE(cnt >= 2 && cnt <= GRP_PAD, "mesh: node copies out of range");
-        for (int k = 0; k < cnt; ++k) pad[(size_t)GRP_PAD * g + k] = grp_mem[grp_off[g] + k];
+        for (int k = 0; k < cnt; ++k) {
+            pad[(size_t)GRP_PAD * g + k] = grp_mem[grp_off[g] + k];
+            of[grp_mem[grp_off[g] + k]] = g;
+        }
     }
     d_grp_pad.upload(pad);
+    d_grp_of.upload(of);
     d_scratch.alloc(64);
     d_part.alloc(REDUCE_PART_DOUBLES);
     uploaded = true;

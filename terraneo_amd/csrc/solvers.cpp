@@ -435,8 +435,113 @@ PCG::PCG(KrylovParams p, std::vector<BVec> tmps, Solver* prec) : p_(p), t_(std::
     TN_REQUIRE(t_.size() >= 4, "PCG needs 4 temporaries");
 }
 
+void LinOp::apply_dot(Ctx& c, const BVec& x, const BVec& y, double* part)
+{
+    apply(c, x, y);
+    const Field& f = x.b[0];
+    if (f.dtype == TN_F64)
+        launch_dot_partials<double>(*f.m, f.ncomp, (const double*)y.b[0].p, (const double*)f.p, part, c.s);
+    else
+        launch_dot_partials<float>(*f.m, f.ncomp, (const float*)y.b[0].p, (const float*)f.p, part, c.s);
+}
+
+int LinOp::dot_blocks(const BVec& x) const { return reduce_blocks(*x.b[0].m, x.b[0].ncomp); }
+
+namespace {
+struct Event {
+    hipEvent_t e = nullptr;
+    Event() { TN_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming)); }
+    ~Event() { (void)hipEventDestroy(e); }
+    Event(const Event&) = delete;
+    Event& operator=(const Event&) = delete;
+};
+}  // namespace
+
+// The recurrence of solve() with z = r, so that (z, r) is (r, r).  The queue is fed in batches of BATCH iterations; a batch's
+// (r, r) values come back behind it and are read while the next one runs, so a
+// solve that has converged runs at most two batches of kernels that return at once.
+void PCG::solve_queued(Ctx& c, LinOp& A, const BVec& x, const BVec& b)
+{
+    constexpr int BATCH = 8;
+    static_assert(CgState::RING % BATCH == 0 && CgState::RING >= 4 * BATCH, "ring of residuals");
+    BVec &r = t_[0], &pp = t_[1], &ap = t_[2];
+    const Field& f = x.b[0];
+    info = IterInfo{};
+    A.apply(c, x, r);
+    v_lincomb(c, r, {1.0, -1.0}, {&b, &r});
+    v_assign(c, pp, r);
+    const double r0 = std::sqrt(v_dot(c, r, r));  // (leaves (r, r) in c.red[0])
+    info.initial_residual = info.final_residual = r0;
+    info.history.push_back(r0);
+    if (r0 < p_.atol || p_.max_iterations < 1) return;
+    CgState st{};
+    st.npap = A.dot_blocks(x);
+    st.nrr = cg_update_blocks(*f.m, f.ncomp);
+    const size_t words = (size_t)CgState::RING + 3 + st.npap + st.nrr;
+    if (scalars_.n != words) scalars_.alloc(words);
+    st.ctl = scalars_.p;
+    st.rr = scalars_.p + 2;
+    st.part_pap = st.rr + CgState::RING + 1;
+    st.part_rr = st.part_pap + st.npap;
+    if (A.dot_partial()) {
+        st.groups = f.m->d_grp_pad.p;
+        st.group_of = f.m->d_grp_of.p;
+    }
+    st.rtol = p_.rtol;
+    st.atol = p_.atol;
+    launch_cg_begin(st, c.red.p, c.s);
+    HostPage page;  // per batch in flight: BATCH residuals and the control word
+    Event ev[2];
+    auto host = [&](int k) { return page.p + (k & 1) * (BATCH + 1); };
+    auto drain = [&](int k) {  // true: converged within batch k
+        TN_HIP(hipEventSynchronize(ev[k & 1].e));
+        check_march_status();
+        const double* h = host(k);
+        const int done = (int)h[BATCH];
+        for (int it = k * BATCH + 1; it <= std::min((k + 1) * BATCH, p_.max_iterations); ++it) {
+            if (done && it > done) break;
+            const double res = std::sqrt(h[it - k * BATCH - 1]);
+            info.iterations = it;
+            info.final_residual = res;
+            info.history.push_back(res);
+        }
+        return done && done <= (k + 1) * BATCH;
+    };
+    const int batches = (p_.max_iterations + BATCH - 1) / BATCH;
+    try {
+        for (int k = 0; k < batches; ++k) {
+            for (int it = k * BATCH + 1; it <= std::min((k + 1) * BATCH, p_.max_iterations); ++it) {
+                A.apply_dot(c, pp, ap, st.part_pap);
+                if (f.dtype == TN_F64)
+                    launch_cg_step<double>(*f.m, f.ncomp, (double*)f.p, (double*)r.b[0].p, (double*)pp.b[0].p,
+                                           (const double*)ap.b[0].p, st, it, c.s);
+                else
+                    launch_cg_step<float>(*f.m, f.ncomp, (float*)f.p, (float*)r.b[0].p, (float*)pp.b[0].p,
+                                          (const float*)ap.b[0].p, st, it, c.s);
+            }
+            TN_HIP(hipMemcpyAsync(host(k), st.rr + CgState::slot(k * BATCH + 1), BATCH * sizeof(double),
+                                  hipMemcpyDeviceToHost, c.s));
+            TN_HIP(hipMemcpyAsync(host(k) + BATCH, st.ctl + CgState::DONE, sizeof(double), hipMemcpyDeviceToHost, c.s));
+            TN_HIP(hipEventRecord(ev[k & 1].e, c.s));
+            if (k > 0 && drain(k - 1)) {
+                // the batch behind returns at once; its copies still write the page
+                TN_HIP(hipEventSynchronize(ev[k & 1].e));
+                return;
+            }
+        }
+        drain(batches - 1);
+    } catch (...) {
+        (void)hipStreamSynchronize(c.s);  // the page is still being written
+        throw;
+    }
+}
+
 void PCG::solve(Ctx& c, LinOp& A, const BVec& x, const BVec& b)
 {
+    if (!prec_ && x.nb == 1) {
+        solve_queued(c, A, x, b);
+        return;
+    }
     Solver& P = prec_ ? *prec_ : (Solver&)id_;
     BVec &r = t_[0], &pp = t_[1], &ap = t_[2], &z = t_[3];
     info = IterInfo{};

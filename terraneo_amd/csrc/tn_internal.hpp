@@ -36,6 +36,15 @@ void set_last_error(const std::string& msg);
 // device memory of the library's objects, with a bounded cache of freed blocks (devmem.cpp)
 void* dev_alloc(size_t bytes);
 void dev_free(void* ptr);
+// a page of pinned host memory for results copied behind queued work
+constexpr size_t HOST_PAGE_BYTES = 4096;
+struct HostPage {
+    double* p;
+    HostPage();
+    ~HostPage();
+    HostPage(const HostPage&) = delete;
+    HostPage& operator=(const HostPage&) = delete;
+};
 
 template <typename T>
 struct DevBuf {
@@ -97,6 +106,7 @@ struct MeshLevel {
     // node has at most five copies, at the icosahedron's poles)
     static constexpr int GRP_PAD = 8;
     DevBuf<int32_t> d_grp_pad;
+    DevBuf<int32_t> d_grp_of;  // [10][n][n]: a lateral node's group, -1 without other copies
     DevBuf<double> d_scratch;  // reduction results (doubles)
     DevBuf<double> d_part;     // per-block partial sums of the reductions (REDUCE_PART_DOUBLES)
     bool uploaded = false;
@@ -143,6 +153,31 @@ constexpr int REDUCE_MAX_BLOCKS = 2048;
 constexpr int REDUCE_PART_DOUBLES = 16 * (REDUCE_MAX_BLOCKS / 2);
 // blocks (= partial sums) of a dot over ncomp fields of mesh m
 int reduce_blocks(const MeshLevel& m, int ncomp);
+
+// Device scalars of a conjugate-gradient solve without preconditioner (k_cg_update).
+// rr[slot(it)]: (r, r) after iteration it, a ring the host drains by batches;
+// ctl[DONE]: the iteration that met the stopping test, 0 before.
+struct CgState {
+    static constexpr int RING = 64;
+    static constexpr int DONE = 0, R0 = 1;
+    double *rr, *ctl;
+    double *part_pap, *part_rr;  // partials of (p, A p) and of (r, r)
+    int npap, nrr;
+    double rtol, atol;
+    // set where A p comes without its interface sum: the mesh's groups, and each
+    // lateral node's group (-1: no other copies)
+    const int32_t *groups = nullptr, *group_of = nullptr;
+    __host__ __device__ static int slot(int it) { return it == 0 ? RING : (it - 1) % RING; }
+};
+int cg_update_blocks(const MeshLevel& m, int ncomp);  // = CgState::nrr
+void launch_cg_begin(const CgState& st, const double* rr0, hipStream_t s);
+// iteration it after ap = A p and its partials: x, r, then p and the stopping test
+template <typename T>
+void launch_cg_step(const MeshLevel& m, int ncomp, T* x, T* r, T* p, const T* ap, const CgState& st, int it,
+                    hipStream_t s);
+// reduce_blocks(m, ncomp) partials of the owned dot a . b, not yet added up
+template <typename T>
+void launch_dot_partials(const MeshLevel& m, int ncomp, const T* a, const T* b, double* part_dev, hipStream_t s);
 
 // out_dev[0] += sum over owned nodes of a . b; ncomp fields of N each
 template <typename T>

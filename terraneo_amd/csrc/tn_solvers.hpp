@@ -85,6 +85,12 @@ void v_multidot(Ctx& c, const BVec& a, const std::vector<const BVec*>& bs, doubl
 
 struct LinOp {
     virtual void apply(Ctx& c, const BVec& x, const BVec& y) = 0;
+    // y = A x and the partial sums of the owned dot x . y (one block; x equal on a
+    // node's copies): dot_blocks(x) doubles at part, to be added in order.  Where
+    // dot_partial() is true, y is left without its interface sum.
+    virtual void apply_dot(Ctx& c, const BVec& x, const BVec& y, double* part);
+    virtual int dot_blocks(const BVec& x) const;
+    virtual bool dot_partial() const { return false; }
     virtual ~LinOp() = default;
 };
 
@@ -163,6 +169,9 @@ class PCG : public Solver {
     IterInfo info;
 
   private:
+    // without preconditioner and on one block: scalars on the device, no host wait per iteration
+    void solve_queued(Ctx& c, LinOp& A, const BVec& x, const BVec& b);
+    DevBuf<double> scalars_;  // CgState's arrays
     KrylovParams p_;
     std::vector<BVec> t_;
     Solver* prec_;

@@ -51,7 +51,9 @@ struct MassArgs {
     const T* x;         // input field (lumped k-mass: the coefficient)
     T* y;               // output, every node copy written (before the interface sum)
     const double* geo;  // the mesh's wedge table [10][n-1][n-1][2][GEO_STRIDE]
+    double* dot = nullptr;  // optional: mass_blocks(n) partial sums of x . y over all node copies
 };
+int mass_blocks(int n);
 
 template <typename T>
 void launch_div(const DivArgs<T>& a, hipStream_t s);
