@@ -8,6 +8,7 @@
 #include <memory>
 #include <string>
 
+#include "tn_coarse_cg.hpp"
 #include "tn_internal.hpp"
 #include "tn_eps_march.hpp"
 #include "tn_mg.hpp"
@@ -192,6 +193,27 @@ int march_seg(int n, int dtype_size)
     return tn::march_seg_for(n, tn::march_block_rows(dtype_size), tn::march_waves_per_cu(dtype_size));
 }
 
+// arguments of a stored operator's kernels but for the vectors; the boundary
+// forms are brought up to date
+template <typename T, typename S>
+tn::StoredArgs<T, S> stored_args(tn_eps* op, const MeshLevel& m, const S* stored, bool penalty, hipStream_t s)
+{
+    const bool need_blk = op->bc_cmb != TN_NEUMANN || op->bc_surf != TN_NEUMANN;
+    const size_t blk_bytes = sizeof(T) * 2 * 10 * (size_t)m.n * m.n * 3;
+    if (need_blk && op->blk.n != blk_bytes) {
+        op->blk.alloc(blk_bytes);
+        op->blk_ready = false;
+    }
+    tn::StoredArgs<T, S> a{stored, nullptr, nullptr, m.d_coords.p, m.n, m.nr, op->bc_cmb, op->bc_surf, 0, nullptr,
+                           nullptr, need_blk ? (const T*)op->blk.p : nullptr, penalty ? op->pen.p : nullptr,
+                           m.d_radii.p, op->penalty_once ? m.d_coords_owned.p : m.d_coords.p};
+    if (need_blk && !op->blk_ready) {
+        tn::launch_stored_blk<T, S>(a, (T*)op->blk.p, s);
+        op->blk_ready = true;
+    }
+    return a;
+}
+
 template <typename T>
 void eps_apply_t(tn_eps* op, const void* src_v, void* dst_v, hipStream_t s)
 {
@@ -234,23 +256,14 @@ void eps_apply_t(tn_eps* op, const void* src_v, void* dst_v, hipStream_t s)
         if (op->cellsum.n != (size_t)ncs * sizeof(T)) op->cellsum.alloc((size_t)ncs * sizeof(T));
         T* csum = (T*)op->cellsum.p;
         T* ctop = csum + 12 * (10LL * (m.n - 1) * (m.n - 1) * (m.nr - 1));
-        const bool need_blk = op->bc_cmb != TN_NEUMANN || op->bc_surf != TN_NEUMANN;
-        const size_t blk_bytes = sizeof(T) * 2 * 10 * (size_t)m.n * m.n * 3;
-        if (need_blk && op->blk.n != blk_bytes) {
-            op->blk.alloc(blk_bytes);
-            op->blk_ready = false;
-        }
         auto run = [&](auto* stored) {
-            using S = std::remove_const_t<std::remove_pointer_t<decltype(stored)>>;
-            tn::StoredArgs<T, S> a{stored, src, dst, m.d_coords.p, m.n, m.nr, op->bc_cmb, op->bc_surf, add ? 1 : 0,
-                                   csum, ctop, need_blk ? (const T*)op->blk.p : nullptr,
-                                   penalty ? op->pen.p : nullptr, m.d_radii.p,
-                                   op->penalty_once ? m.d_coords_owned.p : m.d_coords.p};
-            if (need_blk && !op->blk_ready) {
-                tn::launch_stored_blk<T, S>(a, (T*)op->blk.p, s);
-                op->blk_ready = true;
-            }
-            tn::launch_stored_apply<T, S>(a, op->diagonal, s);
+            auto a = stored_args<T>(op, m, stored, penalty, s);
+            a.src = src;
+            a.dst = dst;
+            a.add = add ? 1 : 0;
+            a.csum = csum;
+            a.ctop = ctop;
+            tn::launch_stored_apply(a, op->diagonal, s);
         };
         if (op->stored_dtype == TN_F64)
             run((const double*)op->stored.p);
@@ -260,9 +273,42 @@ void eps_apply_t(tn_eps* op, const void* src_v, void* dst_v, hipStream_t s)
     if (op->comm_mode == TN_COMM_ADDITIVE) tn::launch_interface_sum<T>(m, 3, dst, s);
 }
 
+template <typename T>
+void coarse_cg_t(tn_eps* op, void* x, const void* b, bool zero, int max_iterations, double rtol, double atol,
+                 hipStream_t s)
+{
+    const MeshLevel& m = const_cast<tn_mesh*>(op->mesh)->lvl.dev();
+    const bool penalty = op->bc_cmb == TN_FREESLIP && op->bc_surf == TN_FREESLIP;
+    if (penalty && !op->penalty_ready) build_penalty(op);
+    auto run = [&](auto* stored) {
+        using S = std::remove_const_t<std::remove_pointer_t<decltype(stored)>>;
+        tn::CoarseCgArgs<T, S> g{stored_args<T>(op, m, stored, penalty, s), (T*)x, (const T*)b, m.d_owned_lat.p,
+                                 m.d_grp_pad.p, m.d_grp_of.p, zero ? 1 : 0, max_iterations, rtol, atol};
+        tn::launch_coarse_cg(g, s);
+    };
+    if (op->stored_dtype == TN_F64)
+        run((const double*)op->stored.p);
+    else
+        run((const float*)op->stored.p);
+}
+
 }  // namespace
 
 namespace tn {
+bool eps_coarse_cg(tn_eps* op, void* x, const void* b, bool zero, int max_iterations, double rtol, double atol,
+                   hipStream_t s)
+{
+    const MeshLevel& m = op->mesh->lvl;
+    if (op->stored_dtype < 0 || op->diagonal || op->apply_mode != TN_REPLACE || op->comm_mode != TN_COMM_ADDITIVE ||
+        x == b || !coarse_cg_fits(m.n, m.nr, op->dtype == TN_F64 ? 8 : 4))
+        return false;
+    if (op->dtype == TN_F64)
+        coarse_cg_t<double>(op, x, b, zero, max_iterations, rtol, atol, s);
+    else
+        coarse_cg_t<float>(op, x, b, zero, max_iterations, rtol, atol, s);
+    return true;
+}
+
 void eps_apply(tn_eps* op, const void* src, void* dst, hipStream_t s)
 {
     if (op->dtype == TN_F64)

@@ -106,6 +106,10 @@ struct EpsOp : LinOp {
     tn_eps* op;
     explicit EpsOp(tn_eps* o) : op(o) {}
     void apply(Ctx& c, const BVec& x, const BVec& y) override { eps_apply(op, x.b[0].p, y.b[0].p, c.s); }
+    bool small_cg(Ctx& c, const BVec& x, const BVec& b, bool zero, int its, double rtol, double atol) override
+    {
+        return x.b[0].dtype == op->dtype && eps_coarse_cg(op, x.b[0].p, b.b[0].p, zero, its, rtol, atol, c.s);
+    }
 };
 
 struct StokesOp : LinOp {
@@ -216,6 +220,7 @@ void gmg_setup(tn_gmg* g, const tn_gmg_options& o, hipStream_t s)
     kp.rtol = o.coarse_rtol;
     kp.atol = o.coarse_atol;
     g->coarse.reset(new PCG(kp, g->ctmp, nullptr));
+    g->coarse->quiet = true;
     Solver* coarse = g->coarse.get();
     if (o.coarse_solver == TN_COARSE_DENSE) {
         // gathers / scatters convert any precision: no bridge needed

@@ -536,8 +536,15 @@ void PCG::solve_queued(Ctx& c, LinOp& A, const BVec& x, const BVec& b)
     }
 }
 
+void PCG::solve_zero(Ctx& c, LinOp& A, const BVec& x, const BVec& b)
+{
+    if (quiet && !prec_ && x.nb == 1 && A.small_cg(c, x, b, true, p_.max_iterations, p_.rtol, p_.atol)) return;
+    Solver::solve_zero(c, A, x, b);
+}
+
 void PCG::solve(Ctx& c, LinOp& A, const BVec& x, const BVec& b)
 {
+    if (quiet && !prec_ && x.nb == 1 && A.small_cg(c, x, b, false, p_.max_iterations, p_.rtol, p_.atol)) return;
     if (!prec_ && x.nb == 1) {
         solve_queued(c, A, x, b);
         return;

@@ -51,4 +51,8 @@ template <typename T>
 void grad_t(tn_stokes* K, const void* p, void* u, bool add, bool comm, hipStream_t s);
 // C++ entry used by the Stokes and solver layers
 void eps_apply(tn_eps* op, const void* src, void* dst, hipStream_t s);
+// unpreconditioned CG on op in one launch where op is stored and small
+// (kernels_coarse_cg.hip); false: not such an operator, nothing done
+bool eps_coarse_cg(tn_eps* op, void* x, const void* b, bool zero, int max_iterations, double rtol, double atol,
+                   hipStream_t s);
 }

@@ -91,6 +91,12 @@ struct LinOp {
     virtual void apply_dot(Ctx& c, const BVec& x, const BVec& y, double* part);
     virtual int dot_blocks(const BVec& x) const;
     virtual bool dot_partial() const { return false; }
+    // unpreconditioned CG for A x = b in one launch, without a record of its
+    // residuals; false: not available for this operator
+    virtual bool small_cg(Ctx&, const BVec& x, const BVec& b, bool zero, int max_iterations, double rtol, double atol)
+    {
+        return false;
+    }
     virtual ~LinOp() = default;
 };
 
@@ -166,7 +172,9 @@ class PCG : public Solver {
   public:
     PCG(KrylovParams p, std::vector<BVec> tmps, Solver* prec);
     void solve(Ctx& c, LinOp& A, const BVec& x, const BVec& b) override;
+    void solve_zero(Ctx& c, LinOp& A, const BVec& x, const BVec& b) override;
     IterInfo info;
+    bool quiet = false;  // no one reads info: LinOp::small_cg may run instead
 
   private:
     // without preconditioner and on one block: scalars on the device, no host wait per iteration
