@@ -122,7 +122,8 @@ tn::Geom<float> geom_of<float>(const MeshLevel& m)
     return {m.d_coords_f.p, m.d_radii_f.p, m.d_geo_f.p, m.n, m.nr};
 }
 
-int device_cus()
+}  // namespace
+int tn::device_cus()
 {
     static int cache[64] = {0};
     int dev = 0;
@@ -135,6 +136,7 @@ int device_cus()
     }
     return cache[dev];
 }
+namespace {
 
 // Segment length (node columns per block) of a march kernel with `own` node
 // rows per block and `waves_per_cu` resident waves per CU: the kernel takes
@@ -149,7 +151,7 @@ int tn::march_seg_for(int n, int own, int waves_per_cu)
     }();
     if (env > 0) return std::min(std::min(env, n), tn::MARCH_SEG_MAX);
     const int64_t per_cu = std::max(1, waves_per_cu / (own + 1));
-    const int64_t nxb = (n + own - 1) / own, cus = device_cus() * per_cu;
+    const int64_t nxb = (n + own - 1) / own, cus = tn::device_cus() * per_cu;
     int best = std::min(n, tn::MARCH_SEG_MAX);
     int64_t best_cost = -1;
     for (int seg = std::min(n, tn::MARCH_SEG_MAX); seg >= std::min(n, 6); --seg) {
@@ -171,7 +173,7 @@ int tn::march_seg_for(int n, int own, int waves_per_cu)
 // longer than the kernel's carried level (MARCH_SEG_MAX columns).
 int tn::march_run_blocks(int cols, int resident)
 {
-    const int64_t cus = device_cus();
+    const int64_t cus = tn::device_cus();
     int64_t best = 1;
     double best_cost = -1.0;
     for (int per_cu = 1; per_cu <= resident; ++per_cu) {

@@ -30,7 +30,7 @@ using tn::MeshLevel;
 tn::FvArgs tn_fv::args() const
 {
     const MeshLevel& L = mesh->lvl;
-    return tn::FvArgs{L.d_coords.p, L.d_radii.p, centers.p, columns.p, n, nr};
+    return tn::FvArgs{L.d_coords.p, L.d_radii.p, centers.p, columns.p, layers.p, n, nr};
 }
 
 namespace {
@@ -132,7 +132,17 @@ int tn_fv_create(tn_mesh* m, tn_fv** out)
         TN_HIP(hipMemset(fv->Rp.p, 0, sizeof(double) * fv->size));
         TN_HIP(hipMemset(fv->Rm.p, 0, sizeof(double) * fv->size));
         TN_HIP(hipMemset(fv->ad.p, 0, sizeof(double) * fv->ad.n));
-        tn::launch_fv_columns(fv->args(), fv->columns.p, nullptr);
+        // layer part of the cell centres, int rho^3 / int rho^2 (without cancellation)
+        std::vector<double> layers(L.nr + 1, 0.0);
+        for (int rc = 1; rc < L.nr; ++rc) {
+            const double r1 = L.radii[rc - 1], r2 = L.radii[rc];
+            layers[rc] = 0.75 * (r1 + r2) * (r1 * r1 + r2 * r2) / (r1 * r1 + r1 * r2 + r2 * r2);
+        }
+        fv->layers.upload(layers);
+        tn::DevBuf<double> centroids(3 * (size_t)10 * (L.n + 1) * (L.n + 1));
+        tn::launch_fv_centroids(fv->args(), centroids.p, nullptr);
+        tn::launch_fv_ghost_columns(fv->pairs.p, fv->npairs, centroids.p, nullptr);
+        tn::launch_fv_columns(fv->args(), centroids.p, fv->columns.p, nullptr);
         tn::launch_fv_centers(fv->args(), fv->centers.p, nullptr);
         ghost_update(fv, fv->centers.p, 3, nullptr);
         TN_HIP(hipStreamSynchronize(nullptr));
@@ -203,7 +213,7 @@ int tn_fct_predictor(tn_fv* fv, double* T, const double* vel, double dt, double 
     TN_REQUIRE(fv && T && vel, "null pointer");
     ghost_update(fv, T, 1, (hipStream_t)s);
     tn::launch_fct_predictor(fv->args(), vel, T, dt, kappa, source, subtract_divergence, fv->TL.p, fv->ad.p,
-                             (hipStream_t)s);
+                             tn::FctFused{}, (hipStream_t)s);
     TN_API_END
 }
 
@@ -213,8 +223,7 @@ int tn_fct_limiter(tn_fv* fv, tn_stream_t s)
     TN_REQUIRE(fv, "null pointer");
     ghost_update(fv, fv->TL.p, 1, (hipStream_t)s);
     tn::launch_fct_limiter(fv->n, fv->nr, fv->TL.p, fv->ad.p, fv->Rp.p, fv->Rm.p, (hipStream_t)s);
-    ghost_update(fv, fv->Rp.p, 1, (hipStream_t)s);
-    ghost_update(fv, fv->Rm.p, 1, (hipStream_t)s);
+    tn::launch_fv_ghost2(fv->pairs.p, fv->npairs, fv->nr, fv->Rp.p, fv->Rm.p, (hipStream_t)s);
     TN_API_END
 }
 
@@ -245,13 +254,13 @@ int tn_fct_explicit_step(tn_fv* fv, double* T, const double* vel, double dt, dou
     TN_REQUIRE(fv && T && vel, "null pointer");
     const hipStream_t st = (hipStream_t)s;
     ghost_update(fv, T, 1, st);
-    tn::launch_fct_predictor(fv->args(), vel, T, dt, kappa, source, subtract_divergence, fv->TL.p, fv->ad.p, st);
-    if (apply_cmb || apply_surf)
-        tn::launch_fv_dirichlet(fv->n, fv->nr, fv->TL.p, apply_cmb, t_cmb, apply_surf, t_surf, st);
+    // the shells' values go into T_L with the predictor, its flux sums into R+ / R-
+    const tn::FctFused fused{apply_cmb, apply_surf, t_cmb, t_surf, fv->Rp.p, fv->Rm.p};
+    tn::launch_fct_predictor(fv->args(), vel, T, dt, kappa, source, subtract_divergence, fv->TL.p, fv->ad.p, fused,
+                             st);
     ghost_update(fv, fv->TL.p, 1, st);
-    tn::launch_fct_limiter(fv->n, fv->nr, fv->TL.p, fv->ad.p, fv->Rp.p, fv->Rm.p, st);
-    ghost_update(fv, fv->Rp.p, 1, st);
-    ghost_update(fv, fv->Rm.p, 1, st);
+    tn::launch_fct_limiter_sums(fv->n, fv->nr, fv->TL.p, fv->Rp.p, fv->Rm.p, st);
+    tn::launch_fv_ghost2(fv->pairs.p, fv->npairs, fv->nr, fv->Rp.p, fv->Rm.p, st);
     tn::launch_fct_correction(fv->n, fv->nr, fv->TL.p, fv->ad.p, fv->Rp.p, fv->Rm.p, T, st);
     TN_API_END
 }
@@ -263,7 +272,8 @@ int tn_fct_upwind_step(tn_fv* fv, double* T, const double* vel, double dt, doubl
     TN_REQUIRE(fv && T && vel, "null pointer");
     const hipStream_t st = (hipStream_t)s;
     ghost_update(fv, T, 1, st);
-    tn::launch_fct_predictor(fv->args(), vel, T, dt, kappa, source, subtract_divergence, fv->TL.p, fv->ad.p, st);
+    tn::launch_fct_predictor(fv->args(), vel, T, dt, kappa, source, subtract_divergence, fv->TL.p, fv->ad.p,
+                             tn::FctFused{}, st);
     TN_HIP(hipMemcpyAsync(T, fv->TL.p, sizeof(double) * fv->size, hipMemcpyDeviceToDevice, st));
     TN_API_END
 }

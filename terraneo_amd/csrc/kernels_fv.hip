@@ -18,7 +18,9 @@
 
 #include <algorithm>
 
+#include "tn_eps_march.hpp"
 #include "tn_fv.hpp"
+#include "tn_march.hpp"
 
 namespace tn {
 
@@ -119,18 +121,14 @@ __device__ __forceinline__ void cross3(const double a[3], const double b[3], dou
 }
 
 // Lateral part of the geometry of hex column (d, x, y), the same at every
-// radius: g[0..12) the lateral face normals Vb x Va of faces 0..3, g[12..15)
-// and g[15..18) the two triangles' (V1 - V0) x (V2 - V0), g[18] the sum of the
-// wedges' |det(V0, V1, V2)|.  Corners c00 = (x, y), c10 = (x+1, y),
-// c01 = (x, y+1), c11 = (x+1, y+1); wedge 0: V0 = c00, V1 = c10, V2 = c01;
-// wedge 1: W0 = c11, W1 = c01, W2 = c10.  Lateral faces (face, Va, Vb):
-// 0 (c00, c01) xi = 0 of wedge 0: n ~ V2 x V0 = c01 x c00; 2 (c00, c10)
-// eta = 0 of wedge 0: V1 x V0 = c10 x c00; 1 (c11, c10): W2 x W0 = c10 x c11;
-// 3 (c11, c01): W1 x W0 = c01 x c11.
-__device__ __forceinline__ void column_geometry(const double* __restrict__ coords, int n, int d, int x, int y,
-                                                double g[FV_COLUMN])
+// radius.  Corners c00 = (x, y), c10 = (x+1, y), c01 = (x, y+1), c11 = (x+1, y+1);
+// wedge 0: V0 = c00, V1 = c10, V2 = c01; wedge 1: W0 = c11, W1 = c01, W2 = c10.
+// Lateral faces (face, Va, Vb), normal Vb x Va: 0 (c00, c01) xi = 0 of wedge 0:
+// n ~ V2 x V0 = c01 x c00; 2 (c00, c10) eta = 0 of wedge 0: V1 x V0 = c10 x c00;
+// 1 (c11, c10): W2 x W0 = c10 x c11; 3 (c11, c01): W1 x W0 = c01 x c11.
+__device__ __forceinline__ void column_corners(const double* __restrict__ coords, int n, int d, int x, int y,
+                                               double c[4][3])
 {
-    double c[4][3];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
         const double* p = coords + 3 * (((int64_t)d * n + x + (k & 1)) * n + y + (k >> 1));
@@ -138,10 +136,229 @@ __device__ __forceinline__ void column_geometry(const double* __restrict__ coord
         c[k][1] = p[1];
         c[k][2] = p[2];
     }
-    const int FA[4] = {0, 3, 0, 3}, FB[4] = {2, 1, 1, 2};  // corner indices of faces 0, 1, 2, 3
+}
+// |det(V0, V1, V2)| of the two wedges (= V0 . (V1 x V2))
+__device__ __forceinline__ void column_dets(const double c[4][3], double det[2])
+{
+    double v12[3], w12[3];
+    cross3(c[1], c[2], v12);
+    cross3(c[2], c[1], w12);
+    det[0] = fabs(c[0][0] * v12[0] + c[0][1] * v12[1] + c[0][2] * v12[2]);
+    det[1] = fabs(c[3][0] * w12[0] + c[3][1] * w12[1] + c[3][2] * w12[2]);
+}
+
+__device__ __forceinline__ double dot3d(const double a[3], const double b[3])
+{
+    return a[0] * b[0] + a[1] * b[1] + a[2] * b[2];
+}
+
+// The layer's part of a cell's geometry, held in a lane's registers: the flux
+// factors and, times kappa, the diffusion factors of the faces.
+struct Layer {
+    double r1, r2, hh;     // radii, (r2 - r1) / 4 (half of h, the mean of the two node levels' weights)
+    double ab, at;         // weights of the bottom / top velocities in a lateral face
+    double q1, q2;         // r^2 / 6 of the radial faces, signed with the layers' order
+    double kl, k4, k5;     // diffusion factors: lateral, radial bottom, radial top
+    double vol;            // (r2^3 - r1^3) / 6
+    __device__ void set(const FvArgs& a, int rc, double kappa)
+    {
+        r1 = a.radii[rc - 1];
+        r2 = a.radii[rc];
+        const double s0 = a.layers[rc - 1], s1 = a.layers[rc], s2 = a.layers[rc + 1];
+        const double h = 0.5 * (r2 - r1);
+        hh = 0.5 * h;
+        ab = (2.0 * r1 + r2) / 3.0;
+        at = (r1 + 2.0 * r2) / 3.0;
+        q1 = (s0 < s1 ? -1.0 : 1.0) * (r1 * r1 / 6.0);
+        q2 = (s2 < s1 ? -1.0 : 1.0) * (r2 * r2 / 6.0);
+        kl = kappa * (h * (r1 + r2) / s1);
+        k4 = kappa * (0.5 * r1 * r1 / fabs(s0 - s1));
+        k5 = kappa * (0.5 * r2 * r2 / fabs(s2 - s1));
+        vol = (r2 - r1) * (r1 * r1 + r1 * r2 + r2 * r2) / 6.0;  // without cancellation
+    }
+};
+
+// A corner column's velocity on one layer: bottom and top node, and their
+// combination in the lateral faces
+struct CornerVel {
+    double b[3], t[3], l[3];
+    __device__ __forceinline__ void load(const double* __restrict__ vel, int64_t N, int64_t node)
+    {
 #pragma unroll
-    for (int f = 0; f < 4; ++f) cross3(c[FB[f]], c[FA[f]], g + 3 * f);
-    double e1[3], e2[3];
+        for (int j = 0; j < 3; ++j) {
+            b[j] = vel[j * N + node];
+            t[j] = vel[j * N + node + 1];
+        }
+    }
+    __device__ __forceinline__ void combine(const Layer& L)
+    {
+#pragma unroll
+        for (int j = 0; j < 3; ++j) l[j] = L.ab * b[j] + L.at * t[j];
+    }
+};
+
+// Face fluxes beta (towards the neighbours), diffusion coefficients and volume of
+// a cell from its column's table g, its layer and the corners c00, c10, c01, c11.
+__device__ __forceinline__ void cell_faces(const double* __restrict__ g, const Layer& L, const CornerVel& c00,
+                                           const CornerVel& c10, const CornerVel& c01, const CornerVel& c11,
+                                           double beta[6], double dc[6], double& M)
+{
+    double f0 = 0, f1 = 0, f2 = 0, f3 = 0, bb = 0, bt = 0;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        f0 += g[j] * (c00.l[j] + c01.l[j]);
+        f1 += g[3 + j] * (c11.l[j] + c10.l[j]);
+        f2 += g[6 + j] * (c00.l[j] + c10.l[j]);
+        f3 += g[9 + j] * (c11.l[j] + c01.l[j]);
+        bb += g[12 + j] * (c00.b[j] + c10.b[j] + c01.b[j]) + g[15 + j] * (c11.b[j] + c01.b[j] + c10.b[j]);
+        bt += g[12 + j] * (c00.t[j] + c10.t[j] + c01.t[j]) + g[15 + j] * (c11.t[j] + c01.t[j] + c10.t[j]);
+    }
+    beta[0] = L.hh * f0;
+    beta[1] = L.hh * f1;
+    beta[2] = L.hh * f2;
+    beta[3] = L.hh * f3;
+    beta[4] = g[19] * (L.q1 * bb);
+    beta[5] = g[19] * (L.q2 * bt);
+#pragma unroll
+    for (int f = 0; f < 4; ++f) dc[f] = L.kl * g[20 + f];
+    dc[4] = L.k4 * g[24];
+    dc[5] = L.k5 * g[24];
+    M = g[18] * L.vol;
+}
+
+// The hex columns of a block: FV_STRIPS waves on neighbouring strips x of one
+// diamond and one chunk of 64 layers, marching together along y, so that a column
+// of nodes or cells that two strips share is read into the caches at one time
+// (with strips far apart the stable step took 258 us and the predictor 710 us at
+// level 7 x 129, with the loads of a column issued in its own step 231 and 756 us,
+// a step ahead of the stores 233 and 650 us).  The columns of all strip groups
+// are split evenly over the blocks.  The corner velocities shared by consecutive
+// columns stay in registers.  f.load(pre, d, x, y, rc) a step ahead,
+// then f(valid, rc, pre, beta, dc, M).
+constexpr int FV_STRIPS = 8;
+__host__ __device__ inline int walk_groups(int n, int nr)
+{
+    return 10 * ((n - 1 + FV_STRIPS - 1) / FV_STRIPS) * ((nr - 1 + 63) / 64);
+}
+template <class F>
+__device__ __forceinline__ void walk_columns(const FvArgs& a, const double* __restrict__ columns,
+                                             const double* __restrict__ vel, double kappa, F& f)
+{
+    const int n = a.n, nr = a.nr, nq = n - 1, ncr = nr - 1;
+    const int64_t N = 10LL * n * n * nr;
+    const int nxg = (nq + FV_STRIPS - 1) / FV_STRIPS, total = walk_groups(n, nr) * nq;
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int tile = xcd_tile(blockIdx.x, gridDim.x);
+    int pos = march::run_begin(total, tile, gridDim.x);
+    const int end = march::run_begin(total, tile + 1, gridDim.x);
+    while (pos < end) {
+        const int group = pos / nq, y0 = pos - group * nq, y1 = min(nq, y0 + end - pos);
+        pos += y1 - y0;
+        const int x = (group % nxg) * FV_STRIPS + w, d = (group / nxg) % 10, chunk = group / (nxg * 10);
+        if (x >= nq) continue;  // (no barrier in the walk)
+        const int rc = 1 + 64 * chunk + (threadIdx.x & 63);
+        const bool valid = rc <= ncr;
+        const int rcc = valid ? rc : ncr;
+        Layer L;
+        L.set(a, rcc, kappa);
+        // corners (x, .), (x + 1, .) at y, y + 1 and, loaded a step ahead, y + 2 (roles
+        // rotate by copies): a step's loads are in flight before the last one's stores
+        CornerVel A0, A1, B0, B1, C0, C1;
+        typename F::Pre cur, nxt;
+        const int64_t row = (int64_t)n * nr;
+        int64_t node = (((int64_t)d * n + x) * n + y0) * nr + rcc - 1;
+        A0.load(vel, N, node);
+        A1.load(vel, N, node + row);
+        node += nr;
+        B0.load(vel, N, node);
+        B1.load(vel, N, node + row);
+        f.load(cur, d, x, y0, rcc);
+        A0.combine(L);
+        A1.combine(L);
+        const double* __restrict__ g = columns + (int64_t)FV_COLUMN * __builtin_amdgcn_readfirstlane((d * nq + x) * nq + y0);
+        for (int y = y0; y < y1; ++y, g += FV_COLUMN) {
+            if (y + 1 < y1) {
+                node += nr;
+                C0.load(vel, N, node);
+                C1.load(vel, N, node + row);
+                f.load(nxt, d, x, y + 1, rcc);
+            }
+            B0.combine(L);
+            B1.combine(L);
+            double beta[6], dc[6], M;
+            cell_faces(g, L, A0, A1, B0, B1, beta, dc, M);
+            f(valid, rcc, cur, beta, dc, M);
+            A0 = B0;
+            A1 = B1;
+            B0 = C0;
+            B1 = C1;
+            cur = nxt;
+        }
+    }
+}
+
+__device__ __forceinline__ int64_t neighbour(int n, int nr, int d, int xc, int yc, int rc, int f)
+{
+    const int ox = f == 0 ? -1 : (f == 1 ? 1 : 0), oy = f == 2 ? -1 : (f == 3 ? 1 : 0),
+              orr = f == 4 ? -1 : (f == 5 ? 1 : 0);
+    return fvi(n, nr, d, xc + ox, yc + oy, rc + orr);
+}
+
+// ---------------------------------------------------------------- kernels
+
+// Column part c of the cell centres: int_K x / |K| = s c with
+// c = sum_w |det_w| (V0 + V1 + V2)_w / 3 / sum_w |det_w| and the layer part
+// s = int rho^3 / int rho^2 (the Felippa rule integrates both exactly)
+__global__ __launch_bounds__(FV_BLOCK) void k_fv_centroids(FvArgs a, double* __restrict__ centroids)
+{
+    const int n = a.n;
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= 10LL * (n - 1) * (n - 1)) return;
+    const int y = (int)(t % (n - 1)), x = (int)((t / (n - 1)) % (n - 1)), d = (int)(t / ((int64_t)(n - 1) * (n - 1)));
+    double c[4][3], det[2];
+    column_corners(a.coords, n, d, x, y, c);
+    column_dets(c, det);
+    double* o = centroids + 3 * (((int64_t)d * (n + 1) + x + 1) * (n + 1) + y + 1);
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+        o[j] = (det[0] * (c[0][j] + c[1][j] + c[2][j]) + det[1] * (c[3][j] + c[2][j] + c[1][j])) /
+               (3.0 * (det[0] + det[1]));
+}
+
+// lateral ghost columns of the centroids
+__global__ __launch_bounds__(FV_BLOCK) void k_fv_ghost_columns(const int32_t* __restrict__ pairs, int cnt,
+                                                               double* __restrict__ centroids)
+{
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= cnt) return;
+    for (int j = 0; j < 3; ++j) centroids[3LL * pairs[2 * t] + j] = centroids[3LL * pairs[2 * t + 1] + j];
+}
+
+// the table of every hex column (FV_COLUMN), one thread per column
+__global__ __launch_bounds__(FV_BLOCK) void k_fv_columns(FvArgs a, const double* __restrict__ centroids,
+                                                         double* __restrict__ columns)
+{
+    const int n = a.n;
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= 10LL * (n - 1) * (n - 1)) return;
+    const int y = (int)(t % (n - 1)), x = (int)((t / (n - 1)) % (n - 1)), d = (int)(t / ((int64_t)(n - 1) * (n - 1)));
+    double c[4][3], det[2], g[FV_COLUMN];
+    column_corners(a.coords, n, d, x, y, c);
+    column_dets(c, det);
+    const int64_t fl = ((int64_t)d * (n + 1) + x + 1) * (n + 1) + y + 1;
+    const double* ci = centroids + 3 * fl;
+    const int FA[4] = {0, 3, 0, 3}, FB[4] = {2, 1, 1, 2};  // corner indices of faces 0, 1, 2, 3
+    const int64_t nb[4] = {fl - (n + 1), fl + (n + 1), fl - 1, fl + 1};
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+        double N[3], dx[3];
+        cross3(c[FB[f]], c[FA[f]], N);
+        for (int j = 0; j < 3; ++j) dx[j] = centroids[3 * nb[f] + j] - ci[j];
+        const double s = dot3d(N, dx);
+        for (int j = 0; j < 3; ++j) g[3 * f + j] = s < 0 ? -N[j] : N[j];
+        g[20 + f] = dot3d(N, N) / fabs(s);
+    }
+    double e1[3], e2[3], nn[3];
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
         e1[j] = c[1][j] - c[0][j];
@@ -154,114 +371,12 @@ __device__ __forceinline__ void column_geometry(const double* __restrict__ coord
         e2[j] = c[1][j] - c[3][j];
     }
     cross3(e1, e2, g + 15);
-    // |det(V0, V1, V2)| per wedge (= V0 . (V1 x V2))
-    double v12[3], w12[3];
-    cross3(c[1], c[2], v12);
-    cross3(c[2], c[1], w12);
-    const double det0 = fabs(c[0][0] * v12[0] + c[0][1] * v12[1] + c[0][2] * v12[2]);
-    const double det1 = fabs(c[3][0] * w12[0] + c[3][1] * w12[1] + c[3][2] * w12[2]);
-    g[18] = det0 + det1;
-    g[19] = 0.0;
-}
-
-// Geometry of real FV cell (d, xc, yc, rc) from its column's lateral part
-// (a.columns, see column_geometry) and the radii.
-__device__ void cell_geometry(const FvArgs& a, const double* __restrict__ vel, int64_t N, int d, int xc, int yc,
-                              int rc, double beta[6], double& M, double S[6][3])
-{
-    const int n = a.n, nr = a.nr;
-    const int x = xc - 1, y = yc - 1, r = rc - 1;
-    double g[FV_COLUMN];
-    {
-        const double2* gp =
-            reinterpret_cast<const double2*>(a.columns + FV_COLUMN * (((int64_t)d * (n - 1) + x) * (n - 1) + y));
-#pragma unroll
-        for (int k = 0; k < FV_COLUMN / 2; ++k) {
-            const double2 v = gp[k];
-            g[2 * k] = v.x;
-            g[2 * k + 1] = v.y;
-        }
-    }
-    // nodal velocity at the 4 corners x {bottom, top}
-    double ub[4][3], ut[4][3];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const int64_t node = (((int64_t)d * n + x + (k & 1)) * n + y + (k >> 1)) * nr + r;
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            ub[k][j] = vel[j * N + node];
-            ut[k][j] = vel[j * N + node + 1];
-        }
-    }
-    const double r1 = a.radii[r], r2 = a.radii[r + 1];
-    const double h = 0.5 * (r2 - r1);
-    const double ab = (2.0 * r1 + r2) / 3.0, at = (r1 + 2.0 * r2) / 3.0;
-    const int FA[4] = {0, 3, 0, 3}, FB[4] = {2, 1, 1, 2};  // corner indices of faces 0, 1, 2, 3
-#pragma unroll
-    for (int f = 0; f < 4; ++f) {
-        const double* nv = g + 3 * f;
-        const double sS = h * (r1 + r2);
-        double w = 0;
-#pragma unroll
-        for (int j = 0; j < 3; ++j)
-            w += nv[j] * (ab * (ub[FA[f]][j] + ub[FB[f]][j]) + at * (ut[FA[f]][j] + ut[FB[f]][j]));
-        beta[f] = 0.5 * h * w;
-        S[f][0] = sS * nv[0];
-        S[f][1] = sS * nv[1];
-        S[f][2] = sS * nv[2];
-    }
-    // radial faces: both wedges' (V1 - V0) x (V2 - V0)
-    const double* n0 = g + 12;
-    const double* n1 = g + 15;
-    double bb = 0, bt = 0;
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-        bb += n0[j] * (ub[0][j] + ub[1][j] + ub[2][j]) + n1[j] * (ub[3][j] + ub[2][j] + ub[1][j]);
-        bt += n0[j] * (ut[0][j] + ut[1][j] + ut[2][j]) + n1[j] * (ut[3][j] + ut[2][j] + ut[1][j]);
-    }
-    beta[4] = r1 * r1 * bb / 6.0;
-    beta[5] = r2 * r2 * bt / 6.0;
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-        S[4][j] = 0.5 * r1 * r1 * (n0[j] + n1[j]);
-        S[5][j] = 0.5 * r2 * r2 * (n0[j] + n1[j]);
-    }
-    // orientation: towards the neighbour's centre (ghost centres included)
-    const double* cc = a.centers + 3 * fvi(n, nr, d, xc, yc, rc);
-#pragma unroll
-    for (int f = 0; f < 6; ++f) {
-        const int ox = f == 0 ? -1 : (f == 1 ? 1 : 0), oy = f == 2 ? -1 : (f == 3 ? 1 : 0),
-                  orr = f == 4 ? -1 : (f == 5 ? 1 : 0);
-        const double* nc = a.centers + 3 * fvi(n, nr, d, xc + ox, yc + oy, rc + orr);
-        const double s = S[f][0] * (nc[0] - cc[0]) + S[f][1] * (nc[1] - cc[1]) + S[f][2] * (nc[2] - cc[2]);
-        if (s < 0) {
-            S[f][0] = -S[f][0];
-            S[f][1] = -S[f][1];
-            S[f][2] = -S[f][2];
-            beta[f] = -beta[f];
-        }
-    }
-    M = g[18] * (r2 - r1) * (r1 * r1 + r1 * r2 + r2 * r2) / 6.0;  // (r2^3 - r1^3) / 6 without cancellation
-}
-
-__device__ __forceinline__ int64_t neighbour(int n, int nr, int d, int xc, int yc, int rc, int f)
-{
-    const int ox = f == 0 ? -1 : (f == 1 ? 1 : 0), oy = f == 2 ? -1 : (f == 3 ? 1 : 0),
-              orr = f == 4 ? -1 : (f == 5 ? 1 : 0);
-    return fvi(n, nr, d, xc + ox, yc + oy, rc + orr);
-}
-
-// ---------------------------------------------------------------- kernels
-
-// lateral geometry of every hex column (column_geometry), one thread per column
-__global__ __launch_bounds__(FV_BLOCK) void k_fv_columns(FvArgs a, double* __restrict__ columns)
-{
-    const int n = a.n;
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= 10LL * (n - 1) * (n - 1)) return;
-    const int y = (int)(t % (n - 1)), x = (int)((t / (n - 1)) % (n - 1)), d = (int)(t / ((int64_t)(n - 1) * (n - 1)));
-    double g[FV_COLUMN];
-    column_geometry(a.coords, n, d, x, y, g);
+    for (int j = 0; j < 3; ++j) nn[j] = g[12 + j] + g[15 + j];
+    const double ar = dot3d(nn, ci);
+    g[18] = det[0] + det[1];
+    g[19] = ar < 0 ? -1.0 : 1.0;
+    g[24] = dot3d(nn, nn) / fabs(ar);
+    g[25] = 0.0;
     double2* o = reinterpret_cast<double2*>(columns + FV_COLUMN * t);
 #pragma unroll
     for (int k = 0; k < FV_COLUMN / 2; ++k) o[k] = make_double2(g[2 * k], g[2 * k + 1]);
@@ -312,42 +427,57 @@ __global__ __launch_bounds__(FV_BLOCK) void k_fv_ghost(const int32_t* __restrict
     for (int c = 0; c < ncomp; ++c) f[dst + c] = f[src + c];
 }
 
+// the same for two scalars at once
+__global__ __launch_bounds__(FV_BLOCK) void k_fv_ghost2(const int32_t* __restrict__ pairs, int cnt, int nr,
+                                                        double* __restrict__ f, double* __restrict__ g)
+{
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= (int64_t)cnt * (nr - 1)) return;
+    const int rc = 1 + (int)(t % (nr - 1));
+    const int k = (int)(t / (nr - 1));
+    const int64_t dst = (int64_t)pairs[2 * k] * (nr + 1) + rc, src = (int64_t)pairs[2 * k + 1] * (nr + 1) + rc;
+    const double a = f[src], b = g[src];
+    f[dst] = a;
+    g[dst] = b;
+}
+
 // local stable time step M / lambda per cell, minimum per block
 // (fct_advection_diffusion.hpp:110-164)
-__global__ __launch_bounds__(FV_BLOCK) void k_fv_dt(FvArgs a, const double* __restrict__ vel, double kappa,
-                                                    double* __restrict__ part)
-{
-    const int n = a.n, nr = a.nr;
-    const int64_t cells = 10LL * (n - 1) * (n - 1) * (nr - 1);
-    const int64_t N = 10LL * n * n * nr;
-    double dtc = 1e300;
-    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < cells;
-         t += (int64_t)gridDim.x * blockDim.x) {
-        int d, xc, yc, rc;
-        cell_real(t, n, nr, d, xc, yc, rc);
-        double beta[6], M, S[6][3];
-        cell_geometry(a, vel, N, d, xc, yc, rc, beta, M, S);
-        const double* ci = a.centers + 3 * fvi(n, nr, d, xc, yc, rc);
+// (geometry as the predictor's: 831 us at lateral level 7 x 129 when every cell
+// read its seven centres, 227 us so)
+struct StableStep {
+    double dt = 1e300;
+    bool diffusion;
+    struct Pre {};
+    __device__ __forceinline__ void load(Pre&, int, int, int, int) {}
+    __device__ __forceinline__ void operator()(bool valid, int, const Pre&, const double beta[6], const double dc[6],
+                                               double M)
+    {
         double lambda = 0;
 #pragma unroll
         for (int f = 0; f < 6; ++f) {
             if (beta[f] < 0) lambda -= beta[f];
-            if (kappa > 0) {
-                const double* cj = a.centers + 3 * neighbour(n, nr, d, xc, yc, rc, f);
-                const double den = S[f][0] * (cj[0] - ci[0]) + S[f][1] * (cj[1] - ci[1]) + S[f][2] * (cj[2] - ci[2]);
-                if (den > 0) lambda += kappa * (S[f][0] * S[f][0] + S[f][1] * S[f][1] + S[f][2] * S[f][2]) / den;
-            }
+            if (diffusion) lambda += dc[f];
         }
-        dtc = fmin(dtc, lambda > 0 ? M / lambda : 1e30);
+        if (valid) dt = fmin(dt, lambda > 0 ? M / lambda : 1e30);
     }
+};
+
+__global__ __launch_bounds__(64 * FV_STRIPS) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_fv_dt(FvArgs a, const double* __restrict__ columns, const double* __restrict__ vel, double kappa,
+                                                    double* __restrict__ part)
+{
+    StableStep st;
+    st.diffusion = kappa > 0;
+    walk_columns(a, columns, vel, kappa, st);
+    double dtc = st.dt;
     // block minimum (order-independent)
-    __shared__ double red[FV_BLOCK / 64];
+    __shared__ double red[FV_STRIPS];
     for (int o = 32; o > 0; o >>= 1) dtc = fmin(dtc, __shfl_xor(dtc, o));
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = dtc;
     __syncthreads();
     if (threadIdx.x == 0) {
         double m = red[0];
-        for (int k = 1; k < FV_BLOCK / 64; ++k) m = fmin(m, red[k]);
+        for (int k = 1; k < FV_STRIPS; ++k) m = fmin(m, red[k]);
         part[blockIdx.x] = m;
     }
 }
@@ -366,47 +496,87 @@ __global__ __launch_bounds__(256) void k_min_finalize(const double* __restrict__
 
 // predictor (fct_advection_diffusion.hpp:261-402): low-order upwind +
 // two-point diffusion T_L, and the pre-scaled antidiffusive fluxes
-// (dt / M) (|beta| / 2) (T_i - T_j), stored face-major [6][fv cells]
-__global__ __launch_bounds__(FV_BLOCK) void k_fct_predictor(FvArgs a, const double* __restrict__ vel,
+// (dt / M) (|beta| / 2) (T_i - T_j), stored face-major [6][fv cells].
+// What binds is memory: velocity and T in, T_L and six fluxes out (88 B a cell,
+// 104 with the flux sums).  A thread per cell that read the centres of its cell
+// and six neighbours and both levels of four corners took 951 us at lateral level
+// 7 x 129; the column / layer split of the geometry needs no centres, and a run of
+// columns loads two corners a step: 650 us, 4.3 TB/s counting the re-reads.
+struct Predict {
+    const double* __restrict__ T;
+    const double* __restrict__ source;
+    double* __restrict__ TL;
+    double* __restrict__ ad;
+    double dt;
+    int subtract_div, n, nr;
+    int64_t fvsize;
+    FctFused fu;
+    struct Pre {
+        int64_t i;
+        double Ti, Tj[6], src;
+    };
+    __device__ __forceinline__ void load(Pre& q, int d, int x, int y, int rcc)
+    {
+        q.i = fvi(n, nr, d, x + 1, y + 1, rcc);
+        q.Ti = T[q.i];
+#pragma unroll
+        for (int f = 0; f < 6; ++f) q.Tj[f] = T[neighbour(n, nr, d, x + 1, y + 1, rcc, f)];
+        q.src = source ? source[q.i] : 0.0;
+    }
+    __device__ __forceinline__ void operator()(bool valid, int rcc, const Pre& q, const double beta[6],
+                                               const double dc[6], double M)
+    {
+        const int64_t i = q.i;
+        const double Ti = q.Ti;
+        const double(&Tj)[6] = q.Tj;
+        const double sc = dt / M;
+        double lo_diag = 0, lo_update = 0, bsum = 0, pp = 0, pm = 0;
+        double fl[6];
+#pragma unroll
+        for (int f = 0; f < 6; ++f) {
+            if (beta[f] >= 0)
+                lo_diag += beta[f];
+            else
+                lo_update += beta[f] * Tj[f];
+            bsum += beta[f];
+            lo_diag += dc[f];
+            lo_update -= dc[f] * Tj[f];
+            fl[f] = sc * (fabs(beta[f]) / 2.0) * (Ti - Tj[f]);
+            if (fl[f] > 0)
+                pp += fl[f];
+            else
+                pm += fl[f];
+        }
+        if (subtract_div) lo_diag -= bsum;
+        double v = Ti - sc * (lo_diag * Ti + lo_update);
+        if (source) v += dt * q.src;
+        if (!valid) return;
+#pragma unroll
+        for (int f = 0; f < 6; ++f) ad[f * fvsize + i] = fl[f];
+        if (fu.pp) {
+            fu.pp[i] = pp;
+            fu.pm[i] = pm;
+        }
+        if (rcc == 1 && fu.apply_cmb) {
+            v = fu.t_cmb;
+            TL[i - 1] = v;
+        }
+        if (rcc == nr - 1 && fu.apply_surf) {
+            v = fu.t_surf;
+            TL[i + 1] = v;
+        }
+        TL[i] = v;
+    }
+};
+
+__global__ __launch_bounds__(64 * FV_STRIPS) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_fct_predictor(FvArgs a, const double* __restrict__ columns, const double* __restrict__ vel,
                                                             const double* __restrict__ T, double dt, double kappa,
                                                             const double* __restrict__ source, int subtract_div,
                                                             double* __restrict__ TL, double* __restrict__ ad,
-                                                            int64_t fvsize)
+                                                            int64_t fvsize, FctFused fu)
 {
-    const int n = a.n, nr = a.nr;
-    const int64_t cells = 10LL * (n - 1) * (n - 1) * (nr - 1);
-    const int64_t N = 10LL * n * n * nr;
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= cells) return;
-    int d, xc, yc, rc;
-    cell_real(t, n, nr, d, xc, yc, rc);
-    double beta[6], M, S[6][3];
-    cell_geometry(a, vel, N, d, xc, yc, rc, beta, M, S);
-    const int64_t i = fvi(n, nr, d, xc, yc, rc);
-    const double Ti = T[i];
-    const double* ci = a.centers + 3 * i;
-    const double sc = dt / M;
-    double lo_diag = 0, lo_update = 0, bsum = 0;
-#pragma unroll
-    for (int f = 0; f < 6; ++f) {
-        const int64_t j = neighbour(n, nr, d, xc, yc, rc, f);
-        const double Tj = T[j];
-        if (beta[f] >= 0)
-            lo_diag += beta[f];
-        else
-            lo_update += beta[f] * Tj;
-        bsum += beta[f];
-        const double* cj = a.centers + 3 * j;
-        const double den = S[f][0] * (cj[0] - ci[0]) + S[f][1] * (cj[1] - ci[1]) + S[f][2] * (cj[2] - ci[2]);
-        const double dc = kappa * ((S[f][0] * S[f][0] + S[f][1] * S[f][1] + S[f][2] * S[f][2]) / den);
-        lo_diag += dc;
-        lo_update -= dc * Tj;
-        ad[f * fvsize + i] = sc * (fabs(beta[f]) / 2.0) * (Ti - Tj);
-    }
-    if (subtract_div) lo_diag -= bsum;
-    double v = Ti - sc * (lo_diag * Ti + lo_update);
-    if (source) v += dt * source[i];
-    TL[i] = v;
+    Predict p{T, source, TL, ad, dt, subtract_div, a.n, a.nr, fvsize, fu};
+    walk_columns(a, columns, vel, kappa, p);
 }
 
 // Dirichlet values on the shells: the real boundary cell and the ghost beyond (helpers.hpp:64-96)
@@ -448,6 +618,30 @@ __global__ __launch_bounds__(FV_BLOCK) void k_fct_limiter(int n, int nr, const d
             pp += fij;
         else
             pm += fij;
+        const double tj = TL[neighbour(n, nr, d, xc, yc, rc, f)];
+        tmax = fmax(tmax, tj);
+        tmin = fmin(tmin, tj);
+    }
+    Rp[i] = pp > 0 ? fmin(1.0, (tmax - ti) / pp) : 1.0;
+    Rm[i] = pm < 0 ? fmin(1.0, (tmin - ti) / pm) : 1.0;
+}
+
+// limiter from the predictor's flux sums in Rp / Rm (each thread replaces its own):
+// 40 instead of 72 B a cell
+__global__ __launch_bounds__(FV_BLOCK) void k_fct_limiter_sums(int n, int nr, const double* __restrict__ TL,
+                                                               double* __restrict__ Rp, double* __restrict__ Rm)
+{
+    const int64_t cells = 10LL * (n - 1) * (n - 1) * (nr - 1);
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= cells) return;
+    int d, xc, yc, rc;
+    cell_real(t, n, nr, d, xc, yc, rc);
+    const int64_t i = fvi(n, nr, d, xc, yc, rc);
+    const double pp = Rp[i], pm = Rm[i];
+    const double ti = TL[i];
+    double tmax = ti, tmin = ti;
+#pragma unroll
+    for (int f = 0; f < 6; ++f) {
         const double tj = TL[neighbour(n, nr, d, xc, yc, rc, f)];
         tmax = fmax(tmax, tj);
         tmin = fmin(tmin, tj);
@@ -581,19 +775,35 @@ int blocks_for(int64_t work) { return (int)((work + FV_BLOCK - 1) / FV_BLOCK); }
 
 int64_t fv_real_cells(int n, int nr) { return 10LL * (n - 1) * (n - 1) * (nr - 1); }
 int64_t fv_size(int n, int nr) { return 10LL * (n + 1) * (n + 1) * (nr + 1); }
-// grid-stride launch of the stable-step kernel: at most FV_DT_BLOCKS partial minima
-constexpr int FV_DT_BLOCKS = 2048;
-int fv_dt_blocks(int n, int nr) { return (int)std::min<int64_t>(blocks_for(fv_real_cells(n, nr)), FV_DT_BLOCKS); }
+// Blocks of the column walk: `per_cu` on every CU (what its registers allow), one
+// column each on small meshes
+static int walk_blocks(int n, int nr, int per_cu)
+{
+    return std::max(1, std::min(walk_groups(n, nr) * (n - 1), device_cus() * per_cu));
+}
+int fv_dt_blocks(int n, int nr) { return walk_blocks(n, nr, 2); }
 
 void launch_fv_centers(const FvArgs& a, double* c, hipStream_t s)
 {
     hipLaunchKernelGGL(k_fv_centers, dim3(blocks_for(fv_real_cells(a.n, a.nr))), dim3(FV_BLOCK), 0, s, a, c);
 }
 
-void launch_fv_columns(const FvArgs& a, double* columns, hipStream_t s)
+void launch_fv_centroids(const FvArgs& a, double* centroids, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_fv_centroids, dim3(blocks_for(10LL * (a.n - 1) * (a.n - 1))), dim3(FV_BLOCK), 0, s, a,
+                       centroids);
+}
+
+void launch_fv_ghost_columns(const int32_t* pairs, int cnt, double* centroids, hipStream_t s)
+{
+    if (cnt == 0) return;
+    hipLaunchKernelGGL(k_fv_ghost_columns, dim3(blocks_for(cnt)), dim3(FV_BLOCK), 0, s, pairs, cnt, centroids);
+}
+
+void launch_fv_columns(const FvArgs& a, const double* centroids, double* columns, hipStream_t s)
 {
     hipLaunchKernelGGL(k_fv_columns, dim3(blocks_for(10LL * (a.n - 1) * (a.n - 1))), dim3(FV_BLOCK), 0, s, a,
-                       columns);
+                       centroids, columns);
 }
 
 void launch_fv_ghost(const int32_t* pairs, int cnt, int nr, int ncomp, double* f, hipStream_t s)
@@ -603,18 +813,26 @@ void launch_fv_ghost(const int32_t* pairs, int cnt, int nr, int ncomp, double* f
                        ncomp, f);
 }
 
+void launch_fv_ghost2(const int32_t* pairs, int cnt, int nr, double* f, double* g, hipStream_t s)
+{
+    if (cnt == 0) return;
+    hipLaunchKernelGGL(k_fv_ghost2, dim3(blocks_for((int64_t)cnt * (nr - 1))), dim3(FV_BLOCK), 0, s, pairs, cnt, nr, f,
+                       g);
+}
+
 void launch_fv_dt(const FvArgs& a, const double* vel, double kappa, double* part, double* out, hipStream_t s)
 {
     const int nb = fv_dt_blocks(a.n, a.nr);
-    hipLaunchKernelGGL(k_fv_dt, dim3(nb), dim3(FV_BLOCK), 0, s, a, vel, kappa, part);
+    hipLaunchKernelGGL(k_fv_dt, dim3(nb), dim3(64 * FV_STRIPS), 0, s, a, a.columns, vel, kappa, part);
     hipLaunchKernelGGL(k_min_finalize, dim3(1), dim3(256), 0, s, part, nb, out);
 }
 
 void launch_fct_predictor(const FvArgs& a, const double* vel, const double* T, double dt, double kappa,
-                          const double* source, int subtract_div, double* TL, double* ad, hipStream_t s)
+                          const double* source, int subtract_div, double* TL, double* ad, const FctFused& fused,
+                          hipStream_t s)
 {
-    hipLaunchKernelGGL(k_fct_predictor, dim3(blocks_for(fv_real_cells(a.n, a.nr))), dim3(FV_BLOCK), 0, s, a, vel, T,
-                       dt, kappa, source, subtract_div, TL, ad, fv_size(a.n, a.nr));
+    hipLaunchKernelGGL(k_fct_predictor, dim3(walk_blocks(a.n, a.nr, 1)), dim3(64 * FV_STRIPS), 0, s, a, a.columns, vel, T, dt, kappa,
+                       source, subtract_div, TL, ad, fv_size(a.n, a.nr), fused);
 }
 
 void launch_fv_dirichlet(int n, int nr, double* f, int apply_cmb, double t_cmb, int apply_surf, double t_surf,
@@ -630,11 +848,17 @@ void launch_fct_limiter(int n, int nr, const double* TL, const double* ad, doubl
                        fv_size(n, nr), Rp, Rm);
 }
 
+void launch_fct_limiter_sums(int n, int nr, const double* TL, double* Rp, double* Rm, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_fct_limiter_sums, dim3(blocks_for(fv_real_cells(n, nr))), dim3(FV_BLOCK), 0, s, n, nr, TL, Rp,
+                       Rm);
+}
+
 void launch_fct_correction(int n, int nr, const double* TL, const double* ad, const double* Rp, const double* Rm,
                            double* T, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_fct_correction, dim3(blocks_for(fv_real_cells(n, nr))), dim3(FV_BLOCK), 0, s, n, nr, TL,
-                       ad, fv_size(n, nr), Rp, Rm, T);
+    hipLaunchKernelGGL(k_fct_correction, dim3(blocks_for(fv_real_cells(n, nr))), dim3(FV_BLOCK), 0, s, n, nr, TL, ad,
+                       fv_size(n, nr), Rp, Rm, T);
 }
 
 void launch_fv_lumped_scale(const double* D, double* u, int64_t N, hipStream_t s)

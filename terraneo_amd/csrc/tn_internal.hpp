@@ -74,6 +74,9 @@ struct DevBuf {
     }
 };
 
+// compute units of the current device
+int device_cus();
+
 // ---------------------------------------------------------------- mesh level
 // Lateral geometry of one wedge, radius-independent part of J^{-T}:
 //   J = A diag(r_mid, r_mid, dr/2),  A = [v1-v0, v2-v0, (v0+v1+v2)/3]
