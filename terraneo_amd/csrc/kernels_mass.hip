@@ -1,0 +1,209 @@
+// Mass operators on wedges: VectorMass (vector_mass.hpp:83-153), lumped KMass
+// (kmass.hpp:97-185).
+#include <algorithm>
+
+#include "tn_eps_march.hpp"
+#include "tn_internal.hpp"
+#include "tn_march.hpp"
+#include "tn_reduce.hpp"
+#include "tn_stokes.hpp"
+
+namespace tn {
+namespace {
+
+// VectorMass and the lumped k-mass (kmass.hpp) as a gather.  The lumped k-mass is
+// the row sum of the k-weighted matrix: with sum_j N_j = 1 its entry is
+// sum_q w_q k_h(q) N_i(q) |det|, the consistent mass matrix applied to the nodal
+// k by the same rule, so both are this kernel (the Schur diagonal of 0.36 M
+// pressure nodes took 426 us as quadrature per node and wedge, under 10 us here).
+// Every node copy is written once, y_i = sum over the wedges of its diamond that
+// contain it of (M_w x)_i; no atomics, so the result repeats bit for bit.  The
+// reference's Felippa 3x2 rule factors into the 3-point triangle rule, exact for
+// the lateral products (the P1 triangle mass (1 + delta_ij) / 24 times
+// |det(V0, V1, V2)|), and the 2-point Gauss rule in zeta for rho^2 hat_a hat_b,
+// which is not exact (degree 4) and is kept:
+//   M_w[i][j] = |det_w| (1 + delta_ij) / 24 x h sum_{g = -+1/sqrt 3} rho(g)^2 hat_a(g) hat_b(g).
+// Summed over the six wedges around a lateral node this is a 7-point lateral
+// stencil (the node and its neighbours (x+-1, y), (x, y+-1), (x-1, y+1),
+// (x+1, y-1)) times a 3-point radial stencil; |det_w| comes from the mesh's
+// wedge table (geo[..][9]).
+//
+// Vectors: a thread per node.
+template <typename T>
+__global__ __launch_bounds__(256) void k_mass_stencil(MassArgs<T> a)
+{
+    const int n = a.n, nr = a.nr, nc = n - 1;
+    const int64_t N = 10LL * n * n * nr;
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= N) return;
+    const int r = (int)(t % nr);
+    const int y = (int)((t / nr) % n);
+    const int x = (int)((t / ((int64_t)nr * n)) % n);
+    const int d = (int)(t / ((int64_t)nr * n * n));
+    auto det = [&](int qx, int qy, int w) -> double {
+        if (qx < 0 || qy < 0 || qx >= nc || qy >= nc) return 0.0;
+        return a.geo[((((int64_t)d * nc + qx) * nc + qy) * 2 + w) * GEO_STRIDE + 9];
+    };
+    // the six wedges around (x, y): quad (x, y) w0; (x-1, y) w0, w1; (x, y-1) w0, w1; (x-1, y-1) w1
+    const double a0 = det(x, y, 0), b0 = det(x - 1, y, 0), b1 = det(x - 1, y, 1);
+    const double c0 = det(x, y - 1, 0), c1 = det(x, y - 1, 1), d1 = det(x - 1, y - 1, 1);
+    constexpr double s = 1.0 / 24.0;
+    constexpr int NB = 7;
+    const int ox[NB] = {0, 1, 0, -1, 0, -1, 1}, oy[NB] = {0, 0, 1, 0, -1, 1, -1};
+    const double wl[NB] = {2.0 * s * (a0 + b0 + b1 + c0 + c1 + d1), s * (a0 + c1), s * (a0 + b1),
+                           s * (b0 + d1),                          s * (c0 + d1), s * (b0 + b1), s * (c0 + c1)};
+    // radial stencil: the node's own level and the levels below / above
+    constexpr double g = 0.57735026918962584;  // 1/sqrt(3)
+    constexpr double hm = 0.5 * (1.0 + g), hp = 0.5 * (1.0 - g);  // bottom hat at zeta = -g, +g
+    double cm = 0.0, c0r = 0.0, cp = 0.0;
+    if (r > 0) {  // layer (r-1, r): the node is its top level
+        const double r1 = a.radii[r - 1], h = 0.5 * (a.radii[r] - r1);
+        const double rm = r1 + h * (1.0 - g), rp = r1 + h * (1.0 + g);
+        c0r += h * (rm * rm * hp * hp + rp * rp * hm * hm);
+        cm = h * (rm * rm + rp * rp) * hm * hp;
+    }
+    if (r < nr - 1) {  // layer (r, r+1): the node is its bottom level
+        const double r1 = a.radii[r], h = 0.5 * (a.radii[r + 1] - r1);
+        const double rm = r1 + h * (1.0 - g), rp = r1 + h * (1.0 + g);
+        c0r += h * (rm * rm * hm * hm + rp * rp * hp * hp);
+        cp = h * (rm * rm + rp * rp) * hm * hp;
+    }
+    double acc[3] = {0, 0, 0};
+#pragma unroll
+    for (int k = 0; k < NB; ++k) {
+        if (wl[k] == 0.0) continue;  // a neighbour outside the diamond (no wedge holds it)
+        const int64_t col = (((int64_t)d * n + x + ox[k]) * n + y + oy[k]) * nr + r;
+        for (int c = 0; c < a.ncomp; ++c) {
+            const T* xc = a.x + c * N + col;
+            double v = c0r * (double)xc[0];
+            if (r > 0) v += cm * (double)xc[-1];
+            if (r < nr - 1) v += cp * (double)xc[1];
+            acc[c] += wl[k] * v;
+        }
+    }
+    for (int c = 0; c < a.ncomp; ++c) a.y[c * N + t] = (T)acc[c];
+}
+
+// One component (the projection's CG, the Schur diagonal): a wave walks an even
+// run of consecutive radial columns, its lanes on 64 levels.  The radial weights
+// stay in registers for the whole run, the lateral ones are wave-uniform, and the
+// next column is loaded while one is summed.  With dot != null it also leaves the
+// block's part of the sum over all node copies of x . y, which for x equal on a
+// node's copies is the owned dot of x with the interface-summed y.  What binds is
+// the vector cache (21 loads per node).  Level 5 x 33: 13.8 us with the dot, against
+// 13.1 us and 5.2 + 3.6 us for a dot pass with a thread per node; level 7 x 129 430
+// against 455 us.
+constexpr int MASS_WAVES = 4;
+template <typename T>
+__global__ __launch_bounds__(64 * MASS_WAVES) void k_mass_columns(MassArgs<T> a)
+{
+    constexpr int NB = 7;
+    const int n = a.n, nr = a.nr, nc = n - 1;
+    const int nlat = 10 * n * n;
+    const int lane = threadIdx.x & 63;
+    const int waves = gridDim.x * MASS_WAVES;
+    const int wave =
+        __builtin_amdgcn_readfirstlane(xcd_tile(blockIdx.x, gridDim.x) * MASS_WAVES + (int)(threadIdx.x >> 6));
+    const int lat0 = march::run_begin(nlat, wave, waves), lat1 = march::run_begin(nlat, wave + 1, waves);
+    struct Col {
+        T v[NB][3];  // levels r - 1, r, r + 1 of the node's column and its six lateral neighbours
+    };
+    double sum = 0.0;
+    for (int r0 = 0; r0 < nr; r0 += 64) {
+        const int r = min(r0 + lane, nr - 1);
+        const bool on = r0 + lane < nr;
+        // column lat's values; neighbours outside the diamond are in no wedge (weight 0): not read
+        auto load = [&](int lat, Col& q) {
+            const int y = lat % n, x = (lat / n) % n;
+            const int off[NB] = {0, n, 1, -n, -1, 1 - n, n - 1};
+            const bool in[NB] = {true,  x < n - 1, y < n - 1, x > 0, y > 0, x > 0 && y < n - 1, x < n - 1 && y > 0};
+#pragma unroll
+            for (int k = 0; k < NB; ++k) {
+                const T* xc = a.x + (int64_t)(lat + (in[k] ? off[k] : 0)) * nr + r;
+                q.v[k][0] = q.v[k][1] = q.v[k][2] = T(0);
+                if (in[k]) {
+                    q.v[k][1] = xc[0];
+                    if (r > 0) q.v[k][0] = xc[-1];
+                    if (r < nr - 1) q.v[k][2] = xc[1];
+                }
+            }
+        };
+        const double ra = a.radii[r > 0 ? r - 1 : r], rb = a.radii[r], rc = a.radii[r < nr - 1 ? r + 1 : r];
+        Col q[2];
+        if (lat0 < lat1) load(lat0, q[0]);
+        // radial stencil: the node's own level and the levels below / above
+        constexpr double g = 0.57735026918962584;  // 1/sqrt(3)
+        constexpr double hm = 0.5 * (1.0 + g), hp = 0.5 * (1.0 - g);  // bottom hat at zeta = -g, +g
+        double cm = 0.0, c0r = 0.0, cp = 0.0;
+        if (r > 0) {  // layer (r-1, r): the node is its top level
+            const double r1 = ra, h = 0.5 * (rb - r1);
+            const double rm = r1 + h * (1.0 - g), rp = r1 + h * (1.0 + g);
+            c0r += h * (rm * rm * hp * hp + rp * rp * hm * hm);
+            cm = h * (rm * rm + rp * rp) * hm * hp;
+        }
+        if (r < nr - 1) {  // layer (r, r+1): the node is its bottom level
+            const double r1 = rb, h = 0.5 * (rc - r1);
+            const double rm = r1 + h * (1.0 - g), rp = r1 + h * (1.0 + g);
+            c0r += h * (rm * rm * hm * hm + rp * rp * hp * hp);
+            cp = h * (rm * rm + rp * rp) * hm * hp;
+        }
+        auto finish = [&](int lat, const Col& q) {
+            const int y = lat % n, x = (lat / n) % n, d = lat / (n * n);
+            auto det = [&](int qx, int qy, int w) -> double {
+                if (qx < 0 || qy < 0 || qx >= nc || qy >= nc) return 0.0;
+                return a.geo[((((int64_t)d * nc + qx) * nc + qy) * 2 + w) * GEO_STRIDE + 9];
+            };
+            // the six wedges around (x, y): quad (x, y) w0; (x-1, y) w0, w1; (x, y-1) w0, w1; (x-1, y-1) w1
+            const double a0 = det(x, y, 0), b0 = det(x - 1, y, 0), b1 = det(x - 1, y, 1);
+            const double c0 = det(x, y - 1, 0), c1 = det(x, y - 1, 1), d1 = det(x - 1, y - 1, 1);
+            constexpr double s = 1.0 / 24.0;
+            const double wl[NB] = {2.0 * s * (a0 + b0 + b1 + c0 + c1 + d1), s * (a0 + c1), s * (a0 + b1),
+                                   s * (b0 + d1),                          s * (c0 + d1), s * (b0 + b1), s * (c0 + c1)};
+            double acc = 0.0;
+#pragma unroll
+            for (int k = 0; k < NB; ++k)
+                acc += wl[k] * (c0r * (double)q.v[k][1] + cm * (double)q.v[k][0] + cp * (double)q.v[k][2]);
+            if (on) {
+                a.y[(int64_t)lat * nr + r] = (T)acc;
+                sum += (double)q.v[0][1] * acc;
+            }
+        };
+        int lat = lat0;
+        for (; lat + 1 < lat1; lat += 2) {
+            load(lat + 1, q[1]);
+            finish(lat, q[0]);
+            if (lat + 2 < lat1) load(lat + 2, q[0]);
+            finish(lat + 1, q[1]);
+        }
+        if (lat < lat1) finish(lat, q[0]);
+    }
+    if (a.dot) block_partial(sum, a.dot);
+}
+
+}  // namespace
+
+int mass_blocks(int n)
+{
+    // a wave per column on small meshes, runs of columns on large ones; 1024 blocks hold
+    // every SIMD's four waves, and the users of the dot add up a partial sum per block
+    const int nlat = 10 * n * n;
+    return std::max(1, std::min((nlat + MASS_WAVES - 1) / MASS_WAVES, REDUCE_MAX_BLOCKS / 2));
+}
+
+template <typename T>
+void launch_mass(const MassArgs<T>& a, hipStream_t s)
+{
+    TN_REQUIRE(a.ncomp == 1 || (a.ncomp == 3 && !a.dot), "mass: ncomp must be 1, or 3 without the dot");
+    TN_REQUIRE(a.geo, "mass: wedge table missing");
+    const int64_t N = 10LL * a.n * a.n * a.nr;
+    if (a.ncomp == 3)
+        hipLaunchKernelGGL((k_mass_stencil<T>), dim3((unsigned)((N + 255) / 256)), dim3(256), 0, s, a);
+    else
+        hipLaunchKernelGGL((k_mass_columns<T>), dim3((unsigned)mass_blocks(a.n)), dim3(64 * MASS_WAVES), 0, s, a);
+    TN_HIP(hipGetLastError());
+}
+
+template void launch_mass<double>(const MassArgs<double>&, hipStream_t);
+template void launch_mass<float>(const MassArgs<float>&, hipStream_t);
+
+}  // namespace tn

@@ -26,14 +26,31 @@ using tn::MeshLevel;
 
 namespace tn {
 
+// the tables of B and B^T, built with the operator (not in the apply path)
+template <typename T>
+void coupling_build(tn_stokes* K)
+{
+    auto& mf = const_cast<tn_mesh*>(K->vel)->lvl.dev();
+    const size_t lat = (size_t)coupling_lat_elems(mf.n);
+    K->coupling.alloc((lat + 6 * (size_t)mf.nr) * sizeof(T));
+    T* t = (T*)K->coupling.p;
+    launch_coupling_tables<T>(mf.d_coords.p, mf.d_radii.p, mf.n, mf.nr, t, t + lat, 0);
+    TN_HIP(hipStreamSynchronize(0));  // applies may come on any stream
+}
+
+template <typename T>
+const T* coupling_rad(const tn_stokes* K)
+{
+    return (const T*)K->coupling.p + coupling_lat_elems(K->vel->lvl.n);
+}
+
 template <typename T>
 void div_t(tn_stokes* K, const void* u, void* p, hipStream_t s)
 {
     auto& mf = const_cast<tn_mesh*>(K->vel)->lvl.dev();
     auto& mc = const_cast<tn_mesh*>(K->pre)->lvl.dev();
-    TN_REQUIRE(K->div_tmp.n == sizeof(T) * (size_t)div_scratch_elems(mc.n, mc.nr), "B: scratch not allocated");
-    DivArgs<T> a{mf.d_coords.p, mf.d_radii.p, mf.n,  mf.nr,         mc.n,         mc.nr,
-                 K->A->bc_cmb,  K->A->bc_surf, (const T*)u, (T*)p, (T*)K->div_tmp.p};
+    DivArgs<T> a{(const T*)K->coupling.p, coupling_rad<T>(K), mf.n, mf.nr, mc.n, mc.nr,
+                 K->A->bc_cmb, K->A->bc_surf, (const T*)u, (T*)p};
     launch_div<T>(a, s);
     launch_interface_sum<T>(mc, 1, (T*)p, s);
 }
@@ -43,10 +60,8 @@ void grad_t(tn_stokes* K, const void* p, void* u, bool add, bool comm, hipStream
 {
     auto& mf = const_cast<tn_mesh*>(K->vel)->lvl.dev();
     auto& mc = const_cast<tn_mesh*>(K->pre)->lvl.dev();
-    constexpr int W = grad_march_waves<T>();
-    const int seg = march_seg_for(mf.n, W - 1, sizeof(T) == 8 ? W : 2 * W);
-    GradArgs<T> a{mf.d_coords.p, mf.d_radii.p, mf.n,          mf.nr,        mc.n, mc.nr, K->A->bc_cmb,
-                  K->A->bc_surf, (const T*)p,   (T*)u, seg, add ? 1 : 0, march_guard()};
+    GradArgs<T> a{(const T*)K->coupling.p, coupling_rad<T>(K), mf.n, mf.nr, mc.n, mc.nr,
+                  K->A->bc_cmb, K->A->bc_surf, (const T*)p, (T*)u, add ? 1 : 0};
     launch_grad<T>(a, s);
     if (comm) launch_interface_sum<T>(mf, 3, (T*)u, s);
 }
@@ -160,9 +175,10 @@ int tn_stokes_create(const tn_mesh* vel, const tn_mesh* pre, tn_eps* A, tn_stoke
     K->vel = vel;
     K->pre = pre;
     K->A = A;
-    // B's scratch (per-cell corner sums) is allocated here, not in the apply path
-    const size_t esize = A->dtype == TN_F64 ? sizeof(double) : sizeof(float);
-    K->div_tmp.alloc(esize * (size_t)tn::div_scratch_elems(pre->lvl.n, pre->lvl.nr));
+    if (A->dtype == TN_F64)
+        tn::coupling_build<double>(K.get());
+    else
+        tn::coupling_build<float>(K.get());
     *out = K.release();
     TN_API_END
 }
