@@ -53,6 +53,8 @@ __device__ __forceinline__ double vec_get(const double2& v, int i) { return i ==
 // for the vectors in flight; at 4 the compiler waits for every load)
 constexpr int STORED_PREFETCH = 6;
 constexpr int STORED_WAVES_PER_EU = 3;
+// the same with a wave per wedge (FP64 storage; a wedge in FP32 fits whole)
+constexpr int STORED_DEEP = 32;
 // The matrix stream is read once per apply and is larger than the L2 and the
 // last-level cache: non-temporal loads keep it from evicting the vectors.
 __device__ __forceinline__ float4 ld_stream(const float4* p)
@@ -746,15 +748,17 @@ __global__ void k_gca_select(const T* __restrict__ flags, int n0, int nr0, int l
 // divergent branch here makes the compiler hoist the whole matrix stream):
 // keep[t] = 0 zeroes level t (Dirichlet), proj[t] = 1 projects it tangentially
 // with the corner normals nrm (free-slip).
-template <typename T, typename S, bool DIAG>
+//
+// Wedges W0 .. W1 - 1, PD matrix vectors in flight per lane.
+template <typename T, typename S, bool DIAG, int PD, int W0, int W1>
 __device__ __forceinline__ void stored_cell_sums(const StoredArgs<T, S>& a, int64_t cell, const int64_t latc[4],
-                                                 int cc, T scale, const T keep[2], const T proj[2],
-                                                 const T nrm[4][3], T yb[4][3], T yt[4][3])
+                                                  int cc, T scale, const T keep[2], const T proj[2],
+                                                  const T nrm[4][3], T yb[4][3], T yt[4][3])
 {
     constexpr int WCORN[2][3] = {{0, 1, 2}, {3, 2, 1}};
     const int64_t N = 10LL * a.n * a.n * a.nr;
 #pragma unroll
-    for (int w = 0; w < 2; ++w) {
+    for (int w = W0; w < W1; ++w) {
         T xs[18];
 #pragma unroll
         for (int j = 0; j < 6; ++j) {
@@ -786,12 +790,11 @@ __device__ __forceinline__ void stored_cell_sums(const StoredArgs<T, S>& a, int6
             // PD loads per wave are in flight (latency, not bandwidth, bounds a
             // stream with one load in flight per wave).
             constexpr int V = stored_vec<S>(), NV = WEDGE_SLOTS / V;
-            constexpr int PD = STORED_PREFETCH;
             using Vec = VecOf<S>;
             const Vec* vp = reinterpret_cast<const Vec*>(a.stored + stored_at<S>(cell, w, 0));
             Vec buf[NV];
 #pragma unroll
-            for (int q = 0; q < PD; ++q) buf[q] = ld_stream(vp + q * 64);
+            for (int q = 0; q < (PD < NV ? PD : NV); ++q) buf[q] = ld_stream(vp + q * 64);
             int k = 0;
 #pragma unroll
             for (int i = 0; i < 18; ++i) {
@@ -807,11 +810,17 @@ __device__ __forceinline__ void stored_cell_sums(const StoredArgs<T, S>& a, int6
     }
 }
 
-template <typename T, typename S, bool DIAG>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(STORED_WAVES_PER_EU, STORED_WAVES_PER_EU))) void k_stored_cells(StoredArgs<T, S> a)
+//
+// SPLIT: where the cells leave the SIMDs with a wave or two, a block of two waves per
+// quad takes a wedge each, with as many matrix vectors in flight as the registers of
+// two waves per SIMD hold: the stream is read in one to three latencies, not in twenty.
+template <typename T, typename S, bool DIAG, bool SPLIT>
+__global__ __launch_bounds__(SPLIT ? 128 : 256)
+    __attribute__((amdgpu_waves_per_eu(SPLIT ? 2 : STORED_WAVES_PER_EU, SPLIT ? 2 : STORED_WAVES_PER_EU)))
+    void k_stored_cells(StoredArgs<T, S> a)
 {
     const int lane = threadIdx.x & 63;
-    const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+    const int64_t wave = SPLIT ? (int64_t)blockIdx.x : ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const int ncr = a.nr - 1, ncl = a.n - 1;
     const int nch = (ncr + 63) >> 6;
     const int64_t ncol = 10LL * ncl * ncl;
@@ -847,7 +856,40 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(STORED_WAVE
         for (int j = 0; j < 3; ++j) yb[k][j] = yt[k][j] = T(0);
     // (the lane condition also keeps the compiler from hoisting the whole
     // matrix stream of both wedges into registers ahead of the arithmetic)
-    if (valid) stored_cell_sums<T, S, DIAG>(a, col * ncr + cc, latc, cc, scale, keep, proj, nrm, yb, yt);
+    if constexpr (!SPLIT) {
+        if (valid)
+            stored_cell_sums<T, S, DIAG, STORED_PREFETCH, 0, 2>(a, col * ncr + cc, latc, cc, scale, keep, proj, nrm, yb,
+                                                                yt);
+    } else {
+        constexpr int PD = sizeof(S) == 8 ? STORED_DEEP : WEDGE_SLOTS / stored_vec<S>();
+        __shared__ T part[18][64];  // wedge 1's sums of corners 1 to 3
+        const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        if (w == 1) {
+            if (valid) {
+                stored_cell_sums<T, S, DIAG, PD, 1, 2>(a, col * ncr + cc, latc, cc, scale, keep, proj, nrm, yb, yt);
+#pragma unroll
+                for (int k = 1; k < 4; ++k)
+#pragma unroll
+                    for (int j = 0; j < 3; ++j) {
+                        part[(k - 1) * 6 + j][lane] = yb[k][j];
+                        part[(k - 1) * 6 + 3 + j][lane] = yt[k][j];
+                    }
+            }
+        } else if (valid) {
+            stored_cell_sums<T, S, DIAG, PD, 0, 1>(a, col * ncr + cc, latc, cc, scale, keep, proj, nrm, yb, yt);
+        }
+        __syncthreads();
+        if (w == 1) return;
+        if (valid) {
+#pragma unroll
+            for (int k = 1; k < 4; ++k)
+#pragma unroll
+                for (int j = 0; j < 3; ++j) {
+                    yb[k][j] += part[(k - 1) * 6 + j][lane];
+                    yt[k][j] += part[(k - 1) * 6 + 3 + j][lane];
+                }
+        }
+    }
     // radial merge (level c = bottom of cell c + top of cell c-1) and write-out
 #pragma unroll
     for (int k = 0; k < 4; ++k)
@@ -1216,11 +1258,16 @@ void launch_stored_apply(const StoredArgs<T, S>& a, bool diagonal, hipStream_t s
     const int64_t N = 10LL * a.n * a.n * a.nr;
     const dim3 gg((unsigned)((N + 255) / 256)), bg(256);
     if (diagonal) {
-        hipLaunchKernelGGL((k_stored_cells<T, S, true>), gr, bl, 0, s, a);
+        hipLaunchKernelGGL((k_stored_cells<T, S, true, false>), gr, bl, 0, s, a);
         TN_HIP(hipGetLastError());
         hipLaunchKernelGGL((k_stored_gather<T, S, true>), gg, bg, 0, s, a);
     } else {
-        hipLaunchKernelGGL((k_stored_cells<T, S, false>), gr, bl, 0, s, a);
+        // one wave per SIMD or less: latency counts (640 waves: FP64 12.4 us, 6.5 split;
+        // FP32 11.5, 8.0); at 2560 waves the bandwidth does (FP32: 18.6 us, 20.3 split)
+        if (waves <= 4 * device_cus())
+            hipLaunchKernelGGL((k_stored_cells<T, S, false, true>), dim3((unsigned)waves), dim3(128), 0, s, a);
+        else
+            hipLaunchKernelGGL((k_stored_cells<T, S, false, false>), gr, bl, 0, s, a);
         TN_HIP(hipGetLastError());
         hipLaunchKernelGGL((k_stored_gather<T, S, false>), gg, bg, 0, s, a);
     }
