@@ -87,25 +87,32 @@ __global__ __launch_bounds__(64 * CG_WAVES) void k_cg_update(T* __restrict__ x, 
 {
     const double done = st.ctl[CgState::DONE];
     const double rr = st.rr[CgState::slot(it - 1)];
+    const int lane = threadIdx.x & 63;
+    const int nlat = (int)(N / nr), ncol = nlat * ncomp, step = gridDim.x * CG_WAVES;
+    const int col0 = blockIdx.x * CG_WAVES + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    // (the first column's values are under way while the partials are added)
+    const int64_t at = (int64_t)min(col0, ncol - 1) * nr + min(lane, nr - 1);
+    const T x0 = x[at], p0 = p[at], r0 = r[at], a0 = ap[at];
     const double pap = partials_total(st.part_pap, st.npap);
     if (done != 0.0 && done < (double)it) return;
     const T alpha = (T)(rr / pap);
     double s = 0.0;
-    const int lane = threadIdx.x & 63;
-    const int nlat = (int)(N / nr), ncol = nlat * ncomp, step = gridDim.x * CG_WAVES;
     const int4* groups = reinterpret_cast<const int4*>(st.groups);
-    for (int col = blockIdx.x * CG_WAVES + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); col < ncol; col += step) {
+    for (int col = col0; col < ncol; col += step) {
         const int c = col / nlat, lat = col - c * nlat;
         const bool own = owned_lat[lat];
         const int g = groups ? st.group_of[lat] : -1;
         const int64_t base = (int64_t)col * nr;
         for (int k = lane; k < nr; k += 64) {
             const int64_t i = base + k;
-            const T xv = x[i], pv = p[i], rv = r[i];
-            T av;
-            if (g < 0) {
+            T xv = x0, pv = p0, rv = r0, av = a0;
+            if (col != col0 || k != lane) {
+                xv = x[i];
+                pv = p[i];
+                rv = r[i];
                 av = ap[i];
-            } else {
+            }
+            if (g >= 0) {
                 const int4 q = groups[2 * g], q2 = groups[2 * g + 1];
                 const T* ac = ap + c * N + k;
                 double v = 0.0 + (double)ac[(int64_t)q.x * nr] + (double)ac[(int64_t)q.y * nr];
@@ -133,6 +140,9 @@ __global__ __launch_bounds__(256) void k_cg_direction(T* __restrict__ p, const T
 {
     const double done = st.ctl[CgState::DONE];
     const double rr_old = st.rr[CgState::slot(it - 1)];
+    // (the first elements are under way while the partials are added)
+    const int64_t first = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, at = first < count ? first : count - 1;
+    const T p0 = p[at], r0 = r[at];
     const double rr = partials_total(st.part_rr, st.nrr);
     if (done != 0.0 && done < (double)it) return;
     const T beta = (T)(rr / rr_old);
@@ -141,7 +151,8 @@ __global__ __launch_bounds__(256) void k_cg_direction(T* __restrict__ p, const T
         const double res = sqrt(rr);
         if (res / st.ctl[CgState::R0] <= st.rtol || res < st.atol) st.ctl[CgState::DONE] = (double)it;
     }
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (int64_t)gridDim.x * blockDim.x)
+    if (first < count) p[first] = r0 + beta * p0;
+    for (int64_t i = first + (int64_t)gridDim.x * blockDim.x; i < count; i += (int64_t)gridDim.x * blockDim.x)
         p[i] = r[i] + beta * p[i];
 }
 

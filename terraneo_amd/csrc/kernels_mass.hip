@@ -87,12 +87,29 @@ __global__ __launch_bounds__(256) void k_mass_stencil(MassArgs<T> a)
 // One component (the projection's CG, the Schur diagonal): a wave walks an even
 // run of consecutive radial columns, its lanes on 64 levels.  The radial weights
 // stay in registers for the whole run, the lateral ones are wave-uniform, and the
-// next column is loaded while one is summed.  With dot != null it also leaves the
+// next column is loaded while one is summed.  A lane loads its own level and takes
+// the two beside it from the neighbouring lanes, so a window of 64 levels gives the
+// levels between its first and last (past 64 levels the windows overlap by two); with
+// 21 loads per node instead of 7 the vector cache was what bound it.  With dot != null it also leaves the
 // block's part of the sum over all node copies of x . y, which for x equal on a
-// node's copies is the owned dot of x with the interface-summed y.  What binds is
-// the vector cache (21 loads per node).  Level 5 x 33: 13.8 us with the dot, against
-// 13.1 us and 5.2 + 3.6 us for a dot pass with a thread per node; level 7 x 129 430
-// against 455 us.
+// node's copies is the owned dot of x with the interface-summed y.
+// Product with its interface sum: level 7 x 129 430 -> 282 us, level 6 x 65 47 us, level
+// 5 x 33 17 -> 12 us (the determinants, too, a column ahead: 14 without).
+// lane i receives lane i-1's (UP) or i+1's value, 0 at the end
+constexpr int LANE_UP = 0x138, LANE_DOWN = 0x130;  // DPP wave_shr:1, wave_shl:1
+template <int CTRL>
+__device__ __forceinline__ float lane_shift(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+}
+template <int CTRL>
+__device__ __forceinline__ double lane_shift(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffLL), CTRL, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, false);
+    return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
+}
 constexpr int MASS_WAVES = 4;
 template <typename T>
 __global__ __launch_bounds__(64 * MASS_WAVES) void k_mass_columns(MassArgs<T> a)
@@ -106,27 +123,31 @@ __global__ __launch_bounds__(64 * MASS_WAVES) void k_mass_columns(MassArgs<T> a)
         __builtin_amdgcn_readfirstlane(xcd_tile(blockIdx.x, gridDim.x) * MASS_WAVES + (int)(threadIdx.x >> 6));
     const int lat0 = march::run_begin(nlat, wave, waves), lat1 = march::run_begin(nlat, wave + 1, waves);
     struct Col {
-        T v[NB][3];  // levels r - 1, r, r + 1 of the node's column and its six lateral neighbours
+        T v[NB];        // the node's column and its six lateral neighbours
+        double det[6];  // the six wedges around it
     };
     double sum = 0.0;
-    for (int r0 = 0; r0 < nr; r0 += 64) {
+    for (int r0 = 0;; r0 += 62) {
         const int r = min(r0 + lane, nr - 1);
-        const bool on = r0 + lane < nr;
-        // column lat's values; neighbours outside the diamond are in no wedge (weight 0): not read
+        const bool on = r0 + lane < nr && (lane > 0 || r0 == 0) && (lane < 63 || r == nr - 1);
+        // column lat's values; neighbours and wedges outside the diamond count 0: not read
         auto load = [&](int lat, Col& q) {
-            const int y = lat % n, x = (lat / n) % n;
+            const int y = lat % n, x = (lat / n) % n, d = lat / (n * n);
             const int off[NB] = {0, n, 1, -n, -1, 1 - n, n - 1};
             const bool in[NB] = {true,  x < n - 1, y < n - 1, x > 0, y > 0, x > 0 && y < n - 1, x < n - 1 && y > 0};
 #pragma unroll
-            for (int k = 0; k < NB; ++k) {
-                const T* xc = a.x + (int64_t)(lat + (in[k] ? off[k] : 0)) * nr + r;
-                q.v[k][0] = q.v[k][1] = q.v[k][2] = T(0);
-                if (in[k]) {
-                    q.v[k][1] = xc[0];
-                    if (r > 0) q.v[k][0] = xc[-1];
-                    if (r < nr - 1) q.v[k][2] = xc[1];
-                }
-            }
+            for (int k = 0; k < NB; ++k) q.v[k] = in[k] ? a.x[(int64_t)(lat + off[k]) * nr + r] : T(0);
+            auto det = [&](int qx, int qy, int w) -> double {
+                if (qx < 0 || qy < 0 || qx >= nc || qy >= nc) return 0.0;
+                return a.geo[((((int64_t)d * nc + qx) * nc + qy) * 2 + w) * GEO_STRIDE + 9];
+            };
+            // quad (x, y) w0; (x-1, y) w0, w1; (x, y-1) w0, w1; (x-1, y-1) w1
+            q.det[0] = det(x, y, 0);
+            q.det[1] = det(x - 1, y, 0);
+            q.det[2] = det(x - 1, y, 1);
+            q.det[3] = det(x, y - 1, 0);
+            q.det[4] = det(x, y - 1, 1);
+            q.det[5] = det(x - 1, y - 1, 1);
         };
         const double ra = a.radii[r > 0 ? r - 1 : r], rb = a.radii[r], rc = a.radii[r < nr - 1 ? r + 1 : r];
         Col q[2];
@@ -148,24 +169,20 @@ __global__ __launch_bounds__(64 * MASS_WAVES) void k_mass_columns(MassArgs<T> a)
             cp = h * (rm * rm + rp * rp) * hm * hp;
         }
         auto finish = [&](int lat, const Col& q) {
-            const int y = lat % n, x = (lat / n) % n, d = lat / (n * n);
-            auto det = [&](int qx, int qy, int w) -> double {
-                if (qx < 0 || qy < 0 || qx >= nc || qy >= nc) return 0.0;
-                return a.geo[((((int64_t)d * nc + qx) * nc + qy) * 2 + w) * GEO_STRIDE + 9];
-            };
-            // the six wedges around (x, y): quad (x, y) w0; (x-1, y) w0, w1; (x, y-1) w0, w1; (x-1, y-1) w1
-            const double a0 = det(x, y, 0), b0 = det(x - 1, y, 0), b1 = det(x - 1, y, 1);
-            const double c0 = det(x, y - 1, 0), c1 = det(x, y - 1, 1), d1 = det(x - 1, y - 1, 1);
+            const double a0 = q.det[0], b0 = q.det[1], b1 = q.det[2], c0 = q.det[3], c1 = q.det[4], d1 = q.det[5];
             constexpr double s = 1.0 / 24.0;
             const double wl[NB] = {2.0 * s * (a0 + b0 + b1 + c0 + c1 + d1), s * (a0 + c1), s * (a0 + b1),
                                    s * (b0 + d1),                          s * (c0 + d1), s * (b0 + b1), s * (c0 + c1)};
             double acc = 0.0;
 #pragma unroll
-            for (int k = 0; k < NB; ++k)
-                acc += wl[k] * (c0r * (double)q.v[k][1] + cm * (double)q.v[k][0] + cp * (double)q.v[k][2]);
+            for (int k = 0; k < NB; ++k) {
+                const T vm = lane_shift<LANE_UP>(q.v[k]), vp = lane_shift<LANE_DOWN>(q.v[k]);
+                const double v0 = r > 0 ? (double)vm : 0.0, v2 = r < nr - 1 ? (double)vp : 0.0;
+                acc += wl[k] * (c0r * (double)q.v[k] + cm * v0 + cp * v2);
+            }
             if (on) {
                 a.y[(int64_t)lat * nr + r] = (T)acc;
-                sum += (double)q.v[0][1] * acc;
+                sum += (double)q.v[0] * acc;
             }
         };
         int lat = lat0;
@@ -176,6 +193,7 @@ __global__ __launch_bounds__(64 * MASS_WAVES) void k_mass_columns(MassArgs<T> a)
             finish(lat + 1, q[1]);
         }
         if (lat < lat1) finish(lat, q[0]);
+        if (r0 + 64 >= nr) break;
     }
     if (a.dot) block_partial(sum, a.dot);
 }
