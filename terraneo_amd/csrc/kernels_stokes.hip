@@ -116,31 +116,48 @@ __host__ __device__ constexpr bool coupling_has(int xo, int yo, int dx, int dy)
     return dx >= (xo ? 0 : -1) && dx <= 1 && dy >= (yo ? 0 : -1) && dy <= 1;
 }
 
-// lateral table: one thread per fine node column; slot values al[3], ga[3]
+// lateral table: a thread per fine node column and slot (slot values al[3], ga[3]; the
+// thread past the last slot writes the normal).  A thread with all seven slots kept them
+// in scratch and took 36 us for 42250 columns, 22 so.
 template <typename T>
 __global__ __launch_bounds__(256) void k_coupling_table(const double* __restrict__ coords, int n, T* __restrict__ tab)
 {
     constexpr int OFF[2][3][2] = {{{0, 0}, {1, 0}, {0, 1}}, {{1, 1}, {0, 1}, {1, 0}}};
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t t = tid >> 3;
+    const int slot = (int)(tid & 7);
+    static_assert(COUPLING_SLOTS == 7 && COUPLING_ENTRIES == 6 * (COUPLING_SLOTS + 1), "eight threads per column");
     if (t >= 10LL * n * n) return;
+    T* o = tab + t * COUPLING_ENTRIES + 6 * slot;
+    if (slot == COUPLING_SLOTS) {
+        for (int j = 0; j < 6; ++j) o[j] = j < 3 ? (T)coords[3 * t + j] : T(0);
+        return;
+    }
     const int y = (int)(t % n), x = (int)((t / n) % n), d = (int)(t / ((int64_t)n * n));
-    double v[COUPLING_SLOTS][6];
-    for (int k = 0; k < COUPLING_SLOTS; ++k)
-        for (int j = 0; j < 6; ++j) v[k][j] = 0.0;
+    double v[6] = {0, 0, 0, 0, 0, 0};
     for (int qx = x - 1; qx <= x; ++qx)
         for (int qy = y - 1; qy <= y; ++qy) {
             if (qx < 0 || qy < 0 || qx > n - 2 || qy > n - 2) continue;
+#pragma unroll
             for (int w = 0; w < 2; ++w) {
-                int m = -1;
-                double P[3][3];
+                int m = -1, il = -1;  // vertex of the wedge here, coarse shape of the slot
+#pragma unroll
                 for (int i = 0; i < 3; ++i) {
-                    const int px = qx + OFF[w][i][0], py = qy + OFF[w][i][1];
-                    if (px == x && py == y) m = i;
-                    const double* c = coords + 3 * (((int64_t)d * n + px) * n + py);
+                    if (qx + OFF[w][i][0] == x && qy + OFF[w][i][1] == y) m = i;
+                    if (coupling_slot(x & 1, y & 1, (qx >> 1) + OFF[w][i][0] - (x >> 1),
+                                      (qy >> 1) + OFF[w][i][1] - (y >> 1)) == slot)
+                        il = i;
+                }
+                if (m < 0 || il < 0) continue;
+                double P[3][3];
+#pragma unroll
+                for (int i = 0; i < 3; ++i) {
+                    const double* c = coords + 3 * (((int64_t)d * n + qx + OFF[w][i][0]) * n + qy + OFF[w][i][1]);
+#pragma unroll
                     for (int j = 0; j < 3; ++j) P[i][j] = c[j];
                 }
-                if (m < 0) continue;
                 double a[3], b[3];
+#pragma unroll
                 for (int j = 0; j < 3; ++j) {
                     a[j] = P[1][j] - P[0][j];
                     b[j] = P[2][j] - P[0][j];
@@ -151,26 +168,20 @@ __global__ __launch_bounds__(256) void k_coupling_table(const double* __restrict
                                       P[0][0] * a[1] - P[0][1] * a[0]};
                 const double nv[3] = {a[1] * b[2] - a[2] * b[1], a[2] * b[0] - a[0] * b[2], a[0] * b[1] - a[1] * b[0]};
                 const double s = a[0] * v1[0] + a[1] * v1[1] + a[2] * v1[2] > 0.0 ? -1.0 : 1.0;
-                const int flw = fine_lateral_wedge_idx(qx & 1, qy & 1, w);
-                for (int il = 0; il < 3; ++il) {
-                    const double M0 = LATM.m[flw][il][0], Mx = LATM.m[flw][il][1], Me = LATM.m[flw][il][2];
-                    const int dx = (qx >> 1) + OFF[w][il][0] - (x >> 1), dy = (qy >> 1) + OFF[w][il][1] - (y >> 1);
-                    double* o = v[coupling_slot(x & 1, y & 1, dx, dy)];
-                    for (int j = 0; j < 3; ++j) {
-                        const double n0 = m == 0 ? Mx + Me : (m == 1 ? -Mx : -Me);
-                        const double vv = m == 0 ? -(v1[j] + v3[j]) : (m == 1 ? v1[j] : v3[j]);
-                        const double n1 = m == 0 ? M0 - Mx - Me : (m == 1 ? Mx : Me);
-                        o[j] += s * (n0 * nv[j] + M0 * vv);
-                        o[3 + j] += s * n1 * nv[j];
-                    }
+                const double* M = LATM.m[fine_lateral_wedge_idx(qx & 1, qy & 1, w)][il];
+                const double M0 = M[0], Mx = M[1], Me = M[2];
+                const double n0 = m == 0 ? Mx + Me : (m == 1 ? -Mx : -Me);
+                const double n1 = m == 0 ? M0 - Mx - Me : (m == 1 ? Mx : Me);
+#pragma unroll
+                for (int j = 0; j < 3; ++j) {
+                    const double vv = m == 0 ? -(v1[j] + v3[j]) : (m == 1 ? v1[j] : v3[j]);
+                    v[j] += s * (n0 * nv[j] + M0 * vv);
+                    v[3 + j] += s * n1 * nv[j];
                 }
             }
         }
-    T* o = tab + t * COUPLING_ENTRIES;
-    for (int k = 0; k < COUPLING_SLOTS; ++k)
-        for (int j = 0; j < 6; ++j) o[6 * k + j] = (T)v[k][j];
-    for (int j = 0; j < COUPLING_ENTRIES - COUPLING_NORMAL; ++j)
-        o[COUPLING_NORMAL + j] = j < 3 ? (T)coords[3 * t + j] : T(0);
+#pragma unroll
+    for (int j = 0; j < 6; ++j) o[j] = (T)v[j];
 }
 
 // radial weights: [6][nr], wA_0..2 and wC_0..2 of fine level r for the coarse levels
@@ -641,8 +652,8 @@ int coupling_run(int64_t columns, int waves_per_simd)
 template <typename T>
 void launch_coupling_tables(const double* coords, const double* radii, int n, int nr, T* lat, T* rad, hipStream_t s)
 {
-    const int64_t cols = 10LL * n * n;
-    hipLaunchKernelGGL(k_coupling_table<T>, dim3((unsigned)((cols + 255) / 256)), dim3(256), 0, s, coords, n, lat);
+    const int64_t threads = 8 * 10LL * n * n;
+    hipLaunchKernelGGL(k_coupling_table<T>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, coords, n, lat);
     TN_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_coupling_radial<T>, dim3((unsigned)((nr + 255) / 256)), dim3(256), 0, s, radii, nr, rad);
     TN_HIP(hipGetLastError());
