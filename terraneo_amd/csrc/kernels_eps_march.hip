@@ -1,7 +1,9 @@
 // epsilon-div-div apply without global atomics: lateral march, CDNA4.
 //
-// Decomposition.  A block of W waves owns W-1 lateral node rows of one
-// diamond and one segment of node columns.  Wave w handles the quad strip
+// Decomposition.  A block of W waves owns W-1 lateral node rows and a run of
+// node columns (matrix apply: equal runs over all strips of all diamonds, which
+// may end one strip and begin the next; diagonal mode: a segment of one strip).
+// Wave w handles the quad strip
 // x = x0 - 1 + w and marches over the quads of that strip in y; its 64 lanes
 // are 64 radial cells (a chunk; chunks of one column are processed one after
 // the other), so every global load and store is radially contiguous.  A
@@ -19,8 +21,8 @@
 // chunk (kept in LDS until that chunk reaches the column).  Every node copy
 // is written exactly once with a plain store (Replace) or one
 // read-modify-write (Add).  The strip at a block edge is computed twice (once
-// as the halo wave 0 of the next block) and the column before a segment once
-// more: (W/(W-1)) * (S+1)/S redundant cell work instead of atomics.
+// as the halo wave 0 of the next block) and the column before a run or segment
+// of S columns once more: (W/(W-1)) * (S+1)/S redundant cell work instead of atomics.
 //
 // Boundary conditions are algebraic at the two boundary node levels, so the
 // per-cell arithmetic is the Neumann formula for every lane:

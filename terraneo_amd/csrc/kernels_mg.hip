@@ -686,7 +686,7 @@ __global__ void k_gca_collect(const T* __restrict__ k, int n, int nr, int levels
 // on-the-fly assembly for cells without a stored matrix): the cells of a
 // Galerkin level whose coarsest ancestor is not flagged get the level's own
 // rediscretized wedge matrices (geometry and nodal viscosity of the level).
-// One thread per (cell, wedge, component block q <= p), as k_gca_build.
+// One thread per (cell, wedge, component block q <= p).
 template <typename T, typename S>
 __global__ void k_gca_select(const T* __restrict__ flags, int n0, int nr0, int levels, const double* __restrict__ geo,
                              const double* __restrict__ radii, const T* __restrict__ eta,
@@ -1263,8 +1263,8 @@ void launch_stored_apply(const StoredArgs<T, S>& a, bool diagonal, hipStream_t s
         TN_HIP(hipGetLastError());
         hipLaunchKernelGGL((k_stored_gather<T, S, true>), gg, bg, 0, s, a);
     } else {
-        // one wave per SIMD or less: latency counts (640 waves: FP64 12.4 us, 6.5 split;
-        // FP32 11.5, 8.0); at 2560 waves the bandwidth does (FP32: 18.6 us, 20.3 split)
+        // one wave per SIMD or less: latency counts (FP64, 160 quads: 12.4 us, 6.5 split, 640
+        // quads 17.1, 11.1; FP32, 640 quads 11.5, 8.0); at 2560 waves the bandwidth does (FP32: 18.6 us, 20.3 split)
         if (waves <= 4 * device_cus())
             hipLaunchKernelGGL((k_stored_cells<T, S, false, true>), dim3((unsigned)waves), dim3(128), 0, s, a);
         else
