@@ -750,11 +750,12 @@ __global__ void k_gca_select(const T* __restrict__ flags, int n0, int nr0, int l
 // keep[t] = 0 zeroes level t (Dirichlet), proj[t] = 1 projects it tangentially
 // with the corner normals nrm (free-slip).
 //
-// Wedges W0 .. W1 - 1, PD matrix vectors in flight per lane.
-template <typename T, typename S, bool DIAG, int PD, int W0, int W1>
+// Wedges W0 .. W1 - 1, PD matrix vectors in flight per lane; begin() runs once a
+// wedge's first loads are under way, before its products.
+template <typename T, typename S, bool DIAG, int PD, int W0, int W1, class Begin>
 __device__ __forceinline__ void stored_cell_sums(const StoredArgs<T, S>& a, int64_t cell, const int64_t latc[4],
                                                   int cc, T scale, const T keep[2], const T proj[2],
-                                                  const T nrm[4][3], T yb[4][3], T yt[4][3])
+                                                  const T nrm[4][3], T yb[4][3], T yt[4][3], Begin begin)
 {
     constexpr int WCORN[2][3] = {{0, 1, 2}, {3, 2, 1}};
     const int64_t N = 10LL * a.n * a.n * a.nr;
@@ -796,6 +797,7 @@ __device__ __forceinline__ void stored_cell_sums(const StoredArgs<T, S>& a, int6
             Vec buf[NV];
 #pragma unroll
             for (int q = 0; q < (PD < NV ? PD : NV); ++q) buf[q] = ld_stream(vp + q * 64);
+            begin();
             int k = 0;
 #pragma unroll
             for (int i = 0; i < 18; ++i) {
@@ -815,12 +817,16 @@ __device__ __forceinline__ void stored_cell_sums(const StoredArgs<T, S>& a, int6
 // SPLIT: where the cells leave the SIMDs with a wave or two, a block of two waves per
 // quad takes a wedge each, with as many matrix vectors in flight as the registers of
 // two waves per SIMD hold: the stream is read in one to three latencies, not in twenty.
+// The second wave loads its wedge meanwhile and goes on from the first one's sums of
+// the corners that both wedges have, so every sum is formed in the one-wave order and
+// a level's bits do not depend on its size.
 template <typename T, typename S, bool DIAG, bool SPLIT>
 __global__ __launch_bounds__(SPLIT ? 128 : 256)
     __attribute__((amdgpu_waves_per_eu(SPLIT ? 2 : STORED_WAVES_PER_EU, SPLIT ? 2 : STORED_WAVES_PER_EU)))
     void k_stored_cells(StoredArgs<T, S> a)
 {
     const int lane = threadIdx.x & 63;
+    const int split = SPLIT ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;  // the wave's wedge
     const int64_t wave = SPLIT ? (int64_t)blockIdx.x : ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const int ncr = a.nr - 1, ncl = a.n - 1;
     const int nch = (ncr + 63) >> 6;
@@ -860,40 +866,40 @@ __global__ __launch_bounds__(SPLIT ? 128 : 256)
     if constexpr (!SPLIT) {
         if (valid)
             stored_cell_sums<T, S, DIAG, STORED_PREFETCH, 0, 2>(a, col * ncr + cc, latc, cc, scale, keep, proj, nrm, yb,
-                                                                yt);
+                                                                yt, [] {});
     } else {
+        // (lanes past the last cell run along with the last cell's matrices and zero
+        // vectors; each wave meets one of the two barriers)
         constexpr int PD = sizeof(S) == 8 ? STORED_DEEP : WEDGE_SLOTS / stored_vec<S>();
-        __shared__ T part[18][64];  // wedge 1's sums of corners 1 to 3
-        const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-        if (w == 1) {
-            if (valid) {
-                stored_cell_sums<T, S, DIAG, PD, 1, 2>(a, col * ncr + cc, latc, cc, scale, keep, proj, nrm, yb, yt);
+        __shared__ T part[12][64];  // wedge 0's sums of corners 1 and 2
+        auto shared = [&](int k, int j, int t) -> T& { return part[((k - 1) * 3 + j) * 2 + t][lane]; };
+        if (split == 0) {
+            stored_cell_sums<T, S, DIAG, PD, 0, 1>(a, col * ncr + cc, latc, cc, scale, keep, proj, nrm, yb, yt, [] {});
 #pragma unroll
-                for (int k = 1; k < 4; ++k)
-#pragma unroll
-                    for (int j = 0; j < 3; ++j) {
-                        part[(k - 1) * 6 + j][lane] = yb[k][j];
-                        part[(k - 1) * 6 + 3 + j][lane] = yt[k][j];
-                    }
-            }
-        } else if (valid) {
-            stored_cell_sums<T, S, DIAG, PD, 0, 1>(a, col * ncr + cc, latc, cc, scale, keep, proj, nrm, yb, yt);
-        }
-        __syncthreads();
-        if (w == 1) return;
-        if (valid) {
-#pragma unroll
-            for (int k = 1; k < 4; ++k)
+            for (int k = 1; k < 3; ++k)
 #pragma unroll
                 for (int j = 0; j < 3; ++j) {
-                    yb[k][j] += part[(k - 1) * 6 + j][lane];
-                    yt[k][j] += part[(k - 1) * 6 + 3 + j][lane];
+                    shared(k, j, 0) = yb[k][j];
+                    shared(k, j, 1) = yt[k][j];
                 }
+            __syncthreads();
+        } else {
+            stored_cell_sums<T, S, DIAG, PD, 1, 2>(a, col * ncr + cc, latc, cc, scale, keep, proj, nrm, yb, yt, [&] {
+                __syncthreads();
+#pragma unroll
+                for (int k = 1; k < 3; ++k)
+#pragma unroll
+                    for (int j = 0; j < 3; ++j) {
+                        yb[k][j] = shared(k, j, 0);
+                        yt[k][j] = shared(k, j, 1);
+                    }
+            });
         }
     }
     // radial merge (level c = bottom of cell c + top of cell c-1) and write-out
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
+    for (int k = 0; k < 4; ++k) {
+        if (SPLIT && (k == 0) != (split == 0)) continue;  // corner 0 has wedge 0 alone
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
             T up = __shfl_up(yt[k][j], 1, 64);
@@ -901,6 +907,7 @@ __global__ __launch_bounds__(SPLIT ? 128 : 256)
             if (valid) a.csum[(int64_t)(k * 3 + j) * ncell + col * ncr + c] = yb[k][j] + up;
             if (lane == toplane) a.ctop[(int64_t)(k * 3 + j) * ncol * nch + col * nch + h] = yt[k][j];
         }
+    }
 }
 
 // Node copy (d, X, Y, level): sum of its lateral quads' corner values, then on
