@@ -398,159 +398,39 @@ __device__ inline void eps_block_geo(const T* __restrict__ geo_w, T r0, T r1, do
     const double alpha = 1.0 / r_mid, beta = 1.0 / half_dr;
     const double kwJ = ksum / 6.0 * r_mid * r_mid * half_dr * (double)geo_w[9];
     double g[6][3];
+#pragma unroll
     for (int a = 0; a < 3; ++a) {
         const double a1 = alpha * (double)geo_w[a], a2 = alpha * (double)geo_w[3 + a], z = beta * (double)geo_w[6 + a];
         const double a0 = -(a1 + a2);
         g[0][a] = a0 - z; g[1][a] = a1 - z; g[2][a] = a2 - z;
         g[3][a] = a0 + z; g[4][a] = a1 + z; g[5][a] = a2 + z;
     }
+#pragma unroll
     for (int i = 0; i < 6; ++i)
+#pragma unroll
         for (int j = 0; j < 6; ++j) {
             const double gg = g[i][0] * g[j][0] + g[i][1] * g[j][1] + g[i][2] * g[j][2];
             A[i][j] = kwJ * ((p == q ? gg : 0.0) + g[i][p] * g[j][q] - (2.0 / 3.0) * g[i][q] * g[j][p]);
         }
 }
 
-// Galerkin matrices sum P^T A P over the 8 fine wedges of a coarse wedge.
+// Galerkin matrices sum P^T A P over the 8 fine wedges of a coarse wedge.  A thread
+// per (coarse cell, coarse wedge, component block q <= p): the fine block A_qp (from
+// the geometry, or read from the fine level's storage), its products with P and the
+// sum in registers (a whole wedge would not fit beside A).  Matrix-free fine operator:
+// bound by the products, stored one: by reading the fine matrices.
 //
-// Matrix-free fine operator: its wedge matrix is a sum of products of the six
-// shape gradients g_i,
-//   A_(i,q),(j,p) = kwJ [ delta_pq g_i.g_j + g_i[p] g_j[q] - 2/3 g_i[q] g_j[p] ],
-// and P acts on the nodes alone, so P^T A P is the same expression in the
-// projected gradients G_a = sum_i P_ia g_i: no 6x6 products.  Two threads per
-// (coarse cell, coarse wedge): HALF 0 the component blocks (0, p), the packed
-// entries [0, 93), HALF 1 the blocks (1, 1), (1, 2), (2, 2), the entries
-// [93, 171).  The sums stay in registers in FP64 (a whole wedge's 171 would need
-// accumulation registers and their moves) and are written once as 16-byte
-// vectors of the tile layout, a wave's 64 consecutive cells side by side.  The
-// weights are wave-uniform (scalar loads).
-// Lateral level 6 -> 5 (65 -> 33 radial nodes, 0.90 GB of FP64 matrices): 14.8 ms
-// with a thread per component block that formed A and both 6x6 products in local
-// arrays; 0.33 ms in this form (2.7 TB/s of writes).
-template <typename T, typename S, typename SF, int HALF>
-__device__ __forceinline__ void gca_geo_half(const GcaArgs<T, S, SF>& a, int64_t cell, int W)
-{
-    constexpr int LO = HALF ? 93 : 0, CNT = HALF ? PACKED - 93 : 93;
-    constexpr int Q0 = HALF ? 1 : 0, Q1 = HALF ? 3 : 1;  // block rows q of this half
-    const int R = (int)(cell % (a.nrc - 1));
-    int64_t lat = cell / (a.nrc - 1);
-    const int Y = (int)(lat % (a.nc - 1));
-    lat /= (a.nc - 1);
-    const int X = (int)(lat % (a.nc - 1));
-    const int d = (int)(lat / (a.nc - 1));
-    const int ncf = a.nf - 1, ncrf = a.nrf - 1;
-    const bool own = a.geometric || R == a.nrc - 2;
-    const double b_top = own ? 1.0 : 0.0, b_bot = own ? 0.0 : 1.0;
-    double out[CNT];
-#pragma unroll
-    for (int i = 0; i < CNT; ++i) out[i] = 0.0;
-#pragma unroll 1
-    for (int k = 0; k < 8; ++k) {
-        const GcaWedge f = GCA_LIST[W][k];
-        const int fx = 2 * X + f.sx, fy = 2 * Y + f.sy, fr = 2 * R + f.sr, w = f.w;
-        const int64_t fquad = ((int64_t)d * ncf + fx) * ncf + fy;
-        const double* gw = a.geo_f + (fquad * 2 + w) * GEO_STRIDE;
-        double ksum = 0.0;
-        if (a.eta_cell_f) {
-            ksum = 6.0 * (double)a.eta_cell_f[fquad * ncrf + fr];
-        } else {
-            // wedge w's lateral corners: (w, w), (1 - w, w), (w, 1 - w)
-            const int64_t l00 = ((int64_t)d * a.nf + fx + w) * a.nf + fy + w;
-            const int64_t l10 = l00 + (w ? -a.nf : a.nf), l01 = l00 + (w ? -1 : 1);
-            const T* e0 = a.eta_f + l00 * a.nrf + fr;
-            const T* e1 = a.eta_f + l10 * a.nrf + fr;
-            const T* e2 = a.eta_f + l01 * a.nrf + fr;
-            ksum = (double)e0[0] + (double)e1[0] + (double)e2[0] + (double)e0[1] + (double)e1[1] + (double)e2[1];
-        }
-        const double r0 = a.radii_f[fr], r1 = a.radii_f[fr + 1];
-        const double half_dr = 0.5 * (r1 - r0), r_mid = 0.5 * (r0 + r1);
-        const double alpha = 1.0 / r_mid, beta = 1.0 / half_dr;
-        const double kwJ = ksum / 6.0 * r_mid * r_mid * half_dr * gw[9];
-        double G[6][3];
-#pragma unroll
-        for (int l = 0; l < 3; ++l) {
-            const double a1 = alpha * gw[l], a2 = alpha * gw[3 + l], z = beta * gw[6 + l];
-            const double a0 = -(a1 + a2);
-            const double g[6] = {a0 - z, a1 - z, a2 - z, a0 + z, a1 + z, a2 + z};
-#pragma unroll
-            for (int c = 0; c < 6; ++c) {
-                double v = 0.0;
-#pragma unroll
-                for (int i = 0; i < 6; ++i) v += GCA_P.C[W][k][i][c] * g[i];
-                G[c][l] = v;
-            }
-#pragma unroll
-            for (int m = 0; m < 3; ++m) {
-                double v = 0.0;
-#pragma unroll
-                for (int i = 0; i < 3; ++i) v += GCA_P.B[W][k][i][m] * g[3 + i];
-                G[m][l] += b_bot * v;
-                G[m + 3][l] += b_top * v;
-            }
-        }
-        // component blocks (q, p): rows r = node + 6 q, columns node + 6 p
-#pragma unroll
-        for (int i = 0; i < 6; ++i) {
-            const double h[3] = {kwJ * G[i][0], kwJ * G[i][1], kwJ * G[i][2]};
-#pragma unroll
-            for (int j = 0; j < 6; ++j) {
-                if (j >= i) {
-                    const double gg = h[0] * G[j][0] + h[1] * G[j][1] + h[2] * G[j][2];
-#pragma unroll
-                    for (int q = Q0; q < Q1; ++q)
-                        out[pk(i + 6 * q, j + 6 * q) - LO] += gg + (1.0 / 3.0) * (h[q] * G[j][q]);
-                }
-#pragma unroll
-                for (int q = Q0; q < Q1; ++q)
-#pragma unroll
-                    for (int p = q + 1; p < 3; ++p)
-                        out[pk(i + 6 * q, j + 6 * p) - LO] += h[p] * G[j][q] - (2.0 / 3.0) * (h[q] * G[j][p]);
-            }
-        }
-    }
-    // vectors wholly inside the half as such, the shared one (entry 93 is no
-    // multiple of the vector length) by elements; the pad slot 171 is not read
-    constexpr int V = stored_vec<S>();
-    constexpr int VA = (LO + V - 1) / V, VB = (LO + CNT) / V;
-    S* base = a.stored_c + stored_at<S>(cell, W, 0);
-    VecOf<S>* o = reinterpret_cast<VecOf<S>*>(base);
-#pragma unroll
-    for (int v = VA; v < VB; ++v) {
-        VecOf<S> x;
-        x.x = (S)out[v * V - LO];
-        x.y = (S)out[v * V + 1 - LO];
-        if constexpr (V == 4) {
-            x.z = (S)out[v * V + 2 - LO];
-            x.w = (S)out[v * V + 3 - LO];
-        }
-        o[v * 64] = x;
-    }
-#pragma unroll
-    for (int e = LO; e < LO + CNT; ++e)
-        if (e < VA * V || e >= VB * V) base[(e / V) * 64 * V + e % V] = (S)out[e - LO];
-}
-
-// grid: 4 blocks per tile of 64 coarse cells (coarse wedge, half)
-template <typename T, typename S, typename SF>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_gca_geo(GcaArgs<T, S, SF> a)
-{
-    const int64_t ncc = 10LL * (a.nc - 1) * (a.nc - 1) * (a.nrc - 1);
-    const int W = (int)(blockIdx.x & 1), half = (int)((blockIdx.x >> 1) & 1);
-    const int64_t cell = (int64_t)(blockIdx.x >> 2) * 64 + threadIdx.x;
-    if (cell >= ncc) return;
-    if (half == 0)
-        gca_geo_half<T, S, SF, 0>(a, cell, W);
-    else
-        gca_geo_half<T, S, SF, 1>(a, cell, W);
-}
-
-// Fine operator with stored matrices: a thread per (coarse cell, coarse wedge,
-// component block q <= p) sums P^T A_qp P over the 8 fine wedges, the 6x6 block
-// and its sum in registers (a whole wedge would not fit beside A).  What binds is
-// reading the fine matrices.  Level 5 -> 4 (0.90 GB read): 2.52 ms with the
-// products in local arrays and P built per thread, 0.34 ms now.
-template <typename T, typename S, typename SF, int Q, int P>
-__device__ __forceinline__ void gca_stored_block(const GcaArgs<T, S, SF>& a, int64_t cell, int W)
+// The coarsest level's CG amplifies the last bits of its matrices into a solve's
+// eighth digit, so the order of the sums is fixed: (A P) by rows, P^T (A P) per fine
+// wedge from zero, then added to the fine wedges before it.  The weights are zero or
+// powers of two, so their products are exact.
+// A thread per block that held A and both products in local arrays, P built per
+// thread: lateral level 6 -> 5 (matrix-free, 65 -> 33 radial nodes, 0.90 GB of FP64
+// matrices written) 14.8 ms, 0.79 so; 5 -> 4 (0.90 GB read) 2.52 and 0.34 ms.  The
+// matrix-free build from the projected gradients (the same matrices, P^T A P never
+// formed) took 0.33 ms, but its sums are others: a two-level solve moved by 1e-7.
+template <typename T, typename S, typename SF, bool FINE_GEO, int Q, int P>
+__device__ __forceinline__ void gca_block(const GcaArgs<T, S, SF>& a, int64_t cell, int W)
 {
     const int R = (int)(cell % (a.nrc - 1));
     int64_t lat = cell / (a.nrc - 1);
@@ -569,24 +449,40 @@ __device__ __forceinline__ void gca_stored_block(const GcaArgs<T, S, SF>& a, int
 #pragma unroll 1
     for (int k = 0; k < 8; ++k) {
         const GcaWedge f = GCA_LIST[W][k];
-        const int64_t fcell =
-            (((int64_t)d * ncf + 2 * X + f.sx) * ncf + 2 * Y + f.sy) * ncrf + 2 * R + f.sr;
-        const SF* base = a.stored_f + stored_at<SF>(fcell, f.w, 0);
-        constexpr int V = stored_vec<SF>();
+        const int fx = 2 * X + f.sx, fy = 2 * Y + f.sy, fr = 2 * R + f.sr, w = f.w;
+        const int64_t fquad = ((int64_t)d * ncf + fx) * ncf + fy;
         double A[6][6];
-#pragma unroll
-        for (int i = 0; i < 6; ++i)
-#pragma unroll
-            for (int j = 0; j < 6; ++j) {
-                if (Q == P && j < i) continue;
-                const int e = pk(i + 6 * Q, j + 6 * P);
-                A[i][j] = (double)base[(e / V) * 64 * V + e % V];
+        if constexpr (FINE_GEO) {
+            double ksum = 0.0;
+            if (a.eta_cell_f) {
+                ksum = 6.0 * (double)a.eta_cell_f[fquad * ncrf + fr];
+            } else {
+                // wedge w's lateral corners: (w, w), (1 - w, w), (w, 1 - w)
+                const int64_t l00 = ((int64_t)d * a.nf + fx + w) * a.nf + fy + w;
+                const int64_t l10 = l00 + (w ? -a.nf : a.nf), l01 = l00 + (w ? -1 : 1);
+                const T* e0 = a.eta_f + l00 * a.nrf + fr;
+                const T* e1 = a.eta_f + l10 * a.nrf + fr;
+                const T* e2 = a.eta_f + l01 * a.nrf + fr;
+                ksum = (double)e0[0] + (double)e1[0] + (double)e2[0] + (double)e0[1] + (double)e1[1] + (double)e2[1];
             }
-        if constexpr (Q == P) {
+            eps_block_geo<double>(a.geo_f + (fquad * 2 + w) * GEO_STRIDE, a.radii_f[fr], a.radii_f[fr + 1], ksum, Q, P, A);
+        } else {
+            const SF* base = a.stored_f + stored_at<SF>(fquad * ncrf + fr, w, 0);
+            constexpr int V = stored_vec<SF>();
 #pragma unroll
-            for (int i = 1; i < 6; ++i)
+            for (int i = 0; i < 6; ++i)
 #pragma unroll
-                for (int j = 0; j < i; ++j) A[i][j] = A[j][i];
+                for (int j = 0; j < 6; ++j) {
+                    if (Q == P && j < i) continue;
+                    const int e = pk(i + 6 * Q, j + 6 * P);
+                    A[i][j] = (double)base[(e / V) * 64 * V + e % V];
+                }
+            if constexpr (Q == P) {
+#pragma unroll
+                for (int i = 1; i < 6; ++i)
+#pragma unroll
+                    for (int j = 0; j < i; ++j) A[i][j] = A[j][i];
+            }
         }
         // weights of the fine dofs 3..5 per lane (the bracket depends on the cell)
         double Pt[3][6];
@@ -610,10 +506,10 @@ __device__ __forceinline__ void gca_stored_block(const GcaArgs<T, S, SF>& a, int
 #pragma unroll
             for (int i = 0; i < 6; ++i) {
                 if (Q == P && j < i) continue;
-                double v = out[i][j];
+                double v = 0.0;
 #pragma unroll
                 for (int l = 0; l < 6; ++l) v += (l < 3 ? GCA_P.C[W][k][l < 3 ? l : 0][i] : Pt[l < 3 ? 0 : l - 3][i]) * t[l];
-                out[i][j] = v;
+                out[i][j] += v;
             }
         }
     }
@@ -630,20 +526,20 @@ __device__ __forceinline__ void gca_stored_block(const GcaArgs<T, S, SF>& a, int
 }
 
 // grid: 12 blocks per tile of 64 coarse cells (coarse wedge, component block)
-template <typename T, typename S, typename SF>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_gca_stored(GcaArgs<T, S, SF> a)
+template <typename T, typename S, typename SF, bool FINE_GEO>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_gca(GcaArgs<T, S, SF> a)
 {
     const int64_t ncc = 10LL * (a.nc - 1) * (a.nc - 1) * (a.nrc - 1);
     const int part = (int)(blockIdx.x % 12), W = part / 6;
     const int64_t cell = (int64_t)(blockIdx.x / 12) * 64 + threadIdx.x;
     if (cell >= ncc) return;
     switch (part % 6) {
-    case 0: gca_stored_block<T, S, SF, 0, 0>(a, cell, W); break;
-    case 1: gca_stored_block<T, S, SF, 0, 1>(a, cell, W); break;
-    case 2: gca_stored_block<T, S, SF, 0, 2>(a, cell, W); break;
-    case 3: gca_stored_block<T, S, SF, 1, 1>(a, cell, W); break;
-    case 4: gca_stored_block<T, S, SF, 1, 2>(a, cell, W); break;
-    default: gca_stored_block<T, S, SF, 2, 2>(a, cell, W); break;
+    case 0: gca_block<T, S, SF, FINE_GEO, 0, 0>(a, cell, W); break;
+    case 1: gca_block<T, S, SF, FINE_GEO, 0, 1>(a, cell, W); break;
+    case 2: gca_block<T, S, SF, FINE_GEO, 0, 2>(a, cell, W); break;
+    case 3: gca_block<T, S, SF, FINE_GEO, 1, 1>(a, cell, W); break;
+    case 4: gca_block<T, S, SF, FINE_GEO, 1, 2>(a, cell, W); break;
+    default: gca_block<T, S, SF, FINE_GEO, 2, 2>(a, cell, W); break;
     }
 }
 
@@ -1248,9 +1144,9 @@ void launch_gca_build(const GcaArgs<T, S, SF>& a, bool fine_geo, hipStream_t s)
     const int64_t tiles = (ncc + 63) / 64;
     TN_REQUIRE(12 * tiles < (1LL << 31), "GCA: mesh too large");
     if (fine_geo)
-        hipLaunchKernelGGL((k_gca_geo<T, S, SF>), dim3((unsigned)(4 * tiles)), dim3(64), 0, s, a);
+        hipLaunchKernelGGL((k_gca<T, S, SF, true>), dim3((unsigned)(12 * tiles)), dim3(64), 0, s, a);
     else
-        hipLaunchKernelGGL((k_gca_stored<T, S, SF>), dim3((unsigned)(12 * tiles)), dim3(64), 0, s, a);
+        hipLaunchKernelGGL((k_gca<T, S, SF, false>), dim3((unsigned)(12 * tiles)), dim3(64), 0, s, a);
     TN_HIP(hipGetLastError());
 }
 
