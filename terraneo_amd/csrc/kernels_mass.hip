@@ -1,6 +1,7 @@
 // Mass operators on wedges: VectorMass (vector_mass.hpp:83-153), lumped KMass
 // (kmass.hpp:97-185).
 #include <algorithm>
+#include <type_traits>
 
 #include "tn_eps_march.hpp"
 #include "tn_internal.hpp"
@@ -11,13 +12,9 @@
 namespace tn {
 namespace {
 
-// VectorMass and the lumped k-mass (kmass.hpp) as a gather.  The lumped k-mass is
-// the row sum of the k-weighted matrix: with sum_j N_j = 1 its entry is
-// sum_q w_q k_h(q) N_i(q) |det|, the consistent mass matrix applied to the nodal
-// k by the same rule, so both are this kernel (the Schur diagonal of 0.36 M
-// pressure nodes took 426 us as quadrature per node and wedge, under 10 us here).
-// Every node copy is written once, y_i = sum over the wedges of its diamond that
-// contain it of (M_w x)_i; no atomics, so the result repeats bit for bit.  The
+// VectorMass as a gather: every node copy is written once, y_i = sum over the wedges
+// of its diamond that contain it of (M_w x)_i; no atomics, so the result repeats bit
+// for bit.  The
 // reference's Felippa 3x2 rule factors into the 3-point triangle rule, exact for
 // the lateral products (the P1 triangle mass (1 + delta_ij) / 24 times
 // |det(V0, V1, V2)|), and the 2-point Gauss rule in zeta for rho^2 hat_a hat_b,
@@ -84,7 +81,7 @@ __global__ __launch_bounds__(256) void k_mass_stencil(MassArgs<T> a)
     for (int c = 0; c < a.ncomp; ++c) a.y[c * N + t] = (T)acc[c];
 }
 
-// One component (the projection's CG, the Schur diagonal): a wave walks an even
+// One component (the projection's CG): a wave walks an even
 // run of consecutive radial columns, its lanes on 64 levels.  The radial weights
 // stay in registers for the whole run, the lateral ones are wave-uniform, and the
 // next column is loaded while one is summed.  A lane loads its own level and takes
@@ -198,6 +195,98 @@ __global__ __launch_bounds__(64 * MASS_WAVES) void k_mass_columns(MassArgs<T> a)
     if (a.dot) block_partial(sum, a.dot);
 }
 
+// Lumped k-weighted mass: row sums of the k-weighted wedge mass matrices in the
+// reference's 6-point quadrature, a thread per node copy that adds the rows of the
+// wedges of its diamond that contain it, in a fixed order.  In exact arithmetic this
+// is the mass product above with the nodal k (sum_j N_j = 1), but it is the Schur
+// diagonal of the solves, whose coarsest-level CG amplifies its last bits, so the
+// quadrature's own sums are kept.  0.36 M pressure nodes: 426 us with the whole 6x6
+// matrix per row in local arrays, 37 us with the row alone, its index a constant.
+__device__ constexpr double Q6P[6][3] = {{0.6666666666666666, 0.1666666666666667, -0.5773502691896257},
+                                        {0.1666666666666667, 0.6666666666666666, -0.5773502691896257},
+                                        {0.1666666666666667, 0.1666666666666667, -0.5773502691896257},
+                                        {0.6666666666666666, 0.1666666666666667, 0.5773502691896257},
+                                        {0.1666666666666667, 0.6666666666666666, 0.5773502691896257},
+                                        {0.1666666666666667, 0.1666666666666667, 0.5773502691896257}};
+__device__ constexpr double Q6W = 0.1666666666666667;
+
+__device__ constexpr double shape6(int q, int j)
+{
+    const double lat = j % 3 == 0 ? 1.0 - Q6P[q][0] - Q6P[q][1] : (j % 3 == 1 ? Q6P[q][0] : Q6P[q][1]);
+    return lat * (j < 3 ? 0.5 * (1 - Q6P[q][2]) : 0.5 * (1 + Q6P[q][2]));
+}
+
+// row ROW of wedge W of quad (qx, qy), layer rc
+template <typename T, int W, int ROW>
+__device__ __forceinline__ double kmass_row(const double* __restrict__ coords, const double* __restrict__ radii,
+                                            const T* __restrict__ k, int n, int nr, int d, int qx, int qy, int rc)
+{
+    constexpr int OFF[2][3][2] = {{{0, 0}, {1, 0}, {0, 1}}, {{1, 1}, {0, 1}, {1, 0}}};
+    double P[3][3], kv[6];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        const int64_t lat = ((int64_t)d * n + qx + OFF[W][i][0]) * n + qy + OFF[W][i][1];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) P[i][c] = coords[3 * lat + c];
+        kv[i] = (double)k[lat * nr + rc];
+        kv[i + 3] = (double)k[lat * nr + rc + 1];
+    }
+    const double r1 = radii[rc], r2 = radii[rc + 1], gr = 0.5 * (r2 - r1);
+    double M[6] = {0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int q = 0; q < 6; ++q) {
+        double J[3][3];  // lateral Jacobian (kernel_helpers.hpp:153-176)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            J[c][0] = P[1][c] - P[0][c];
+            J[c][1] = P[2][c] - P[0][c];
+            J[c][2] = (1 - Q6P[q][0] - Q6P[q][1]) * P[0][c] + Q6P[q][0] * P[1][c] + Q6P[q][1] * P[2][c];
+        }
+        const double det = fabs(J[0][0] * (J[1][1] * J[2][2] - J[1][2] * J[2][1]) -
+                                J[0][1] * (J[1][0] * J[2][2] - J[1][2] * J[2][0]) +
+                                J[0][2] * (J[1][0] * J[2][1] - J[1][1] * J[2][0]));
+        const double rr = r1 + 0.5 * (r2 - r1) * (1 + Q6P[q][2]);
+        double kq = 0.0;
+#pragma unroll
+        for (int j = 0; j < 6; ++j) kq += shape6(q, j) * kv[j];
+        const double f = Q6W * kq * rr * rr * gr * det;
+#pragma unroll
+        for (int j = 0; j < 6; ++j) M[j] += f * shape6(q, ROW) * shape6(q, j);
+    }
+    double s = 0.0;
+#pragma unroll
+    for (int j = 0; j < 6; ++j) s += M[j];
+    return s;
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void k_kmass_lumped(const double* __restrict__ coords, const double* __restrict__ radii,
+                                                      const T* __restrict__ k, T* __restrict__ out, int n, int nr)
+{
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= 10LL * n * n * nr) return;
+    const int lat = (int)(t / nr), lev = (int)(t - (int64_t)lat * nr);
+    const int Y = lat % n, X = (lat / n) % n, d = lat / (n * n), nc = n - 1;
+    double acc = 0.0;
+    // the six wedges around (X, Y) of layer rc: (X-1, Y-1) w1; (X-1, Y) w0, w1; (X, Y-1) w0, w1; (X, Y) w0
+    auto layer = [&](int rc, auto top) {
+        constexpr int B = decltype(top)::value ? 3 : 0;
+        if (X > 0 && Y > 0) acc += kmass_row<T, 1, B>(coords, radii, k, n, nr, d, X - 1, Y - 1, rc);
+        if (X > 0 && Y < nc) {
+            acc += kmass_row<T, 0, B + 1>(coords, radii, k, n, nr, d, X - 1, Y, rc);
+            acc += kmass_row<T, 1, B + 2>(coords, radii, k, n, nr, d, X - 1, Y, rc);
+        }
+        if (X < nc && Y > 0) {
+            acc += kmass_row<T, 0, B + 2>(coords, radii, k, n, nr, d, X, Y - 1, rc);
+            acc += kmass_row<T, 1, B + 1>(coords, radii, k, n, nr, d, X, Y - 1, rc);
+        }
+        if (X < nc && Y < nc) acc += kmass_row<T, 0, B>(coords, radii, k, n, nr, d, X, Y, rc);
+    };
+    if (lev > 0) layer(lev - 1, std::true_type{});
+    if (lev < nr - 1) layer(lev, std::false_type{});
+    out[t] = (T)acc;
+}
+
 }  // namespace
 
 int mass_blocks(int n)
@@ -220,6 +309,17 @@ void launch_mass(const MassArgs<T>& a, hipStream_t s)
         hipLaunchKernelGGL((k_mass_columns<T>), dim3((unsigned)mass_blocks(a.n)), dim3(64 * MASS_WAVES), 0, s, a);
     TN_HIP(hipGetLastError());
 }
+
+template <typename T>
+void launch_kmass_lumped(const double* coords, const double* radii, int n, int nr, const T* k, T* out, hipStream_t s)
+{
+    const int64_t N = 10LL * n * n * nr;
+    hipLaunchKernelGGL((k_kmass_lumped<T>), dim3((unsigned)((N + 255) / 256)), dim3(256), 0, s, coords, radii, k, out, n,
+                       nr);
+    TN_HIP(hipGetLastError());
+}
+template void launch_kmass_lumped<double>(const double*, const double*, int, int, const double*, double*, hipStream_t);
+template void launch_kmass_lumped<float>(const double*, const double*, int, int, const float*, float*, hipStream_t);
 
 template void launch_mass<double>(const MassArgs<double>&, hipStream_t);
 template void launch_mass<float>(const MassArgs<float>&, hipStream_t);

@@ -248,8 +248,7 @@ int tn_kmass_lumped(const tn_mesh* m, int dtype, const void* k, void* d, tn_stre
     auto& L = const_cast<tn_mesh*>(m)->lvl.dev();
     auto go = [&](auto* dd) {
         using T = std::remove_pointer_t<decltype(dd)>;
-        tn::MassArgs<T> a{L.d_radii.p, L.n, L.nr, 1, (const T*)k, dd, L.d_geo.p};
-        tn::launch_mass<T>(a, (hipStream_t)s);
+        tn::launch_kmass_lumped<T>(L.d_coords.p, L.d_radii.p, L.n, L.nr, (const T*)k, dd, (hipStream_t)s);
         tn::launch_interface_sum<T>(L, 1, dd, (hipStream_t)s);
     };
     if (dtype == TN_F64)

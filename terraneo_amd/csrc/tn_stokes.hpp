@@ -44,7 +44,7 @@ template <typename T>
 struct MassArgs {
     const double* radii;
     int n, nr, ncomp;
-    const T* x;         // input field (lumped k-mass: the coefficient)
+    const T* x;         // input field
     T* y;               // output, every node copy written (before the interface sum)
     const double* geo;  // the mesh's wedge table [10][n-1][n-1][2][GEO_STRIDE]
     double* dot = nullptr;  // optional: mass_blocks(n) partial sums of x . y over all node copies
@@ -57,5 +57,8 @@ template <typename T>
 void launch_grad(const GradArgs<T>& a, hipStream_t s);
 template <typename T>
 void launch_mass(const MassArgs<T>& a, hipStream_t s);
+// lumped k-weighted mass of the nodal field k, every node copy written (before the interface sum)
+template <typename T>
+void launch_kmass_lumped(const double* coords, const double* radii, int n, int nr, const T* k, T* out, hipStream_t s);
 
 }  // namespace tn
