@@ -476,7 +476,8 @@ void PCG::solve_queued(Ctx& c, LinOp& A, const BVec& x, const BVec& b)
     if (r0 < p_.atol || p_.max_iterations < 1) return;
     CgState st{};
     st.npap = A.dot_blocks(x);
-    st.nrr = cg_update_blocks(*f.m, f.ncomp);
+    // with a whole A p the blocks, and so the order of the sums, of the host-side dots
+    st.nrr = A.dot_partial() ? cg_update_blocks(*f.m, f.ncomp) : reduce_blocks(*f.m, f.ncomp);
     const size_t words = (size_t)CgState::RING + 3 + st.npap + st.nrr;
     if (scalars_.n != words) scalars_.alloc(words);
     st.ctl = scalars_.p;

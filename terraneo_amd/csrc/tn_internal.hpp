@@ -172,7 +172,8 @@ struct CgState {
     const int32_t *groups = nullptr, *group_of = nullptr;
     __host__ __device__ static int slot(int it) { return it == 0 ? RING : (it - 1) % RING; }
 };
-int cg_update_blocks(const MeshLevel& m, int ncomp);  // = CgState::nrr
+// CgState::nrr where the update also adds a node's copies up
+int cg_update_blocks(const MeshLevel& m, int ncomp);
 void launch_cg_begin(const CgState& st, const double* rr0, hipStream_t s);
 // iteration it after ap = A p and its partials: x, r, then p and the stopping test
 template <typename T>
