@@ -7,7 +7,7 @@
 
 namespace tn {
 
-constexpr int COARSE_CG_NODES = 2048;   // node copies, 4 per thread
+constexpr int COARSE_CG_NODES = 2048;   // node copies, columns padded to a power of two of lanes: 4 per thread
 constexpr int COARSE_CG_LDS = 155 * 1024;  // of 160 KB
 
 template <typename T, typename S>
@@ -21,10 +21,11 @@ struct CoarseCgArgs {
     int zero;                  // 1: start from x = 0
     int max_iterations;
     double rtol, atol;
+    int lanes_log2 = 0;        // lanes of a column (set by the launcher)
 };
 // whether an n x n x nr operator with elements of esize bytes fits
 bool coarse_cg_fits(int n, int nr, int esize);
 template <typename T, typename S>
-void launch_coarse_cg(const CoarseCgArgs<T, S>& g, hipStream_t s);
+void launch_coarse_cg(CoarseCgArgs<T, S> g, hipStream_t s);
 
 }  // namespace tn
