@@ -117,7 +117,7 @@ struct StokesOp : LinOp {
     explicit StokesOp(tn_stokes* k) : K(k) {}
     void apply(Ctx& c, const BVec& x, const BVec& y) override
     {
-        stokes_apply(K, x.b[0].p, x.b[1].p, y.b[0].p, y.b[1].p, c.s);
+        stokes_apply(K, x.b[0].p, x.b[1].p, y.b[0].p, y.b[1].p, Coupling::solver, c.s);
     }
 };
 
@@ -429,9 +429,9 @@ int tn_stokes_solve(tn_stokes* K, int method, tn_gmg* prec_u, const void* schur_
             void apply(Ctx& c, const BVec& x, const BVec& y) override
             {
                 if (K->A->dtype == TN_F64)
-                    grad_t<double>(K, x.b[0].p, y.b[0].p, false, true, c.s);
+                    grad_t<double>(K, x.b[0].p, y.b[0].p, false, true, Coupling::solver, c.s);
                 else
-                    grad_t<float>(K, x.b[0].p, y.b[0].p, false, true, c.s);
+                    grad_t<float>(K, x.b[0].p, y.b[0].p, false, true, Coupling::solver, c.s);
             }
         } bt;
         bt.K = K;

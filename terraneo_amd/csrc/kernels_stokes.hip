@@ -1,5 +1,7 @@
 // Stokes coupling: B (Divergence, divergence.hpp:117-323), p_c += -int div(u_h) q_H,
-// and its transpose B^T (Gradient, gradient.hpp:115-325), u += -int p_H div(v_h).
+// and its transpose B^T (Gradient, gradient.hpp:115-325), u += -int p_H div(v_h): the
+// products that a program asks for.  The solves keep the form by cells, whose roundings
+// their results rest on (kernels_coupling_cells.hip).
 //
 // Velocity lives on the fine mesh, pressure on the mesh one level coarser; each
 // fine wedge integrates with the 6-point Felippa 3x2 rule and the coarse shape
@@ -52,50 +54,13 @@
 #include <type_traits>
 
 #include "tn_cell.hpp"
+#include "tn_coupling.hpp"
 #include "tn_eps_march.hpp"
 #include "tn_march.hpp"
 #include "tn_stokes.hpp"
 
 namespace tn {
 namespace {
-
-__device__ constexpr double GAUSS2 = 0.57735026918962576451;  // 1/sqrt(3)
-
-// coarse lateral shape il on fine lateral wedge flw: alpha + beta xi + gamma eta
-// (integrands.hpp:103-190; flw from kernel_helpers.hpp:600-608)
-__host__ __device__ constexpr double coarse_lat_coef(int flw, int il, int k)
-{
-    constexpr double C[4][3][3] = {{{1.0, -0.5, -0.5}, {0.0, 0.5, 0.0}, {0.0, 0.0, 0.5}},
-                                   {{0.5, -0.5, -0.5}, {0.5, 0.5, 0.0}, {0.0, 0.0, 0.5}},
-                                   {{0.5, -0.5, -0.5}, {0.0, 0.5, 0.0}, {0.5, 0.0, 0.5}},
-                                   {{0.0, 0.5, 0.5}, {0.5, -0.5, 0.0}, {0.5, 0.0, -0.5}}};
-    return C[flw][il][k];
-}
-
-// int over the reference triangle of (alpha + beta xi + gamma eta) * {1, xi, eta}
-struct LatMoments {
-    double m[4][3][3];  // [flw][il][M0, Mx, Me]
-};
-__host__ __device__ constexpr LatMoments make_lat_moments()
-{
-    LatMoments r{};
-    for (int f = 0; f < 4; ++f)
-        for (int i = 0; i < 3; ++i) {
-            const double al = coarse_lat_coef(f, i, 0), be = coarse_lat_coef(f, i, 1), ga = coarse_lat_coef(f, i, 2);
-            r.m[f][i][0] = al / 2 + (be + ga) / 6;
-            r.m[f][i][1] = al / 6 + be / 12 + ga / 24;
-            r.m[f][i][2] = al / 6 + be / 24 + ga / 12;
-        }
-    return r;
-}
-__device__ constexpr LatMoments LATM = make_lat_moments();
-
-__device__ inline int fine_lateral_wedge_idx(int xp, int yp, int w)
-{
-    // kernel_helpers.hpp:600-608 (xp, yp: parities of the fine quad indices)
-    constexpr int ind[2][2][2] = {{{0, 1}, {2, 3}}, {{3, 2}, {1, 0}}};
-    return ind[w][yp][xp];
-}
 
 // Table slot of coarse column offset (dx, dy) from (x >> 1, y >> 1) for a fine
 // column of parities (xo, yo); the offsets in reach:

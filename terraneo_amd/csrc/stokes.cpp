@@ -45,31 +45,46 @@ const T* coupling_rad(const tn_stokes* K)
 }
 
 template <typename T>
-void div_t(tn_stokes* K, const void* u, void* p, hipStream_t s)
+void div_t(tn_stokes* K, const void* u, void* p, Coupling form, hipStream_t s)
 {
     auto& mf = const_cast<tn_mesh*>(K->vel)->lvl.dev();
     auto& mc = const_cast<tn_mesh*>(K->pre)->lvl.dev();
-    DivArgs<T> a{(const T*)K->coupling.p, coupling_rad<T>(K), mf.n, mf.nr, mc.n, mc.nr,
-                 K->A->bc_cmb, K->A->bc_surf, (const T*)u, (T*)p};
-    launch_div<T>(a, s);
+    if (form == Coupling::solver) {
+        TN_REQUIRE(K->div_tmp.n == sizeof(T) * (size_t)div_scratch_elems(mc.n, mc.nr), "B: scratch not allocated");
+        DivCellArgs<T> a{mf.d_coords.p, mf.d_radii.p, mf.n, mf.nr, mc.n, mc.nr,
+                         K->A->bc_cmb, K->A->bc_surf, (const T*)u, (T*)p, (T*)K->div_tmp.p};
+        launch_div_cells<T>(a, s);
+    } else {
+        DivArgs<T> a{(const T*)K->coupling.p, coupling_rad<T>(K), mf.n, mf.nr, mc.n, mc.nr,
+                     K->A->bc_cmb, K->A->bc_surf, (const T*)u, (T*)p};
+        launch_div<T>(a, s);
+    }
     launch_interface_sum<T>(mc, 1, (T*)p, s);
 }
 
 template <typename T>
-void grad_t(tn_stokes* K, const void* p, void* u, bool add, bool comm, hipStream_t s)
+void grad_t(tn_stokes* K, const void* p, void* u, bool add, bool comm, Coupling form, hipStream_t s)
 {
     auto& mf = const_cast<tn_mesh*>(K->vel)->lvl.dev();
     auto& mc = const_cast<tn_mesh*>(K->pre)->lvl.dev();
-    GradArgs<T> a{(const T*)K->coupling.p, coupling_rad<T>(K), mf.n, mf.nr, mc.n, mc.nr,
-                  K->A->bc_cmb, K->A->bc_surf, (const T*)p, (T*)u, add ? 1 : 0};
-    launch_grad<T>(a, s);
+    if (form == Coupling::solver) {
+        constexpr int W = grad_march_waves<T>();
+        const int seg = march_seg_for(mf.n, W - 1, sizeof(T) == 8 ? W : 2 * W);
+        GradCellArgs<T> a{mf.d_coords.p, mf.d_radii.p, mf.n, mf.nr, mc.n, mc.nr, K->A->bc_cmb,
+                          K->A->bc_surf, (const T*)p, (T*)u, seg, add ? 1 : 0, march_guard()};
+        launch_grad_cells<T>(a, s);
+    } else {
+        GradArgs<T> a{(const T*)K->coupling.p, coupling_rad<T>(K), mf.n, mf.nr, mc.n, mc.nr,
+                      K->A->bc_cmb, K->A->bc_surf, (const T*)p, (T*)u, add ? 1 : 0};
+        launch_grad<T>(a, s);
+    }
     if (comm) launch_interface_sum<T>(mf, 3, (T*)u, s);
 }
 
 // EpsDivDivStokes::apply_impl (epsilon_divdiv_stokes.hpp:55-84):
 // A in Replace + skipped communication, B^T in Add + additive communication
 // (which also completes A's partial sums), B in Replace + communication.
-void stokes_apply(tn_stokes* K, const void* u, const void* p, void* yu, void* yp, hipStream_t s)
+void stokes_apply(tn_stokes* K, const void* u, const void* p, void* yu, void* yp, Coupling form, hipStream_t s)
 {
     tn_eps* A = K->A;
     const int am = A->apply_mode, cm = A->comm_mode;
@@ -89,16 +104,16 @@ void stokes_apply(tn_stokes* K, const void* u, const void* p, void* yu, void* yp
     A->comm_mode = cm;
     A->diagonal = dg;
     if (A->dtype == TN_F64) {
-        grad_t<double>(K, p, yu, true, true, s);
-        div_t<double>(K, u, yp, s);
+        grad_t<double>(K, p, yu, true, true, form, s);
+        div_t<double>(K, u, yp, form, s);
     } else {
-        grad_t<float>(K, p, yu, true, true, s);
-        div_t<float>(K, u, yp, s);
+        grad_t<float>(K, p, yu, true, true, form, s);
+        div_t<float>(K, u, yp, form, s);
     }
 }
 
-template void grad_t<double>(tn_stokes*, const void*, void*, bool, bool, hipStream_t);
-template void grad_t<float>(tn_stokes*, const void*, void*, bool, bool, hipStream_t);
+template void grad_t<double>(tn_stokes*, const void*, void*, bool, bool, Coupling, hipStream_t);
+template void grad_t<float>(tn_stokes*, const void*, void*, bool, bool, Coupling, hipStream_t);
 
 }  // namespace tn
 
@@ -175,6 +190,9 @@ int tn_stokes_create(const tn_mesh* vel, const tn_mesh* pre, tn_eps* A, tn_stoke
     K->vel = vel;
     K->pre = pre;
     K->A = A;
+    // the scratch of B in the solves (per-cell corner sums)
+    const size_t esize = A->dtype == TN_F64 ? sizeof(double) : sizeof(float);
+    K->div_tmp.alloc(esize * (size_t)tn::div_scratch_elems(pre->lvl.n, pre->lvl.nr));
     if (A->dtype == TN_F64)
         tn::coupling_build<double>(K.get());
     else
@@ -195,7 +213,7 @@ int tn_stokes_apply(tn_stokes* K, const void* u, const void* p, void* yu, void* 
     TN_API_BEGIN
     TN_REQUIRE(K && u && p && yu && yp, "null pointer");
     tn::check_march_status();
-    tn::stokes_apply(K, u, p, yu, yp, (hipStream_t)s);
+    tn::stokes_apply(K, u, p, yu, yp, tn::Coupling::product, (hipStream_t)s);
     TN_API_END
 }
 
@@ -204,9 +222,9 @@ int tn_div_apply(tn_stokes* K, const void* u, void* p, tn_stream_t s)
     TN_API_BEGIN
     TN_REQUIRE(K && u && p, "null pointer");
     if (K->A->dtype == TN_F64)
-        tn::div_t<double>(K, u, p, (hipStream_t)s);
+        tn::div_t<double>(K, u, p, tn::Coupling::product, (hipStream_t)s);
     else
-        tn::div_t<float>(K, u, p, (hipStream_t)s);
+        tn::div_t<float>(K, u, p, tn::Coupling::product, (hipStream_t)s);
     TN_API_END
 }
 
@@ -217,9 +235,9 @@ int tn_grad_apply(tn_stokes* K, const void* p, void* u, int apply_mode, int comm
     tn::check_march_status();
     const bool add = apply_mode == TN_ADD, comm = comm_mode == TN_COMM_ADDITIVE;
     if (K->A->dtype == TN_F64)
-        tn::grad_t<double>(K, p, u, add, comm, (hipStream_t)s);
+        tn::grad_t<double>(K, p, u, add, comm, tn::Coupling::product, (hipStream_t)s);
     else
-        tn::grad_t<float>(K, p, u, add, comm, (hipStream_t)s);
+        tn::grad_t<float>(K, p, u, add, comm, tn::Coupling::product, (hipStream_t)s);
     TN_API_END
 }
 

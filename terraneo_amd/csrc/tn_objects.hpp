@@ -42,13 +42,17 @@ struct tn_stokes {
     const tn_mesh* pre = nullptr;
     tn_eps* A = nullptr;  // viscous block on the velocity mesh; its BCs govern B and B^T
     tn::DevBuf<unsigned char> rhs_tmp;  // nodal buoyancy before the mass matrix (tn_stokes_rhs_from_temperature)
+    tn::DevBuf<unsigned char> div_tmp;  // B's per-cell corner sums in the solves (div_scratch_elems)
     tn::DevBuf<unsigned char> coupling;  // tables of B and B^T (kernels_stokes.hip), in A's type
 };
 
 namespace tn {
-void stokes_apply(tn_stokes* K, const void* u, const void* p, void* yu, void* yp, hipStream_t s);
+// B and B^T: the column stencils for a single product, the cell form for the solves,
+// whose results it fixes (kernels_coupling_cells.hip)
+enum class Coupling { product, solver };
+void stokes_apply(tn_stokes* K, const void* u, const void* p, void* yu, void* yp, Coupling form, hipStream_t s);
 template <typename T>
-void grad_t(tn_stokes* K, const void* p, void* u, bool add, bool comm, hipStream_t s);
+void grad_t(tn_stokes* K, const void* p, void* u, bool add, bool comm, Coupling form, hipStream_t s);
 // C++ entry used by the Stokes and solver layers
 void eps_apply(tn_eps* op, const void* src, void* dst, hipStream_t s);
 // unpreconditioned CG on op in one launch where op is stored and small
