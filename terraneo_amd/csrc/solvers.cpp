@@ -457,13 +457,16 @@ struct Event {
 };
 }  // namespace
 
-// The recurrence of solve() with z = r, so that (z, r) is (r, r).  The queue is fed in batches of BATCH iterations; a batch's
-// (r, r) values come back behind it and are read while the next one runs, so a
-// solve that has converged runs at most two batches of kernels that return at once.
+// The recurrence of solve() with z = r, so that (z, r) is (r, r).  The queue is fed in
+// batches of up to BATCH iterations; a batch's residuals come back behind it and are
+// read while the next one runs.  An iteration queued behind the one that meets the
+// stopping test leaves the vectors alone, but its product runs in full, so no more is
+// queued than half the iterations that the residuals' decay still asks for: one at
+// first and near the end, two batches in between.
 void PCG::solve_queued(Ctx& c, LinOp& A, const BVec& x, const BVec& b)
 {
     constexpr int BATCH = 8;
-    static_assert(CgState::RING % BATCH == 0 && CgState::RING >= 4 * BATCH, "ring of residuals");
+    static_assert(CgState::RING >= 2 * BATCH, "ring of residuals");
     BVec &r = t_[0], &pp = t_[1], &ap = t_[2];
     const Field& f = x.b[0];
     info = IterInfo{};
@@ -478,11 +481,11 @@ void PCG::solve_queued(Ctx& c, LinOp& A, const BVec& x, const BVec& b)
     st.npap = A.dot_blocks(x);
     // with a whole A p the blocks, and so the order of the sums, of the host-side dots
     st.nrr = A.dot_partial() ? cg_update_blocks(*f.m, f.ncomp) : reduce_blocks(*f.m, f.ncomp);
-    const size_t words = (size_t)CgState::RING + 3 + st.npap + st.nrr;
+    const size_t words = (size_t)CgState::WORDS + st.npap + st.nrr;
     if (scalars_.n != words) scalars_.alloc(words);
     st.ctl = scalars_.p;
-    st.rr = scalars_.p + 2;
-    st.part_pap = st.rr + CgState::RING + 1;
+    st.rr = scalars_.p + CgState::RR;
+    st.part_pap = scalars_.p + CgState::WORDS;
     st.part_rr = st.part_pap + st.npap;
     if (A.dot_partial()) {
         st.groups = f.m->d_grp_pad.p;
@@ -491,46 +494,64 @@ void PCG::solve_queued(Ctx& c, LinOp& A, const BVec& x, const BVec& b)
     st.rtol = p_.rtol;
     st.atol = p_.atol;
     launch_cg_begin(st, c.red.p, c.s);
-    HostPage page;  // per batch in flight: BATCH residuals and the control word
-    Event ev[2];
-    auto host = [&](int k) { return page.p + (k & 1) * (BATCH + 1); };
-    auto drain = [&](int k) {  // true: converged within batch k
-        TN_HIP(hipEventSynchronize(ev[k & 1].e));
+    // the scalars as they are behind a batch, one copy per batch in flight
+    static_assert(2 * CgState::WORDS * sizeof(double) <= HOST_PAGE_BYTES, "two batches' scalars");
+    HostPage page;
+    struct Batch {
+        Event ev;
+        int end = 0;
+    } flight[2];
+    int queued = 0, seen = 0, first = 0, last = 0;  // iterations; batches [first, last) in flight
+    auto host = [&](int k) { return page.p + (k & 1) * CgState::WORDS; };
+    // iterations worth queueing beyond those seen
+    auto look_ahead = [&] {
+        if (seen == 0) return 1;
+        const double target = std::max(p_.rtol * r0, p_.atol), res = info.final_residual;
+        const int w = std::min(seen, BATCH);
+        const double decay = std::max(std::log(r0 / res) / seen, std::log(info.history[seen - w] / res) / w);
+        double left = decay > 0.0 ? std::log(res / target) / decay : 4.0 * BATCH;
+        if (!(left < 4.0 * BATCH)) left = 4.0 * BATCH;  // (also no target, or no number)
+        return std::max(1, (int)(0.5 * left));
+    };
+    auto drain = [&] {  // true: converged within the oldest batch in flight
+        Batch& bt = flight[first & 1];
+        TN_HIP(hipEventSynchronize(bt.ev.e));
         check_march_status();
-        const double* h = host(k);
-        const int done = (int)h[BATCH];
-        for (int it = k * BATCH + 1; it <= std::min((k + 1) * BATCH, p_.max_iterations); ++it) {
-            if (done && it > done) break;
-            const double res = std::sqrt(h[it - k * BATCH - 1]);
-            info.iterations = it;
+        const double* h = host(first++);
+        const int done = (int)h[CgState::DONE];
+        while (seen < bt.end && !(done && seen >= done)) {
+            const double res = std::sqrt(h[CgState::RR + CgState::slot(++seen)]);
+            info.iterations = seen;
             info.final_residual = res;
             info.history.push_back(res);
         }
-        return done && done <= (k + 1) * BATCH;
+        return done && done <= bt.end;
     };
-    const int batches = (p_.max_iterations + BATCH - 1) / BATCH;
     try {
-        for (int k = 0; k < batches; ++k) {
-            for (int it = k * BATCH + 1; it <= std::min((k + 1) * BATCH, p_.max_iterations); ++it) {
-                A.apply_dot(c, pp, ap, st.part_pap);
-                if (f.dtype == TN_F64)
-                    launch_cg_step<double>(*f.m, f.ncomp, (double*)f.p, (double*)r.b[0].p, (double*)pp.b[0].p,
-                                           (const double*)ap.b[0].p, st, it, c.s);
-                else
-                    launch_cg_step<float>(*f.m, f.ncomp, (float*)f.p, (float*)r.b[0].p, (float*)pp.b[0].p,
-                                          (const float*)ap.b[0].p, st, it, c.s);
+        while (seen < p_.max_iterations) {
+            const int n = std::min({BATCH, p_.max_iterations - queued, seen + look_ahead() - queued});
+            if (n > 0 && last - first < 2) {
+                for (int it = queued + 1; it <= queued + n; ++it) {
+                    A.apply_dot(c, pp, ap, st.part_pap);
+                    if (f.dtype == TN_F64)
+                        launch_cg_step<double>(*f.m, f.ncomp, (double*)f.p, (double*)r.b[0].p, (double*)pp.b[0].p,
+                                               (const double*)ap.b[0].p, st, it, c.s);
+                    else
+                        launch_cg_step<float>(*f.m, f.ncomp, (float*)f.p, (float*)r.b[0].p, (float*)pp.b[0].p,
+                                              (const float*)ap.b[0].p, st, it, c.s);
+                }
+                queued += n;
+                TN_HIP(hipMemcpyAsync(host(last), st.ctl, CgState::WORDS * sizeof(double), hipMemcpyDeviceToHost, c.s));
+                TN_HIP(hipEventRecord(flight[last & 1].ev.e, c.s));
+                flight[last++ & 1].end = queued;
+                continue;
             }
-            TN_HIP(hipMemcpyAsync(host(k), st.rr + CgState::slot(k * BATCH + 1), BATCH * sizeof(double),
-                                  hipMemcpyDeviceToHost, c.s));
-            TN_HIP(hipMemcpyAsync(host(k) + BATCH, st.ctl + CgState::DONE, sizeof(double), hipMemcpyDeviceToHost, c.s));
-            TN_HIP(hipEventRecord(ev[k & 1].e, c.s));
-            if (k > 0 && drain(k - 1)) {
-                // the batch behind returns at once; its copies still write the page
-                TN_HIP(hipEventSynchronize(ev[k & 1].e));
+            if (drain()) {
+                // (the copy of the batch behind still writes the page)
+                if (first < last) TN_HIP(hipEventSynchronize(flight[first & 1].ev.e));
                 return;
             }
         }
-        drain(batches - 1);
     } catch (...) {
         (void)hipStreamSynchronize(c.s);  // the page is still being written
         throw;

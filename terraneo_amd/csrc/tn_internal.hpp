@@ -158,11 +158,12 @@ constexpr int REDUCE_PART_DOUBLES = 16 * (REDUCE_MAX_BLOCKS / 2);
 int reduce_blocks(const MeshLevel& m, int ncomp);
 
 // Device scalars of a conjugate-gradient solve without preconditioner (k_cg_update).
-// rr[slot(it)]: (r, r) after iteration it, a ring the host drains by batches;
-// ctl[DONE]: the iteration that met the stopping test, 0 before.
+// ctl[DONE]: the iteration that met the stopping test, 0 before; rr[slot(it)]: (r, r)
+// after iteration it, a ring the host drains by batches.  ctl and rr are one array of
+// WORDS doubles, copied to the host together.
 struct CgState {
     static constexpr int RING = 64;
-    static constexpr int DONE = 0, R0 = 1;
+    static constexpr int DONE = 0, R0 = 1, RR = 2, WORDS = RR + RING + 1;
     double *rr, *ctl;
     double *part_pap, *part_rr;  // partials of (p, A p) and of (r, r)
     int npap, nrr;
