@@ -412,6 +412,7 @@ int tn_mesh_create_radii(int lat_level, int nr, const double* radii, tn_mesh** o
 int tn_mesh_destroy(tn_mesh* m)
 {
     TN_API_BEGIN
+    tn::dev_wait();
     delete m;
     TN_API_END
 }
@@ -600,6 +601,7 @@ int tn_eps_create(const tn_mesh* m, int dtype, const void* eta, int bc_cmb, int 
 int tn_eps_destroy(tn_eps* op)
 {
     TN_API_BEGIN
+    tn::dev_wait();
     delete op;
     TN_API_END
 }

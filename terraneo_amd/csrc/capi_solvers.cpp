@@ -294,6 +294,7 @@ int tn_gmg_create(int nlevels, tn_eps* const* ops, const tn_gmg_options* opts, t
 int tn_gmg_destroy(tn_gmg* g)
 {
     TN_API_BEGIN
+    tn::dev_wait();
     delete g;
     TN_API_END
 }

@@ -12,6 +12,8 @@
 //  * a freed block may still be read by work in flight on any stream, so a block
 //    freed since the device's last synchronisation here is handed out only after
 //    a device synchronisation (what hipFree did at every free);
+//  * destroying an object, and the end of a solve, wait for the device (dev_wait),
+//    also as hipFree did: the caller may free or overwrite its own arrays then;
 //  * at most 1/16 of the device's memory is cached, the rest is freed at once;
 //  * the cache is emptied when an allocation fails (then retried) and when the
 //    last live block of the device is freed.
@@ -128,6 +130,24 @@ void dev_free(void* ptr)
         c.dirty = true;
     }
     if (c.live == 0) release(c);
+}
+
+void dev_wait()
+{
+    std::vector<int> held;
+    {
+        Pool& p = pool();
+        std::lock_guard<std::mutex> lk(p.mu);
+        for (const auto& d : p.dev)
+            if (d.second.live > 0) held.push_back(d.first);
+    }
+    int current = 0;
+    if (held.empty() || hipGetDevice(&current) != hipSuccess) return;
+    for (int d : held) {
+        if (d != current) (void)hipSetDevice(d);
+        (void)hipDeviceSynchronize();
+        if (d != current) (void)hipSetDevice(current);
+    }
 }
 
 // Pinned pages: a solve takes one or two; freed pages are kept (as many as

@@ -157,6 +157,7 @@ int tn_fv_create(tn_mesh* m, tn_fv** out)
 int tn_fv_destroy(tn_fv* fv)
 {
     TN_API_BEGIN
+    tn::dev_wait();
     delete fv;
     TN_API_END
 }

@@ -41,6 +41,8 @@ BVec VecStore::make(const BVec& like) { return make_like(like, like.b[0].dtype);
 
 VecStore::~VecStore()
 {
+    // (a solve's last updates of the caller's vectors may still be queued)
+    if (!ptrs_.empty()) dev_wait();
     for (void* p : ptrs_) dev_free(p);
 }
 

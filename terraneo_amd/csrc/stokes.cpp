@@ -204,6 +204,7 @@ int tn_stokes_create(const tn_mesh* vel, const tn_mesh* pre, tn_eps* A, tn_stoke
 int tn_stokes_destroy(tn_stokes* K)
 {
     TN_API_BEGIN
+    tn::dev_wait();
     delete K;
     TN_API_END
 }

@@ -36,6 +36,9 @@ void set_last_error(const std::string& msg);
 // device memory of the library's objects, with a bounded cache of freed blocks (devmem.cpp)
 void* dev_alloc(size_t bytes);
 void dev_free(void* ptr);
+// waits for the work on every device that holds such memory; for the destruction of
+// objects, whose queued work may also read arrays of the caller's
+void dev_wait();
 // a page of pinned host memory for results copied behind queued work
 constexpr size_t HOST_PAGE_BYTES = 4096;
 struct HostPage {
