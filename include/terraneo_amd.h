@@ -123,6 +123,11 @@ int tn_free(void* ptr);
 int tn_memcpy_h2d(void* dst, const void* src, size_t bytes);
 int tn_memcpy_d2h(void* dst, const void* src, size_t bytes);
 int tn_sync(void);
+/* The library keeps the device blocks of destroyed objects for its next objects, up to
+ * 1/16 of the device's memory and until the last object is gone.  This frees them (and
+ * idle pinned pages), for a host program whose own allocator needs the space; waits for
+ * the work that may still read them.  Live objects are not touched. */
+int tn_release_cached_memory(void);
 /* Test hook, no counterpart in the reference: polls per bounded hand-off wait
  * of the march kernels (default 2^20).  A small value forces the waits to give
  * up, so the error path above can be exercised; every kernel still exits. */

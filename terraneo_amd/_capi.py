@@ -53,6 +53,7 @@ SIGNATURES = {
     "tn_memcpy_h2d": (i32, [vp, vp, C.c_size_t]),
     "tn_memcpy_d2h": (i32, [vp, vp, C.c_size_t]),
     "tn_sync": (i32, []),
+    "tn_release_cached_memory": (i32, []),
     "tn_set_wait_limit": (i32, [i32]),
     "tn_mesh_create": (i32, [i32, i32, f64, f64, pvp]),
     "tn_mesh_create_subdomains": (i32, [i32, i32, f64, f64, i32, i32, pvp]),

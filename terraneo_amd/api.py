@@ -209,6 +209,12 @@ class Eps:
         check(lib().tn_eps_set_penalty_once(self.h, int(bool(once))))
 
 
+def release_cached_memory():
+    """Give the device blocks that the library keeps of destroyed objects (up to 1/16 of the
+    device's memory) back, e.g. before a large allocation of torch's."""
+    check(lib().tn_release_cached_memory())
+
+
 # ---------------------------------------------------------------- mesh-level helpers
 def vector_mass(mesh, x, y, stream=None):
     check(lib().tn_vector_mass_apply(mesh.h, dtype_code(x.dtype), _ptr(x), _ptr(y), _stream_ptr(stream)))

@@ -329,7 +329,19 @@ int tn_malloc(void** ptr, size_t bytes)
 {
     TN_API_BEGIN
     TN_REQUIRE(ptr, "null out pointer");
-    TN_HIP(hipMalloc(ptr, bytes));
+    hipError_t e = hipMalloc(ptr, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        tn::dev_trim();
+        e = hipMalloc(ptr, bytes);
+    }
+    TN_HIP(e);
+    TN_API_END
+}
+int tn_release_cached_memory(void)
+{
+    TN_API_BEGIN
+    tn::dev_trim();
     TN_API_END
 }
 int tn_free(void* ptr)

@@ -15,8 +15,9 @@
 //  * destroying an object, and the end of a solve, wait for the device (dev_wait),
 //    also as hipFree did: the caller may free or overwrite its own arrays then;
 //  * at most 1/16 of the device's memory is cached, the rest is freed at once;
-//  * the cache is emptied when an allocation fails (then retried) and when the
-//    last live block of the device is freed.
+//  * the cache is emptied when an allocation of the library fails (then retried),
+//    when the last live block of the device is freed and on dev_trim, by which the
+//    host program gets it back for its own allocator.
 // Blocks belong to the device they were allocated on; all calls are serialised
 // by one mutex, so any thread may allocate and free.
 #include <map>
@@ -119,8 +120,8 @@ void dev_free(void* ptr)
     DeviceCache& c = p.dev[b.device];
     --c.live;
     if (c.limit == 0) {
-        size_t avail = 0, total = 0;
-        c.limit = hipMemGetInfo(&avail, &total) == hipSuccess ? total / 16 : 1;
+        hipDeviceProp_t prop;
+        c.limit = hipGetDeviceProperties(&prop, b.device) == hipSuccess ? prop.totalGlobalMem / 16 : 1;
     }
     if (c.cached + b.bytes > c.limit) {
         (void)hipFree(ptr);
@@ -150,8 +151,8 @@ void dev_wait()
     }
 }
 
-// Pinned pages: a solve takes one or two; freed pages are kept (as many as
-// were ever in use at once).
+// Pinned pages: a solve takes one; freed pages are kept (as many as were ever in
+// use at once) until dev_trim.
 namespace {
 struct Pages {
     std::mutex mu;
@@ -181,6 +182,21 @@ HostPage::~HostPage()
 {
     std::lock_guard<std::mutex> lk(pages().mu);
     pages().idle.push_back(p);
+}
+
+void dev_trim()
+{
+    {
+        Pool& p = pool();
+        std::lock_guard<std::mutex> lk(p.mu);
+        for (auto& d : p.dev) release(d.second);  // (hipFree waits for the block's device)
+    }
+    std::vector<double*> idle;
+    {
+        std::lock_guard<std::mutex> lk(pages().mu);
+        idle.swap(pages().idle);
+    }
+    for (double* q : idle) (void)hipHostFree(q);
 }
 
 }  // namespace tn

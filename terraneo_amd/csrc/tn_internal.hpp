@@ -39,6 +39,8 @@ void dev_free(void* ptr);
 // waits for the work on every device that holds such memory; for the destruction of
 // objects, whose queued work may also read arrays of the caller's
 void dev_wait();
+// frees the blocks and pinned pages kept for reuse
+void dev_trim();
 // a page of pinned host memory for results copied behind queued work
 constexpr size_t HOST_PAGE_BYTES = 4096;
 struct HostPage {
