@@ -9,10 +9,11 @@
 //
 // FV fields carry one ghost layer: [10][n+1][n+1][nr+1], r fastest; real
 // cells (xc, yc, rc) in [1, n-1]^2 x [1, nr-1] are the FE hex cells
-// (xc-1, yc-1, rc-1).  Every kernel runs one thread per real cell (or per
+// (xc-1, yc-1, rc-1).  A kernel runs one thread per real cell (or per
 // FE node for the projection), radially consecutive threads on radially
 // consecutive cells, so every field access of a wave is one contiguous
-// radial run.  Nothing is accumulated with atomics: every output element is
+// radial run; the stable step and the predictor walk along columns where the mesh
+// fills their lanes (walk_columns).  Nothing is accumulated with atomics: every output element is
 // written by one thread, so results repeat bit for bit.
 #include <hip/hip_runtime.h>
 
@@ -297,6 +298,46 @@ __device__ __forceinline__ void walk_columns(const FvArgs& a, const double* __re
     }
 }
 
+// The same a thread per cell: the column's table and both levels of four corners for
+// each.  For the meshes that leave the walk's lanes or its CUs empty (walk_pays); the
+// arithmetic, and so the result, is the walk's.
+template <class F>
+__device__ __forceinline__ void visit_cells(const FvArgs& a, const double* __restrict__ columns,
+                                            const double* __restrict__ vel, double kappa, F& f)
+{
+    const int n = a.n, nr = a.nr, nq = n - 1, ncr = nr - 1;
+    const int64_t N = 10LL * n * n * nr, cells = 10LL * nq * nq * ncr;
+    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < cells; t += (int64_t)gridDim.x * blockDim.x) {
+        const int q = (int)(t / ncr), rc = 1 + (int)(t - (int64_t)q * ncr);
+        const int y = q % nq, x = (q / nq) % nq, d = q / (nq * nq);
+        double g[FV_COLUMN];
+        const double2* row = reinterpret_cast<const double2*>(columns + (int64_t)FV_COLUMN * q);
+#pragma unroll
+        for (int k = 0; k < FV_COLUMN / 2; ++k) {
+            const double2 v = row[k];
+            g[2 * k] = v.x;
+            g[2 * k + 1] = v.y;
+        }
+        CornerVel c00, c10, c01, c11;
+        const int64_t node = (((int64_t)d * n + x) * n + y) * nr + rc - 1, step = (int64_t)n * nr;
+        c00.load(vel, N, node);
+        c10.load(vel, N, node + step);
+        c01.load(vel, N, node + nr);
+        c11.load(vel, N, node + step + nr);
+        typename F::Pre pre;
+        f.load(pre, d, x, y, rc);
+        Layer L;
+        L.set(a, rc, kappa);
+        c00.combine(L);
+        c10.combine(L);
+        c01.combine(L);
+        c11.combine(L);
+        double beta[6], dc[6], M;
+        cell_faces(g, L, c00, c10, c01, c11, beta, dc, M);
+        f(true, rc, pre, beta, dc, M);
+    }
+}
+
 __device__ __forceinline__ int64_t neighbour(int n, int nr, int d, int xc, int yc, int rc, int f)
 {
     const int ox = f == 0 ? -1 : (f == 1 ? 1 : 0), oy = f == 2 ? -1 : (f == 3 ? 1 : 0),
@@ -463,23 +504,38 @@ struct StableStep {
     }
 };
 
-__global__ __launch_bounds__(64 * FV_STRIPS) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_fv_dt(FvArgs a, const double* __restrict__ columns, const double* __restrict__ vel, double kappa,
-                                                    double* __restrict__ part)
+// block minimum (order-independent) into part[blockIdx.x]
+__device__ __forceinline__ void block_min(double v, double* __restrict__ part)
+{
+    __shared__ double red[16];
+    for (int o = 32; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double m = red[0];
+        for (int k = 1; k < (int)(blockDim.x >> 6); ++k) m = fmin(m, red[k]);
+        part[blockIdx.x] = m;
+    }
+}
+
+__global__ __launch_bounds__(64 * FV_STRIPS) __attribute__((amdgpu_waves_per_eu(4, 4)))
+void k_fv_dt(FvArgs a, const double* __restrict__ columns, const double* __restrict__ vel, double kappa,
+             double* __restrict__ part)
 {
     StableStep st;
     st.diffusion = kappa > 0;
     walk_columns(a, columns, vel, kappa, st);
-    double dtc = st.dt;
-    // block minimum (order-independent)
-    __shared__ double red[FV_STRIPS];
-    for (int o = 32; o > 0; o >>= 1) dtc = fmin(dtc, __shfl_xor(dtc, o));
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = dtc;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double m = red[0];
-        for (int k = 1; k < FV_STRIPS; ++k) m = fmin(m, red[k]);
-        part[blockIdx.x] = m;
-    }
+    block_min(st.dt, part);
+}
+
+__global__ __launch_bounds__(FV_BLOCK) void k_fv_dt_cells(FvArgs a, const double* __restrict__ columns,
+                                                          const double* __restrict__ vel, double kappa,
+                                                          double* __restrict__ part)
+{
+    StableStep st;
+    st.diffusion = kappa > 0;
+    visit_cells(a, columns, vel, kappa, st);
+    block_min(st.dt, part);
 }
 
 __global__ __launch_bounds__(256) void k_min_finalize(const double* __restrict__ part, int nblk,
@@ -569,14 +625,22 @@ struct Predict {
     }
 };
 
-__global__ __launch_bounds__(64 * FV_STRIPS) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_fct_predictor(FvArgs a, const double* __restrict__ columns, const double* __restrict__ vel,
-                                                            const double* __restrict__ T, double dt, double kappa,
-                                                            const double* __restrict__ source, int subtract_div,
-                                                            double* __restrict__ TL, double* __restrict__ ad,
-                                                            int64_t fvsize, FctFused fu)
+__global__ __launch_bounds__(64 * FV_STRIPS) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void k_fct_predictor(FvArgs a, const double* __restrict__ columns, const double* __restrict__ vel, const double* __restrict__ T,
+        double dt, double kappa, const double* __restrict__ source, int subtract_div, double* __restrict__ TL,
+        double* __restrict__ ad, int64_t fvsize, FctFused fu)
 {
     Predict p{T, source, TL, ad, dt, subtract_div, a.n, a.nr, fvsize, fu};
     walk_columns(a, columns, vel, kappa, p);
+}
+
+__global__ __launch_bounds__(FV_BLOCK)
+void k_fct_predictor_cells(FvArgs a, const double* __restrict__ columns, const double* __restrict__ vel, const double* __restrict__ T,
+        double dt, double kappa, const double* __restrict__ source, int subtract_div, double* __restrict__ TL,
+        double* __restrict__ ad, int64_t fvsize, FctFused fu)
+{
+    Predict p{T, source, TL, ad, dt, subtract_div, a.n, a.nr, fvsize, fu};
+    visit_cells(a, columns, vel, kappa, p);
 }
 
 // Dirichlet values on the shells: the real boundary cell and the ghost beyond (helpers.hpp:64-96)
@@ -781,7 +845,25 @@ static int walk_blocks(int n, int nr, int per_cu)
 {
     return std::max(1, std::min(walk_groups(n, nr) * (n - 1), device_cus() * per_cu));
 }
-int fv_dt_blocks(int n, int nr) { return walk_blocks(n, nr, 2); }
+// Whether the column walk beats the form by cells: a chunk's lanes filled with `fill`
+// layers or more on average, and four columns or more for each CU's first block (on
+// fewer the walk has no columns to keep corners for).  Both forms measured at levels 3
+// to 7 with 3 to 200 radial nodes.  The stable step reads little and breaks even at 24
+// layers (level 7: 8 layers 104 us walked, 58 by cells; 24: 106, 108; 64: 120, 259), the
+// predictor at 40 (8 layers 162, 50; 32: 252, 233; 40: 269, 287; 2 x 34.5: 491, 475; 64:
+// 334, 445).  At level 4 the forms are within 4 us of each other.
+constexpr int WALK_FILL_DT = 24, WALK_FILL_PREDICTOR = 40;
+static bool walk_pays(int n, int nr, int fill)
+{
+    const int chunks = (nr - 1 + 63) / 64;
+    return nr - 1 >= fill * chunks && walk_groups(n, nr) * (n - 1) >= 4 * device_cus();
+}
+// at most FV_DT_BLOCKS partial minima of the form by cells
+constexpr int FV_DT_BLOCKS = 2048;
+int fv_dt_blocks(int n, int nr)
+{
+    return walk_pays(n, nr, WALK_FILL_DT) ? walk_blocks(n, nr, 2) : std::min(blocks_for(fv_real_cells(n, nr)), FV_DT_BLOCKS);
+}
 
 void launch_fv_centers(const FvArgs& a, double* c, hipStream_t s)
 {
@@ -823,7 +905,10 @@ void launch_fv_ghost2(const int32_t* pairs, int cnt, int nr, double* f, double* 
 void launch_fv_dt(const FvArgs& a, const double* vel, double kappa, double* part, double* out, hipStream_t s)
 {
     const int nb = fv_dt_blocks(a.n, a.nr);
-    hipLaunchKernelGGL(k_fv_dt, dim3(nb), dim3(64 * FV_STRIPS), 0, s, a, a.columns, vel, kappa, part);
+    if (walk_pays(a.n, a.nr, WALK_FILL_DT))
+        hipLaunchKernelGGL(k_fv_dt, dim3(nb), dim3(64 * FV_STRIPS), 0, s, a, a.columns, vel, kappa, part);
+    else
+        hipLaunchKernelGGL(k_fv_dt_cells, dim3(nb), dim3(FV_BLOCK), 0, s, a, a.columns, vel, kappa, part);
     hipLaunchKernelGGL(k_min_finalize, dim3(1), dim3(256), 0, s, part, nb, out);
 }
 
@@ -831,8 +916,12 @@ void launch_fct_predictor(const FvArgs& a, const double* vel, const double* T, d
                           const double* source, int subtract_div, double* TL, double* ad, const FctFused& fused,
                           hipStream_t s)
 {
-    hipLaunchKernelGGL(k_fct_predictor, dim3(walk_blocks(a.n, a.nr, 1)), dim3(64 * FV_STRIPS), 0, s, a, a.columns, vel, T, dt, kappa,
-                       source, subtract_div, TL, ad, fv_size(a.n, a.nr), fused);
+    if (walk_pays(a.n, a.nr, WALK_FILL_PREDICTOR))
+        hipLaunchKernelGGL(k_fct_predictor, dim3(walk_blocks(a.n, a.nr, 1)), dim3(64 * FV_STRIPS), 0, s, a, a.columns, vel,
+                           T, dt, kappa, source, subtract_div, TL, ad, fv_size(a.n, a.nr), fused);
+    else
+        hipLaunchKernelGGL(k_fct_predictor_cells, dim3(blocks_for(fv_real_cells(a.n, a.nr))), dim3(FV_BLOCK), 0, s, a,
+                           a.columns, vel, T, dt, kappa, source, subtract_div, TL, ad, fv_size(a.n, a.nr), fused);
 }
 
 void launch_fv_dirichlet(int n, int nr, double* f, int apply_cmb, double t_cmb, int apply_surf, double t_surf,
