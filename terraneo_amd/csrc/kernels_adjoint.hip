@@ -203,6 +203,46 @@ __global__ __launch_bounds__(256) void k_grad_log_cell_eta(Geom<T> g, const T* _
     }
 }
 
+// The same a thread per cell, with the march's arithmetic.
+template <typename T>
+__global__ __launch_bounds__(256) void k_grad_cells(Geom<T> g, const T* __restrict__ eta_cell, const T* __restrict__ u,
+                                                    const T* __restrict__ lam, int bc_cmb, int bc_surf,
+                                                    T* __restrict__ grad, int64_t cells)
+{
+    constexpr int G = 2 * GEO_STRIDE;
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= cells) return;
+    const int ncr = g.nr - 1, ncl = g.n - 1;
+    const int q = (int)(t / ncr), rc = (int)(t - (int64_t)q * ncr);
+    const int lat = ((q / ncl / ncl) * g.n + (q / ncl) % ncl) * g.n + q % ncl;
+    AdjWalk<T> A{u, lam, g.coords, 10LL * g.n * g.n * g.nr, g.nr, rc, rc == 0 ? bc_cmb : (int)TN_NEUMANN,
+                 rc == ncr - 1 ? bc_surf : (int)TN_NEUMANN, bc_cmb == TN_FREESLIP || bc_surf == TN_FREESLIP};
+    typename AdjWalk<T>::Raw raw[4];
+    A.load(lat, raw[0]);
+    A.load(lat + g.n, raw[1]);
+    A.load(lat + 1, raw[2]);
+    A.load(lat + g.n + 1, raw[3]);
+    T table[G];
+#pragma unroll
+    for (int k = 0; k < G; ++k) table[k] = g.geo[(int64_t)q * G + k];
+    const T e = eta_cell[t];
+    const T r0 = g.radii[rc], r1 = g.radii[rc + 1];
+    const T half_dr = T(0.5) * (r1 - r0), r_mid = T(0.5) * (r0 + r1);
+    const T alpha = T(1) / r_mid, beta = T(1) / half_dr, kr = r_mid * r_mid * half_dr * T(1.0 / 6.0);
+    AdjCorner<T> c[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) A.corner(raw[k], c[k]);
+    T d12[3], e12[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        d12[k] = c[1].D[k] + c[2].D[k];
+        e12[k] = c[1].E[k] + c[2].E[k];
+    }
+    const T acc = adj_wedge(c[0], c[1], c[2], d12, e12, table, alpha, beta, kr) +
+                  adj_wedge(c[3], c[2], c[1], d12, e12, table + GEO_STRIDE, alpha, beta, kr);
+    grad[t] = -e * acc;
+}
+
 }  // namespace
 
 template <typename T>
@@ -213,12 +253,26 @@ void launch_grad_log_cell_eta(const Geom<T>& g, const T* eta_cell, const T* u, c
     const int64_t quads = 10LL * ncl * ncl;
     TN_REQUIRE(10LL * g.n * g.n < (1LL << 31), "gradient: mesh too large");
     const int P = ncr > 32 ? 1 : std::min(ADJ_RUNS, 64 / ncr), chunks = ncr > 32 ? (ncr + 63) / 64 : 1;
+    // The march pays where a wave's lanes hold 40 layers or more on average and every lane
+    // of one round of resident waves gets four cells; else a thread per cell, as fast or
+    // faster than on all smaller or emptier meshes measured (levels 3 to 7, 3 to 200 radial
+    // nodes).  FP64, free-slip, us by march and by cells: level 7 x 3 nodes 38 and 14, x 9
+    // 43 and 43, x 17 59 and 80, x 70 355 and 352; level 6 x 9 18 and 12, x 33 27 and 39;
+    // level 5 x 17 10.4 and 8.1, x 65 16 and 20.
+    const int waves_simd = sizeof(T) == 8 ? 2 : 3;
+    const int64_t cells = quads * ncr;
+    if ((P > 1 ? P * ncr : ncr / chunks) < 40 || cells < 4LL * 64 * 4 * device_cus() * waves_simd) {
+        hipLaunchKernelGGL(k_grad_cells<T>, dim3((unsigned)((cells + 255) / 256)), dim3(256), 0, s, g, eta_cell, u, lam,
+                           bc_cmb, bc_surf, grad, cells);
+        TN_HIP(hipGetLastError());
+        return;
+    }
     // Equal runs for one round of resident waves (two per SIMD in FP64, three in FP32), or
     // for further rounds so that no run is longer than 40 quads (10 x 128 x 128 quads of 99
     // layers, FP64: 461 us in one round, 417 in four).  Four runs side by side and more:
     // two rounds' worth (10 x 128 x 128 of 8 layers: 60 us in one, 47 in two, 57 in four; a
     // thread per cell took 54).
-    const int64_t waves = std::max<int64_t>(1, 4LL * device_cus() * (P > 3 ? 4 : sizeof(T) == 8 ? 2 : 3) / chunks);
+    const int64_t waves = std::max<int64_t>(1, 4LL * device_cus() * (P > 3 ? 4 : waves_simd) / chunks);
     const int64_t rounds = (quads + waves * P * 40 - 1) / (waves * P * 40);
     const int64_t runs = std::min<int64_t>(quads, waves * P * rounds);
     const int64_t groups = (runs + P - 1) / P;
