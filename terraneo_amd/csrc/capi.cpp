@@ -136,20 +136,23 @@ int tn::device_cus()
     }
     return cache[dev];
 }
-namespace {
-
-// Segment length (node columns per block) of a march kernel with `own` node
-// rows per block and `waves_per_cu` resident waves per CU: the kernel takes
-// ceil(blocks / resident blocks) rounds of (seg + 1) quad columns each; pick
-// the segment that minimises that product.  TN_MARCH_SEG overrides (tuning).
-}  // namespace
-int tn::march_seg_for(int n, int own, int waves_per_cu)
+// Node columns per block that the program's environment asks for, 0: the library's
+// choice (TN_MARCH_SEG, tuning)
+static int march_seg_asked()
 {
     static const int env = [] {
         const char* e = std::getenv("TN_MARCH_SEG");
-        return e ? std::atoi(e) : 0;
+        return e ? std::min(std::atoi(e), tn::MARCH_SEG_MAX) : 0;
     }();
-    if (env > 0) return std::min(std::min(env, n), tn::MARCH_SEG_MAX);
+    return env;
+}
+// Segment length (node columns per block) of a march kernel with `own` node
+// rows per block and `waves_per_cu` resident waves per CU: the kernel takes
+// ceil(blocks / resident blocks) rounds of (seg + 1) quad columns each; pick
+// the segment that minimises that product.
+int tn::march_seg_for(int n, int own, int waves_per_cu)
+{
+    if (march_seg_asked() > 0) return std::min(march_seg_asked(), n);
     const int64_t per_cu = std::max(1, waves_per_cu / (own + 1));
     const int64_t nxb = (n + own - 1) / own, cus = tn::device_cus() * per_cu;
     int best = std::min(n, tn::MARCH_SEG_MAX);
@@ -173,6 +176,7 @@ int tn::march_seg_for(int n, int own, int waves_per_cu)
 // longer than the kernel's carried level (MARCH_SEG_MAX columns).
 int tn::march_run_blocks(int cols, int resident)
 {
+    if (march_seg_asked() > 0) return (cols + march_seg_asked() - 1) / march_seg_asked();
     const int64_t cus = tn::device_cus();
     int64_t best = 1;
     double best_cost = -1.0;
@@ -189,11 +193,6 @@ int tn::march_run_blocks(int cols, int resident)
     return (int)best;
 }
 namespace {
-
-int march_seg(int n, int dtype_size)
-{
-    return tn::march_seg_for(n, tn::march_block_rows(dtype_size), tn::march_waves_per_cu(dtype_size));
-}
 
 // arguments of a stored operator's kernels but for the vectors; the boundary
 // forms are brought up to date
@@ -245,12 +244,9 @@ void eps_apply_t(tn_eps* op, const void* src_v, void* dst_v, hipStream_t s)
         const tn::Geom<T> g = geom_of<T>(m);
         // penalty positions: every copy (the reference's rule) or the owned copy only
         const double* pen_coords = op->penalty_once ? m.d_coords_owned.p : m.d_coords.p;
-        const int rows = tn::march_block_rows((int)sizeof(T));
         tn::MarchArgs<T> a{src, dst, eta, eta_cell, g.geo, g.coords, g.radii, pen_coords, m.d_radii.p,
                            need_blk ? (const T*)op->blk.p : nullptr, penalty ? op->pen.p : nullptr,
-                           m.n, m.nr, march_seg(m.n, (int)sizeof(T)),
-                           tn::march_run_blocks(10 * ((m.n + rows - 1) / rows) * m.n, tn::march_resident(sizeof(T))), op->bc_cmb, op->bc_surf, add ? 1 : 0,
-                           tn::march_guard()};
+                           m.n, m.nr, op->bc_cmb, op->bc_surf, add ? 1 : 0, tn::march_guard()};
         tn::launch_eps_march<T>(a, op->diagonal, s);
     } else {
         // the gather writes every node copy once (boundary test side and penalty fused)

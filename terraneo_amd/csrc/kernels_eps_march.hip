@@ -903,11 +903,12 @@ int march_waves()
     return w;
 }
 
-int march_block_rows(int dtype_size) { return (dtype_size == 8 ? march_waves<double>() : march_waves<float>()) - 1; }
-
-int march_waves_per_cu(int dtype_size) { return march_block_rows(dtype_size) + 1; }
-
-int march_resident(int dtype_size) { return dtype_size == 4 && march_waves<float>() <= 12 ? 2 : 1; }
+// blocks of the matrix apply that a CU holds (LDS: 149 KB in FP64, 65 KB in FP32)
+template <typename T>
+int march_resident()
+{
+    return sizeof(T) == 4 && march_waves<T>() <= 12 ? 2 : 1;
+}
 
 // matrix-apply kernel variant: 0 the per-quad-load march, 1 the carried-corner
 // march, 2 the same with each step's loads issued a step ahead (TN_EPS_KERNEL
@@ -923,24 +924,29 @@ int eps_kernel_variant()
 }
 
 template <typename T, int W>
-void launch_march_w(const MarchArgs<T>& a, bool diagonal, hipStream_t s)
+void launch_march_w(MarchArgs<T> a, bool diagonal, hipStream_t s)
 {
     constexpr int OWN = W - 1;
-    const int nxb = (a.n + OWN - 1) / OWN, nys = (a.n + a.seg - 1) / a.seg;
-    const dim3 gr((unsigned)(10 * nxb * nys)), bl(64 * W);
+    const int nxb = (a.n + OWN - 1) / OWN;
+    const dim3 bl(64 * W);
     // the carried-corner kernel is built for 8, 12 and 16 waves per block
     const int var = W >= 8 ? eps_kernel_variant() : 0;
-    if (diagonal) {
-        hipLaunchKernelGGL((k_eps_march<T, true, W>), gr, bl, 0, s, a, a.geo, a.coords, a.blk, a.coords_d, a.pen);
-    } else if (var == 0) {
-        hipLaunchKernelGGL((k_eps_march<T, false, W>), gr, bl, 0, s, a, a.geo, a.coords, a.blk, a.coords_d, a.pen);
+    if (diagonal || var == 0) {
+        a.seg = march_seg_for(a.n, OWN, W);
+        TN_REQUIRE(a.seg >= 1 && a.seg <= MARCH_SEG_MAX, "march kernel: segment length out of range");
+        const dim3 gr((unsigned)(10 * nxb * ((a.n + a.seg - 1) / a.seg)));
+        if (diagonal)
+            hipLaunchKernelGGL((k_eps_march<T, true, W>), gr, bl, 0, s, a, a.geo, a.coords, a.blk, a.coords_d, a.pen);
+        else
+            hipLaunchKernelGGL((k_eps_march<T, false, W>), gr, bl, 0, s, a, a.geo, a.coords, a.blk, a.coords_d, a.pen);
     } else {
         if constexpr (W >= 8) {
             const int cfg = ((a.bc_cmb != TN_NEUMANN || a.bc_surf != TN_NEUMANN) ? 1 : 0) | (a.pen ? 2 : 0) |
                             (a.eta_cell ? 4 : 0) | (var == 2 ? 8 : 0);
-            const dim3 fr((unsigned)a.blocks);
-            TN_REQUIRE(a.blocks >= 1 && ((int64_t)10 * nxb * a.n + a.blocks - 1) / a.blocks <= MARCH_SEG_MAX,
+            const int cols = 10 * nxb * a.n, blocks = march_run_blocks(cols, march_resident<T>());
+            TN_REQUIRE(blocks >= 1 && (cols + blocks - 1) / blocks <= MARCH_SEG_MAX,
                        "march kernel: run of columns out of range");
+            const dim3 fr((unsigned)blocks);
             TN_REQUIRE(3ULL * 10 * a.n * a.n * a.nr * sizeof(T) < (1ULL << 32),
                        "apply: field larger than 4 GB (buffer resources address 32-bit byte offsets)");
             switch (cfg) {
@@ -961,7 +967,6 @@ template <typename T>
 void launch_eps_march(const MarchArgs<T>& a, bool diagonal, hipStream_t s)
 {
     TN_REQUIRE(a.nr - 1 >= 2, "march kernel: at least 2 radial cells");
-    TN_REQUIRE(a.seg >= 1 && a.seg <= MARCH_SEG_MAX, "march kernel: segment length out of range");
     TN_REQUIRE(10LL * (a.n - 1) * (a.n - 1) * 2 * GEO_STRIDE < (1LL << 31), "march kernel: mesh too large");
     // at lateral level 7 x 129, Dirichlet, the carried-corner kernel measures 0.47 ms in
     // FP64 (16 waves) and 0.27 ms in FP32 (12 waves); an LDS-tiled variant that staged
@@ -972,7 +977,6 @@ void launch_eps_march(const MarchArgs<T>& a, bool diagonal, hipStream_t s)
         case 8: launch_march_w<T, 8>(a, diagonal, s); break;
         case 12: launch_march_w<T, 12>(a, diagonal, s); break;
         default: launch_march_w<T, 16>(a, diagonal, s); break;
-            break;
     }
 }
 

@@ -47,19 +47,12 @@ struct MarchArgs {
     const T* blk;             // [2][10 n n][3] boundary quadratic forms, or null (both shells Neumann)
     const double* pen;        // fs/fs penalty: [0..3) beta, [4..13) S, [13..16) gamma = S beta, or null
     int n, nr;
-    int seg;                  // node columns per block in the march direction (diagonal mode)
-    int blocks;               // blocks = equal runs of node columns (matrix apply)
     int bc_cmb, bc_surf;
     int add;                  // 1: dst += A x, 0: dst = A x
     MarchGuard guard;
+    int seg = 0;              // node columns per block of k_eps_march (set by the launcher)
 };
 
-// node rows owned per block (waves per block - 1) for an element size in bytes
-int march_block_rows(int dtype_size);
-// resident waves per CU at the kernel's register use (element size in bytes)
-int march_waves_per_cu(int dtype_size);
-// blocks of the matrix apply that a CU holds (LDS: 149 KB in FP64, 65 KB in FP32)
-int march_resident(int dtype_size);
 // blocks of the matrix apply over `cols` node columns
 int march_run_blocks(int cols, int resident);
 // segment length of a march kernel (own node rows per block, resident waves per CU)
