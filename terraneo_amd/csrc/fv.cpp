@@ -30,7 +30,7 @@ using tn::MeshLevel;
 tn::FvArgs tn_fv::args() const
 {
     const MeshLevel& L = mesh->lvl;
-    return tn::FvArgs{L.d_coords.p, L.d_radii.p, centers.p, columns.p, layers.p, n, nr};
+    return tn::FvArgs{L.d_coords.p, L.d_radii.p, columns.p, layers.p, n, nr};
 }
 
 namespace {

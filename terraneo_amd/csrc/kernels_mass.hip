@@ -70,7 +70,8 @@ __global__ __launch_bounds__(256) void k_mass_stencil(MassArgs<T> a)
     for (int k = 0; k < NB; ++k) {
         if (wl[k] == 0.0) continue;  // a neighbour outside the diamond (no wedge holds it)
         const int64_t col = (((int64_t)d * n + x + ox[k]) * n + y + oy[k]) * nr + r;
-        for (int c = 0; c < a.ncomp; ++c) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
             const T* xc = a.x + c * N + col;
             double v = c0r * (double)xc[0];
             if (r > 0) v += cm * (double)xc[-1];
@@ -78,7 +79,8 @@ __global__ __launch_bounds__(256) void k_mass_stencil(MassArgs<T> a)
             acc[c] += wl[k] * v;
         }
     }
-    for (int c = 0; c < a.ncomp; ++c) a.y[c * N + t] = (T)acc[c];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) a.y[c * N + t] = (T)acc[c];
 }
 
 // One component (the projection's CG): a wave walks an even

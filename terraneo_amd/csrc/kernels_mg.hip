@@ -355,13 +355,10 @@ __host__ __device__ constexpr GcaWeights make_gca_weights()
 {
     GcaWeights t{};
     constexpr int OFF[2][3][2] = {{{0, 0}, {1, 0}, {0, 1}}, {{1, 1}, {0, 1}, {1, 0}}};
-    constexpr GcaWedge L[2][8] = {
-        {{0, 0, 0, 0}, {1, 0, 0, 0}, {0, 1, 0, 0}, {0, 0, 1, 0}, {1, 0, 1, 0}, {0, 1, 1, 0}, {0, 0, 0, 1}, {0, 0, 1, 1}},
-        {{1, 0, 0, 1}, {0, 1, 0, 1}, {1, 1, 0, 1}, {1, 0, 1, 1}, {0, 1, 1, 1}, {1, 1, 1, 1}, {1, 1, 0, 0}, {1, 1, 1, 0}}};
     for (int W = 0; W < 2; ++W)
         for (int k = 0; k < 8; ++k)
             for (int i = 0; i < 6; ++i) {
-                const GcaWedge f = L[W][k];
+                const GcaWedge f = GCA_LIST[W][k];
                 const int m = i % 3;
                 // the fine dof's offset from the coarse cell's corner, in fine steps
                 const int a = f.sx + OFF[f.w][m][0], b = f.sy + OFF[f.w][m][1], c = f.sr + (i >= 3 ? 1 : 0);

@@ -9,7 +9,6 @@ namespace tn {
 struct FvArgs {
     const double* coords;   // [10][n][n][3] unit lateral positions
     const double* radii;    // [nr]
-    const double* centers;  // [10][n+1][n+1][nr+1][3] cell centres (ghost layers included)
     const double* columns;  // [10][n-1][n-1][FV_COLUMN] lateral geometry of each hex column
     const double* layers;   // [nr+1] radial part of the cell centres (ghost layers at the shells: 0)
     int n, nr;
@@ -72,7 +71,7 @@ struct tn_fv {
     tn_mesh* mesh = nullptr;
     int n = 0, nr = 0;
     int64_t size = 0;                 // FV scalar elements (ghosts included)
-    tn::DevBuf<double> centers;       // [size][3]
+    tn::DevBuf<double> centers;       // [size][3], for tn_fv_cell_centers
     tn::DevBuf<double> columns;       // [10 (n-1)^2][FV_COLUMN] lateral column geometry
     tn::DevBuf<double> layers;        // [nr+1] radial part of the cell centres
     tn::DevBuf<double> TL, Rp, Rm;    // FV scalars; their radial ghost cells at the shells stay zero
