@@ -76,6 +76,10 @@ class StokesProblem:
         cell [10][n-1][n-1][nr-1] (torch FP64 on the device).  Rebuilds the
         viscous block, the multigrid hierarchy and the Schur preconditioner."""
         torch = _torch()
+        # the last viscosity's objects go first, all at once: destroying one waits for the
+        # device, and its blocks serve the new ones
+        self.gmg = self.K = self.A = None
+        self.ops, self._dummies = [], []
         self.eta = eta.contiguous() if eta is not None else None
         self.eta_cell = eta_cell.contiguous() if eta_cell is not None else None
         bc = self.bc
