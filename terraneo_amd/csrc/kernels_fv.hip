@@ -232,7 +232,8 @@ __device__ __forceinline__ void cell_faces(const double* __restrict__ g, const L
 // of nodes or cells that two strips share is read into the caches at one time
 // (with strips far apart the stable step took 258 us and the predictor 710 us at
 // level 7 x 129, with the loads of a column issued in its own step 231 and 756 us,
-// a step ahead of the stores 233 and 650 us).  The columns of all strip groups
+// a step ahead of the stores 233 and 650 us; call times, the predictor as a stage of
+// its own).  The columns of all strip groups
 // are split evenly over the blocks.  The corner velocities shared by consecutive
 // columns stay in registers.  f.load(pre, d, x, y, rc) a step ahead,
 // then f(valid, rc, pre, beta, dc, M).
@@ -484,8 +485,8 @@ __global__ __launch_bounds__(FV_BLOCK) void k_fv_ghost2(const int32_t* __restric
 
 // local stable time step M / lambda per cell, minimum per block
 // (fct_advection_diffusion.hpp:110-164)
-// (geometry as the predictor's: 831 us at lateral level 7 x 129 when every cell
-// read its seven centres, 227 us so)
+// (geometry as the predictor's: 750 us at lateral level 7 x 129 when every cell
+// read its seven centres, 174 us so; both repeated alone, in an energy step 831 and 206)
 struct StableStep {
     double dt = 1e300;
     bool diffusion;
@@ -555,9 +556,10 @@ __global__ __launch_bounds__(256) void k_min_finalize(const double* __restrict__
 // (dt / M) (|beta| / 2) (T_i - T_j), stored face-major [6][fv cells].
 // What binds is memory: velocity and T in, T_L and six fluxes out (88 B a cell,
 // 104 with the flux sums).  A thread per cell that read the centres of its cell
-// and six neighbours and both levels of four corners took 951 us at lateral level
+// and six neighbours and both levels of four corners took 962 us at lateral level
 // 7 x 129; the column / layer split of the geometry needs no centres, and a run of
-// columns loads two corners a step: 650 us, 4.3 TB/s counting the re-reads.
+// columns loads two corners a step: 646 us as a stage of its own, 715 us in the step,
+// where the flux sums are written too (731 in the energy case, behind other work).
 struct Predict {
     const double* __restrict__ T;
     const double* __restrict__ source;

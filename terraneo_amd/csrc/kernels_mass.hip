@@ -92,8 +92,9 @@ __global__ __launch_bounds__(256) void k_mass_stencil(MassArgs<T> a)
 // 21 loads per node instead of 7 the vector cache was what bound it.  With dot != null it also leaves the
 // block's part of the sum over all node copies of x . y, which for x equal on a
 // node's copies is the owned dot of x with the interface-summed y.
-// Product with its interface sum: level 7 x 129 430 -> 282 us, level 6 x 65 47 us, level
-// 5 x 33 17 -> 12 us (the determinants, too, a column ahead: 14 without).
+// With its part of the dot, FP64: level 7 x 129 314 us, level 6 x 65 44 us, level 5 x 33
+// 11 us (13 without the determinants a column ahead); a thread per node, without the
+// dot, 456, 58 and 13 us.
 // lane i receives lane i-1's (UP) or i+1's value, 0 at the end
 constexpr int LANE_UP = 0x138, LANE_DOWN = 0x130;  // DPP wave_shr:1, wave_shl:1
 template <int CTRL>

@@ -1163,8 +1163,9 @@ void launch_stored_apply(const StoredArgs<T, S>& a, bool diagonal, hipStream_t s
         TN_HIP(hipGetLastError());
         hipLaunchKernelGGL((k_stored_gather<T, S, true>), gg, bg, 0, s, a);
     } else {
-        // one wave per SIMD or less: latency counts (FP64, 160 quads: 12.4 us, 6.5 split, 640
-        // quads 17.1, 11.1; FP32, 640 quads 11.5, 8.0); at 2560 waves the bandwidth does (FP32: 18.6 us, 20.3 split)
+        // one wave per SIMD or less: latency counts (64 layers, a wave per quad and split: FP64,
+        // 160 quads 15.7 and 8.2 us, 640 quads 23.5 and 21.0; FP32, 640 quads 13.1 and 12.7); at
+        // 2560 waves the bandwidth does (FP32, 17 layers: 18.6 us, 20.3 split)
         if (waves <= 4 * device_cus())
             hipLaunchKernelGGL((k_stored_cells<T, S, false, true>), dim3((unsigned)waves), dim3(128), 0, s, a);
         else

@@ -44,11 +44,12 @@
 //
 // Both are bound by the latency of a step's loads.  The table entries of a column are
 // loaded like a vector (a lane each) one step ahead and spread over the lanes through
-// LDS: as scalar loads, ready only when needed, B took 80 us where it now takes 35.
-// Velocity at 10 x 65 x 65 x 65 nodes, FP64, free-slip, us: B^T (Add) 85 as a march
-// over cells with hand-offs between waves, 38 now (with 66 + 66 MB of velocity read
-// and written, 16 MB of table: 3.9 TB/s); B 74 as a cell pass with a gather, 35 now.
-// At 10 x 9 x 9 x 9 nodes 24 -> 7 and 15 -> 7.  FP32 against FP64 (relative L2): 9.4e-7
+// LDS: as scalar loads, ready only when needed, B took 80 us where it now takes 37.
+// Velocity at 10 x 65 x 65 x 65 nodes, FP64, free-slip, kernels in us: B^T (Add) 89 as a
+// march over cells with hand-offs between waves, 38 now where its velocity is still in
+// the caches (repeated alone: 66 + 66 MB read and written, 16 MB of table: 3.9 TB/s) and
+// 48 in the block apply, behind the viscous block (103 as a march); B 73 + 6 as a cell
+// pass with a gather, 37 now.  At 10 x 9 x 9 x 9 nodes 25 -> 5 and 16 -> 10.  FP32 against FP64 (relative L2): 9.4e-7
 // as cell geometry in FP32, 0.8e-7 with vectors made in FP64 and rounded once (B 1.2e-7).
 #include <algorithm>
 #include <type_traits>
